@@ -11,7 +11,7 @@
 //    coset expansion), grouped by pass shape; one launch per shape and step;
 //  - leaves: every table's row-pair leaves in one launch;
 //  - Merkle: step s of every table's tree (a wide level, or a subtree top of
-//    up to 9 levels through LDS) in one launch per step;
+//    up to 6 levels through LDS) in one launch per step;
 //  - the roots gathered into one array and copied to pinned host memory.
 // Blocks of a launch are assigned to tables by a prefix sum over their block
 // counts, largest table first so the small ones fill the tail. The kernels
@@ -92,18 +92,18 @@ struct Writer {
 }  // namespace
 
 // Tree steps of one table with L leaves (power of two): wide levels one per
-// step while more than 2^14 children remain, then subtree tops.
+// step while more than TREE_TOP_CHILDREN children remain, then tree tops.
 std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t L) {
     std::vector<std::pair<TreeStep, uint32_t>> out;  // (step, blocks)
     uint64_t *nodes = (uint64_t *)nodes_b;
     uint64_t C = L;
-    while (C > (1u << 14)) {
-        TreeStep s{nodes, C - 1, C / 2 - 1, 256, 1};
-        out.push_back({s, (uint32_t)(C / 512)});
+    while (C > TREE_TOP_CHILDREN) {
+        TreeStep s{nodes, C - 1, C / 2 - 1, TREE_WIDE_SPAN, 1};
+        out.push_back({s, (uint32_t)(C / (2 * TREE_WIDE_SPAN))});
         C /= 2;
     }
     while (C > 1) {
-        const uint32_t span = (uint32_t)(C / 2 < 256 ? C / 2 : 256);
+        const uint32_t span = (uint32_t)(C / 2 < TREE_TOP_SPAN ? C / 2 : TREE_TOP_SPAN);
         const uint64_t blocks = C / (2 * span);
         TreeStep s{nodes, C - 1, C / 2 - 1, span, 32};
         out.push_back({s, (uint32_t)blocks});

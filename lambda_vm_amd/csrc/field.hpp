@@ -20,6 +20,7 @@
 // generic (flat) ones also count against lgkmcnt and so make every LDS wait
 // wait for the memory loads in flight as well.
 typedef __attribute__((address_space(1))) uint64_t gmem_u64;
+typedef __attribute__((address_space(1))) uint32_t gmem_u32;
 #define LVM_GLOBAL(p) ((gmem_u64 *)(p))
 #define LVM_GLOBAL_CONST(p) ((const gmem_u64 *)(p))
 

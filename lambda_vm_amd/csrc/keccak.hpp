@@ -156,4 +156,127 @@ __device__ __forceinline__ void keccak_pair_node(const uint64_t lft[4], const ui
     for (int i = 0; i < 4; i++) out[i] = ((uint64_t)h[i] << 32) | l[i];
 }
 
+// ---- one permutation over 16 lanes ----
+//
+// A single Keccak-f on one lane is a serial chain of ~4300 VALU instructions,
+// each taking its wave's issue slot for four cycles whatever the number of
+// active lanes: 7.2 us, which every level of a tree top pays with the chip
+// idle. Here a 16-lane DPP row holds one state: lane (y, half) = bits 0..2 and
+// bit 3 of the lane number holds the 32-bit halves of row y, x = 0..4 in five
+// registers (lanes y = 5..7 hold zero). Per round:
+//  - column parities: XOR over the 8 lanes of a half, three DPP steps (zero
+//    lanes do not contribute);
+//  - theta, and rho as one funnel shift per word with the other half (lane ^ 8)
+//    brought by a row rotate; a rotation by 0 or by 32..63 lands in the other
+//    half, which the next step's addresses undo;
+//  - pi through LDS: every lane stores its five words and reads the five of its
+//    new row (row stride 65 words: the reads of a 32-lane half-wave hit
+//    distinct banks);
+//  - chi is local to the lane.
+// About 55 instructions and one LDS round trip per round, four states a wave.
+struct CoopKeccak {
+    uint32_t sh[5];   // rho: funnel shift of word x
+    uint32_t rd[5];   // pi: LDS word of the new row's word x
+    uint32_t wr;      // LDS word of word 0 (word x at wr + COOP_ROW * x)
+    uint32_t m_lo, m_hi;  // iota: all ones in the lane holding that half of word 0
+};
+constexpr uint32_t COOP_ROW = 65;
+constexpr uint32_t COOP_ZERO = 5 * COOP_ROW;       // a word that stays zero
+constexpr uint32_t COOP_WORDS = COOP_ZERO + 1;     // LDS words per wave
+
+// rotation of lane (x, y), index x + 5y
+constexpr uint32_t KECCAK_RHO[25] = {0,  1,  62, 28, 27, 36, 44, 6,  55, 20, 3,  10, 43,
+                                     25, 39, 41, 45, 15, 21, 8,  18, 2,  61, 56, 14};
+constexpr uint64_t rho_of_column(int x) {  // y = 0..4, six bits each
+    uint64_t v = 0;
+    for (int y = 0; y < 5; y++) v |= (uint64_t)KECCAK_RHO[x + 5 * y] << (6 * y);
+    return v;
+}
+constexpr uint64_t rho_of_row(int y) {  // x = 0..4, six bits each
+    uint64_t v = 0;
+    for (int x = 0; x < 5; x++) v |= (uint64_t)KECCAK_RHO[x + 5 * y] << (6 * x);
+    return v;
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_ROR8 = 0x128;
+
+// Lane constants, and the wave's zero word (call with the wave converged).
+__device__ __forceinline__ void coop_setup(CoopKeccak &k, uint32_t *ws) {
+    const uint32_t lane = threadIdx.x & 63, y = lane & 7, half = (lane >> 3) & 1, base = lane & 48;
+#pragma unroll
+    for (int x = 0; x < 5; x++) {
+        const uint32_t n = (uint32_t)(rho_of_column(x) >> (6 * y)) & 63u;
+        k.sh[x] = (64u - n) & 31u;
+    }
+#pragma unroll
+    for (int X = 0; X < 5; X++) {
+        // B[X, Y] comes from lane row X, word x = 3Y + X mod 5
+        const uint32_t x = (3 * y + X) % 5;
+        const uint32_t n = (uint32_t)(rho_of_row(X) >> (6 * x)) & 63u;
+        const uint32_t swap = (n == 0 || n >= 32) ? 1u : 0u;
+        k.rd[X] = y < 5 ? x * COOP_ROW + base + ((half ^ swap) << 3) + X : COOP_ZERO;
+    }
+    k.wr = lane;
+    k.m_lo = (y == 0 && half == 0) ? ~0u : 0u;
+    k.m_hi = (y == 0 && half == 1) ? ~0u : 0u;
+    if (lane == 0) ws[COOP_ZERO] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Keccak-f of the four states of the wave (a[x] of lane (y, half) as above);
+// ws: the wave's COOP_WORDS words of LDS. Every lane of the wave takes part.
+__device__ __forceinline__ void keccak_f1600_coop(uint32_t a[5], const CoopKeccak &k, uint32_t *ws) {
+#pragma unroll
+    for (int round = 0; round < 24; round++) {
+        uint32_t c[5], r[5];
+#pragma unroll
+        for (int x = 0; x < 5; x++) c[x] = a[x] ^ dpp<DPP_XOR1>(a[x]);
+#pragma unroll
+        for (int x = 0; x < 5; x++) c[x] ^= dpp<DPP_XOR2>(c[x]);
+#pragma unroll
+        for (int x = 0; x < 5; x++) c[x] ^= dpp<DPP_HALF_MIRROR>(c[x]);
+#pragma unroll
+        for (int x = 0; x < 5; x++) r[x] = __builtin_amdgcn_alignbit(c[x], dpp<DPP_ROR8>(c[x]), 31);
+#pragma unroll
+        for (int x = 0; x < 5; x++) a[x] = xor3(a[x], c[(x + 4) % 5], r[(x + 1) % 5]);
+#pragma unroll
+        for (int x = 0; x < 5; x++)
+            ws[k.wr + COOP_ROW * x] = __builtin_amdgcn_alignbit(a[x], dpp<DPP_ROR8>(a[x]), k.sh[x]);
+        // one wave's LDS accesses stay in order: no wait, only no reordering
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint32_t b[5];
+#pragma unroll
+        for (int x = 0; x < 5; x++) b[x] = ws[k.rd[x]];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int x = 0; x < 5; x++) a[x] = chi(b[x], b[(x + 1) % 5], b[(x + 2) % 5]);
+        // a ^ (constant & mask)
+        a[0] = __builtin_amdgcn_bitop3_b32(a[0], KECCAK_RC_LO[round], k.m_lo, 0x78);
+        a[0] = __builtin_amdgcn_bitop3_b32(a[0], KECCAK_RC_HI[round], k.m_hi, 0x78);
+    }
+}
+
+// The state of Keccak-256 over two 32-byte nodes (one permutation): `src` is
+// the 16 words left || right, read only by lanes with `on`.
+template <class Ptr>
+__device__ __forceinline__ void coop_load_pair(uint32_t a[5], Ptr src, bool on) {
+    const uint32_t lane = threadIdx.x & 63, y = lane & 7, half = (lane >> 3) & 1;
+#pragma unroll
+    for (int x = 0; x < 5; x++) {
+        const uint32_t i = 5 * y + x;  // 64-bit lane of the state
+        uint32_t v = 0;
+        if (on && i < 8) v = src[2 * i + half];
+        if (i == 8 && half == 0) v = 0x01;
+        if (i == 16 && half == 1) v = 0x80000000u;
+        a[x] = v;
+    }
+}
+
 }  // namespace lvm

@@ -199,9 +199,15 @@ struct LeafJob {
 struct TreeStep {
     uint64_t *nodes;
     uint64_t cstart, pstart;  // first child / first parent index of the level
-    uint32_t span;            // parents per block at the first level (<= 256)
+    uint32_t span;            // parents per block at the first level
     uint32_t levels;          // levels this step builds
 };
+// Trees of more children than this have their level hashed one node per lane;
+// below, the step is a tree top: blocks of TREE_TOP_SPAN parents, all their
+// levels, one permutation per 16 lanes (merkle.hip).
+constexpr uint64_t TREE_TOP_CHILDREN = 1u << 14;
+constexpr uint32_t TREE_TOP_SPAN = 32;
+constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
                            hipStream_t st);
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,

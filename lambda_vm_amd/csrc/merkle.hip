@@ -124,11 +124,8 @@ __global__ __launch_bounds__(256) void keccak_fp3_pair_leaves_kernel(const uint6
     for (int k = 0; k < 4; k++) o[k] = ((uint64_t)h[k] << 32) | l[k];
 }
 
-// One level of parents [begin, begin+count).
-__global__ __launch_bounds__(256) void merkle_level_kernel(uint64_t *nodes, uint64_t begin, uint64_t count) {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) return;
-    const uint64_t p = begin + k;
+// parent p = Keccak(node[2p+1] || node[2p+2]), one lane per node
+__device__ __forceinline__ void merkle_parent(uint64_t *nodes, uint64_t p) {
     const uint64_t *l = nodes + 4 * (2 * p + 1);
     const uint64_t *r = nodes + 4 * (2 * p + 2);
     uint64_t lv[4] = {l[0], l[1], l[2], l[3]}, rv[4] = {r[0], r[1], r[2], r[3]}, o[4];
@@ -140,67 +137,76 @@ __global__ __launch_bounds__(256) void merkle_level_kernel(uint64_t *nodes, uint
     d[3] = o[3];
 }
 
-// Up to 9 tree levels per launch: block b takes the 2*span children
-// [cstart + 2*span*b, ...) of one level (span <= 256 parents), writes their
-// parents, keeps them in LDS and keeps hashing pairs, at most `levels`
-// levels in all, writing every level it produces to the node array.
-__device__ __forceinline__ void merkle_subtree_body(uint64_t *nodes, uint64_t cstart, uint64_t pstart, uint32_t span,
-                                                    uint32_t levels, uint64_t b) {
-    __shared__ uint64_t dig[256][4];
-    const uint32_t t = threadIdx.x;
+// One level of parents [begin, begin+count).
+__global__ __launch_bounds__(256) void merkle_level_kernel(uint64_t *nodes, uint64_t begin, uint64_t count) {
+    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= count) return;
+    merkle_parent(nodes, begin + k);
+}
+
+// Up to 6 tree levels per launch, one permutation per 16 lanes: block b takes
+// the 2*span children [cstart + 2*span*b, ...) of one level (span <=
+// TREE_TOP_SPAN parents), writes their parents, keeps them in LDS and keeps
+// hashing pairs, writing every level it produces to the node array. The
+// levels are a serial chain of permutations, so what counts is the latency of
+// one: 512 threads hold 32 states (two waves per SIMD at the first level).
+// A tree of 2^11 leaves: 98 -> 48 us against one lane per node with its rounds
+// unrolled; 2^17 leaves (top of 2^14): 130 -> 62 us.
+constexpr uint32_t TREE_THREADS = 512;
+__device__ __forceinline__ void merkle_top_body(uint64_t *nodes, uint64_t cstart, uint64_t pstart, uint32_t span,
+                                                uint64_t b) {
+    __shared__ uint32_t s_pi[TREE_THREADS / 64][COOP_WORDS];
+    __shared__ uint32_t s_dig[2][TREE_TOP_SPAN][8];
+    uint32_t *ws = s_pi[threadIdx.x >> 6];
+    CoopKeccak k;
+    coop_setup(k, ws);
+    const uint32_t g = threadIdx.x >> 4, lane = threadIdx.x & 15, y = lane & 7, half = lane >> 3;
+    uint32_t *nodes32 = (uint32_t *)nodes;
     uint64_t pbase = pstart + (uint64_t)span * b;  // first parent of this block at the current level
-    if (t < span) {
-        const uint64_t *l = nodes + 4 * (cstart + 2 * (uint64_t)span * b + 2 * t);
-        uint64_t lv[4] = {l[0], l[1], l[2], l[3]}, rv[4] = {l[4], l[5], l[6], l[7]}, o[4];
-        keccak_pair_node<true>(lv, rv, o);
-        uint64_t *d = nodes + 4 * (pbase + t);
+    uint32_t cur = 0;
+    for (uint32_t cnt = span;; cnt >>= 1) {
+        // waves with no state at this level have nothing to do (uniform per wave)
+        if ((threadIdx.x >> 6) * 4 < cnt) {
+            const bool on = g < cnt;
+            uint32_t a[5];
+            if (cnt == span)
+                coop_load_pair(a, (const gmem_u32 *)nodes32 + 8 * (cstart + 2 * ((uint64_t)span * b + g)), on);
+            else
+                coop_load_pair(a, s_dig[cur ^ 1][2 * (on ? g : 0)], on);
+            keccak_f1600_coop(a, k, ws);
+            if (on && y == 0) {
+                gmem_u32 *d = (gmem_u32 *)nodes32 + 8 * (pbase + g);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            d[k] = o[k];
-            dig[t][k] = o[k];
-        }
-    }
-    // next levels: the block's nodes at level start L0 = pbase; the parent of
-    // node x is (x - 1) / 2, and a block's nodes stay contiguous
-    uint32_t cnt = span;
-    for (uint32_t lv_done = 1; cnt > 1 && lv_done < levels; lv_done++) {
-        __syncthreads();
-        const uint32_t half = cnt / 2;
-        const uint64_t next = (pbase - 1) / 2;
-        uint64_t o[4];
-        if (t < half) {
-            uint64_t lv[4] = {dig[2 * t][0], dig[2 * t][1], dig[2 * t][2], dig[2 * t][3]};
-            uint64_t rv[4] = {dig[2 * t + 1][0], dig[2 * t + 1][1], dig[2 * t + 1][2], dig[2 * t + 1][3]};
-            keccak_pair_node<true>(lv, rv, o);
-        }
-        __syncthreads();
-        if (t < half) {
-            uint64_t *d = nodes + 4 * (next + t);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                d[k] = o[k];
-                dig[t][k] = o[k];
+                for (int x = 0; x < 4; x++) {
+                    d[2 * x + half] = a[x];
+                    s_dig[cur][g][2 * x + half] = a[x];
+                }
             }
         }
-        pbase = next;
-        cnt = half;
+        if (cnt == 1) break;
+        __syncthreads();
+        cur ^= 1;
+        pbase = (pbase - 1) / 2;  // the parent of node x is (x - 1) / 2; a block's nodes stay contiguous
     }
 }
 
-__global__ __launch_bounds__(256) void merkle_subtree_kernel(uint64_t *nodes, uint64_t cstart, uint64_t pstart,
-                                                             uint32_t span) {
-    merkle_subtree_body(nodes, cstart, pstart, span, 32, blockIdx.x);
+__global__ __launch_bounds__(TREE_THREADS) void merkle_top_kernel(uint64_t *nodes, uint64_t cstart, uint64_t pstart,
+                                                                  uint32_t span) {
+    merkle_top_body(nodes, cstart, pstart, span, blockIdx.x);
 }
 
 // One tree step for each of several trees: blocks [prefix[t], prefix[t+1])
-// run step t (a single wide level with levels = 1, or a subtree top).
-__global__ __launch_bounds__(256) void merkle_steps_batched_kernel(const TreeStep *__restrict__ steps,
-                                                                   const uint32_t *__restrict__ prefix,
-                                                                   uint32_t count) {
+// run step t (one wide level, TREE_THREADS parents per block, or a tree top).
+__global__ __launch_bounds__(TREE_THREADS) void merkle_steps_batched_kernel(const TreeStep *__restrict__ steps,
+                                                                            const uint32_t *__restrict__ prefix,
+                                                                            uint32_t count) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const TreeStep s = steps[t];
-    merkle_subtree_body(s.nodes, s.cstart, s.pstart, s.span, s.levels, b - prefix[t]);
+    if (s.span > TREE_TOP_SPAN)
+        merkle_parent(s.nodes, s.pstart + (uint64_t)s.span * (b - prefix[t]) + threadIdx.x);
+    else
+        merkle_top_body(s.nodes, s.cstart, s.pstart, s.span, b - prefix[t]);
 }
 
 // Copy each tree's root (node 0) into roots[t].
@@ -242,18 +248,18 @@ void merkle_build_inner(uint8_t *nodes_b, uint64_t L, hipStream_t st) {
     // children of the current level: C nodes starting at C - 1 (C a power of two)
     uint64_t C = L;
     // wide levels: one fully parallel launch per level
-    while (C > (1u << 14)) {
+    while (C > TREE_TOP_CHILDREN) {
         const uint64_t count = C / 2;
         hipLaunchKernelGGL(merkle_level_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, nodes,
                            count - 1, count);
         C = count;
     }
-    // narrow top: up to 9 levels per launch through LDS
+    // narrow top: up to 6 levels per launch through LDS
     while (C > 1) {
-        const uint32_t span = (uint32_t)(C / 2 < 256 ? C / 2 : 256);
+        const uint32_t span = (uint32_t)(C / 2 < TREE_TOP_SPAN ? C / 2 : TREE_TOP_SPAN);
         const uint64_t blocks = C / (2 * span);
-        hipLaunchKernelGGL(merkle_subtree_kernel, dim3((unsigned)blocks), dim3(256), 0, st, nodes, C - 1, C / 2 - 1,
-                           span);
+        hipLaunchKernelGGL(merkle_top_kernel, dim3((unsigned)blocks), dim3(TREE_THREADS), 0, st, nodes, C - 1,
+                           C / 2 - 1, span);
         C = blocks;
     }
 }
@@ -266,7 +272,7 @@ void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
                                hipStream_t st) {
     if (blocks)
-        hipLaunchKernelGGL(merkle_steps_batched_kernel, dim3(blocks), dim3(256), 0, st, d_steps, d_prefix, count);
+        hipLaunchKernelGGL(merkle_steps_batched_kernel, dim3(blocks), dim3(TREE_THREADS), 0, st, d_steps, d_prefix, count);
 }
 
 void launch_gather_roots(uint64_t *const *d_trees, uint32_t count, uint64_t *d_roots, hipStream_t st) {
