@@ -91,12 +91,11 @@ struct Writer {
 
 }  // namespace
 
-// Tree steps of one table with L leaves (power of two): wide levels one per
+// Tree steps above C nodes (a power of two): wide levels one per
 // step while more than TREE_TOP_CHILDREN children remain, then tree tops.
-std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t L) {
+std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t C) {
     std::vector<std::pair<TreeStep, uint32_t>> out;  // (step, blocks)
     uint64_t *nodes = (uint64_t *)nodes_b;
-    uint64_t C = L;
     while (C > TREE_TOP_CHILDREN) {
         TreeStep s{nodes, C - 1, C / 2 - 1, TREE_WIDE_SPAN, 1};
         out.push_back({s, (uint32_t)(C / (2 * TREE_WIDE_SPAN))});
@@ -182,8 +181,9 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         for (size_t t : b->order) {
             const lvm_table_desc &d = b->in[t];
             const uint64_t L = d.n * d.blowup / 2;
-            jobs.push_back({b->lde[t], d.m, L, (uint64_t *)(b->nodes[t] + (L - 1) * 32)});
-            total += (L + 255) / 256;
+            const uint32_t span = L <= LEAF_TOP_LEAVES ? leaf_top_span(L) : 0;
+            jobs.push_back({b->lde[t], d.m, L, (uint64_t *)b->nodes[t], span, 0});
+            total += span ? L / span : (L + TREE_WIDE_SPAN - 1) / TREE_WIDE_SPAN;
             if (total >= (1ull << 31)) return fail(LVM_ERR_ARG, "batched launch exceeds 2^31 blocks");
             prefix.push_back((uint32_t)total);
         }
@@ -202,7 +202,8 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         size_t max_tree = 0;
         for (size_t t = 0; t < T; t++) {
             const lvm_table_desc &d = b->in[t];
-            st[t] = tree_steps(b->nodes[t], d.n * d.blowup / 2);
+            const uint64_t L = d.n * d.blowup / 2;
+            st[t] = tree_steps(b->nodes[t], L <= LEAF_TOP_LEAVES ? L / leaf_top_span(L) : L);
             max_tree = std::max(max_tree, st[t].size());
         }
         for (size_t s = 0; s < max_tree; s++) {

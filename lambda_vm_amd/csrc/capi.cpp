@@ -111,15 +111,16 @@ int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blow
         TRY(ntt_coset_expand(coef.as<uint64_t>(), (uint32_t)w, lde.as<uint64_t>(), (uint32_t)w, (uint32_t)w,
                              log2u(n), log2u(blowup), d_weights, d->tb, st));
     }
+    uint64_t C;
     {
         ProfScope ps("keccak_leaves", st);
-        keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, nodes.as<uint8_t>() + (L - 1) * 32, st);
-        if (split) keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, pre.as<uint8_t>() + (L - 1) * 32, st);
+        C = keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, nodes.as<uint8_t>(), st);
+        if (split) keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, pre.as<uint8_t>(), st);
     }
     {
         ProfScope ps("merkle_inner", st);
-        merkle_build_inner(nodes.as<uint8_t>(), L, st);
-        if (split) merkle_build_inner(pre.as<uint8_t>(), L, st);
+        merkle_build_inner(nodes.as<uint8_t>(), C, st);
+        if (split) merkle_build_inner(pre.as<uint8_t>(), C, st);
     }
     LVM_HIP(hipGetLastError());
     uint8_t root[32];
@@ -349,13 +350,14 @@ int commit_owned_rows(Device *d, hipStream_t st, DevBuf &rows, size_t N, size_t 
     const size_t L = N / 2;
     DevBuf nodes;
     TRY(nodes.alloc((2 * L - 1) * 32, st));
+    uint64_t C;
     {
         ProfScope ps("keccak_leaves", st);
-        keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, nodes.as<uint8_t>() + (L - 1) * 32, st);
+        C = keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, nodes.as<uint8_t>(), st);
     }
     {
         ProfScope ps("merkle_inner", st);
-        merkle_build_inner(nodes.as<uint8_t>(), L, st);
+        merkle_build_inner(nodes.as<uint8_t>(), C, st);
     }
     LVM_HIP(hipGetLastError());
     uint8_t root[32];

@@ -15,9 +15,9 @@
 #include <cstring>
 #include <vector>
 
-#include "keccak.hpp"
 #include "lvm_internal.hpp"
 #include "prof.hpp"
+#include "tree_top.hpp"
 
 namespace lvm {
 
@@ -29,16 +29,17 @@ __device__ __forceinline__ void st3(uint64_t *p, fp3 v) {
 }
 
 // One fold of a codeword of 2*half Fp3 values into `out` (half values);
-// `leaves` (nullable) receives the half/2 layer leaves.
+// `nodes` (nullable) is the layer's tree, whose half/2 leaves are hashed in the
+// same pass; span > 0: a small layer, span leaves per block and the levels above.
 struct FoldJob {
     const uint64_t *in;
     uint64_t *out;
-    uint64_t *leaves;
+    uint64_t *nodes;
     uint64_t half;
     uint64_t z0, z1, z2;
     uint64_t ginv;  // inverse of the codeword's coset offset
     uint32_t log_half;
-    uint32_t pad;
+    uint32_t span;
 };
 
 __device__ __forceinline__ fp3 fold_one(const uint64_t *in, uint64_t j, fp3 zeta, uint64_t ginv, uint32_t log_half,
@@ -52,14 +53,14 @@ __device__ __forceinline__ fp3 fold_one(const uint64_t *in, uint64_t j, fp3 zeta
     return f3_add(sum, f3_mul_base(f3_mul(zeta, diff), tw));
 }
 
-// Thread t of one fold: out has half elements; leaves (nullable) receives
-// half/2 digests.
+// Thread t of one fold: out has half elements; the leaves (with nodes) are
+// half/2 digests, padded_leaves(half/2) = half/2.
 __device__ __forceinline__ void fri_fold_body(const FoldJob &j, uint64_t t, const uint64_t *ilo,
                                               const uint64_t *ihi) {
     const uint64_t *__restrict__ in = j.in;
     uint64_t *__restrict__ out = j.out;
-    uint64_t *__restrict__ leaves = j.leaves;
     const uint64_t half = j.half, ginv = j.ginv;
+    uint64_t *__restrict__ leaves = j.nodes ? j.nodes + 4 * (half / 2 - 1) : nullptr;
     const uint32_t log_half = j.log_half;
     const fp3 zeta{j.z0, j.z1, j.z2};
     if (leaves) {
@@ -91,19 +92,74 @@ __device__ __forceinline__ void fri_fold_body(const FoldJob &j, uint64_t t, cons
     }
 }
 
-__global__ __launch_bounds__(256) void fri_fold_kernel(FoldJob j, const uint64_t *ilo, const uint64_t *ihi) {
-    fri_fold_body(j, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, ilo, ihi);
+// Block b of a small layer: its span leaves' 2*span folded elements, one per
+// thread, then leaves and the tree levels above them, one permutation per 16
+// lanes. A layer of up to LEAF_TOP_LEAVES leaves has too few to fill the chip
+// with one leaf per lane; what its tree costs is the chain of permutations.
+__device__ __forceinline__ void fri_fold_top(const FoldJob &j, uint64_t b, const uint64_t *ilo, const uint64_t *ihi) {
+    __shared__ TreeTopLds s;
+    __shared__ uint64_t s_val[TREE_TOP_SPAN][6];  // a leaf's two elements, canonical
+    const TreeTop t(s);
+    const uint64_t first = (uint64_t)j.span * b, L = j.half / 2;
+    if (threadIdx.x < 2 * j.span) {
+        const uint64_t e = 2 * first + threadIdx.x;
+        const fp3 v = fold_one(j.in, e, fp3{j.z0, j.z1, j.z2}, j.ginv, j.log_half, ilo, ihi);
+        st3(j.out + 3 * e, v);
+        uint64_t *o = &s_val[threadIdx.x >> 1][3 * (threadIdx.x & 1)];
+        o[0] = canon(v.c0);
+        o[1] = canon(v.c1);
+        o[2] = canon(v.c2);
+    }
+    __syncthreads();
+    if (t.wave_on(j.span)) {
+        const bool on = t.g < j.span;
+        uint32_t a[5];
+#pragma unroll
+        for (int x = 0; x < 5; x++) {
+            const uint32_t i = 5 * t.y + x;
+            a[x] = 0;
+            if (on && i < 6) {
+                const uint64_t c = s_val[t.g][i];
+                a[x] = __builtin_bswap32(t.half ? (uint32_t)c : (uint32_t)(c >> 32));
+            }
+            if (i == 6 && t.half == 0) a[x] = 0x01;
+            if (i == 16 && t.half == 1) a[x] = 0x80000000u;
+        }
+        t.permute(a);
+        if (on) t.put(a, j.nodes, L - 1 + first + t.g, s, 0);
+    }
+    tree_top_levels(t, s, j.nodes, L - 1 + first, j.span, 0);
+}
+
+// blocks of one fold: threads per block and how many
+constexpr uint32_t FOLD_THREADS = TREE_THREADS;
+inline uint64_t fold_blocks(const FoldJob &j) {
+    if (j.span) return j.half / 2 / j.span;
+    return ((j.nodes ? j.half / 2 : j.half) + FOLD_THREADS - 1) / FOLD_THREADS;
+}
+
+__device__ __forceinline__ void fri_fold_block(const FoldJob &j, uint64_t b, const uint64_t *ilo,
+                                               const uint64_t *ihi) {
+    if (j.span)
+        fri_fold_top(j, b, ilo, ihi);
+    else
+        fri_fold_body(j, b * FOLD_THREADS + threadIdx.x, ilo, ihi);
+}
+
+__global__ __launch_bounds__(FOLD_THREADS) void fri_fold_kernel(FoldJob j, const uint64_t *ilo, const uint64_t *ihi) {
+    fri_fold_block(j, blockIdx.x, ilo, ihi);
 }
 
 // The same fold for several codewords in one launch: blocks [prefix[t],
 // prefix[t+1]) run jobs[t].
-__global__ __launch_bounds__(256) void fri_fold_batched_kernel(const FoldJob *__restrict__ jobs,
-                                                               const uint32_t *__restrict__ prefix, uint32_t count,
-                                                               const uint64_t *ilo, const uint64_t *ihi) {
+__global__ __launch_bounds__(FOLD_THREADS) void fri_fold_batched_kernel(const FoldJob *__restrict__ jobs,
+                                                                        const uint32_t *__restrict__ prefix,
+                                                                        uint32_t count, const uint64_t *ilo,
+                                                                        const uint64_t *ihi) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const FoldJob j = jobs[t];
-    fri_fold_body(j, (uint64_t)(b - prefix[t]) * blockDim.x + threadIdx.x, ilo, ihi);
+    fri_fold_block(j, b - prefix[t], ilo, ihi);
 }
 
 // Symmetric evaluations and authentication paths of one layer for every
@@ -151,6 +207,9 @@ struct lvm_fri {
 namespace {
 bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
 unsigned log2u(uint64_t x) { return (unsigned)__builtin_ctzll(x); }
+
+// leaves per block of a committed layer's fold (FoldJob::span)
+uint32_t fold_span(uint64_t L) { return L <= LEAF_TOP_LEAVES ? leaf_top_span(L) : 0; }
 
 void free_fri(lvm_fri *f) {
     if (f->cur && f->cur_owned) lvm_free(f->cur);
@@ -217,17 +276,16 @@ static int fri_fold_impl(lvm_fri *f, const uint64_t zeta[3], bool commit, uint8_
     }
     const uint64_t ginv = inv(f->offset);
     const uint32_t log_half = log2u(half);
+    const uint32_t span = commit ? fold_span(layer.L) : 0;
     {
         ProfScope ps(commit ? "fri_fold_leaves" : "fri_fold", st);
-        uint64_t threads = commit ? half / 2 : half;
-        const FoldJob j{f->cur, out, commit ? (uint64_t *)(layer.nodes + (layer.L - 1) * 32) : (uint64_t *)nullptr,
-                        half, zeta[0], zeta[1], zeta[2], ginv, log_half, 0};
-        hipLaunchKernelGGL(fri_fold_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, j,
+        const FoldJob j{f->cur, out, (uint64_t *)layer.nodes, half, zeta[0], zeta[1], zeta[2], ginv, log_half, span};
+        hipLaunchKernelGGL(fri_fold_kernel, dim3((unsigned)fold_blocks(j)), dim3(FOLD_THREADS), 0, st, j,
                            d->tb.inv_lo, d->tb.inv_hi);
     }
     if (commit) {
         ProfScope ps("fri_merkle", st);
-        merkle_build_inner(layer.nodes, layer.L, st);
+        merkle_build_inner(layer.nodes, span ? layer.L / span : layer.L, st);
     }
     StageScope ss(st);
     hipError_t e = hipGetLastError();
@@ -304,13 +362,13 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
                 release();
                 return fail(LVM_ERR_NOMEM, "FRI tree allocation failed");
             }
-            tsteps[t] = tree_steps(layers[t].nodes, layers[t].L);
+            const uint32_t span = fold_span(layers[t].L);
+            tsteps[t] = tree_steps(layers[t].nodes, span ? layers[t].L / span : layers[t].L);
             max_steps = std::max(max_steps, tsteps[t].size());
         }
-        jobs[t] = FoldJob{f->cur, outs[t],
-                          commit ? (uint64_t *)(layers[t].nodes + (layers[t].L - 1) * 32) : (uint64_t *)nullptr,
-                          half, zetas[3 * t], zetas[3 * t + 1], zetas[3 * t + 2], inv(f->offset), log2u(half), 0};
-        total += ((commit ? half / 2 : half) + 255) / 256;
+        jobs[t] = FoldJob{f->cur, outs[t], (uint64_t *)layers[t].nodes, half, zetas[3 * t], zetas[3 * t + 1],
+                          zetas[3 * t + 2], inv(f->offset), log2u(half), commit ? fold_span(layers[t].L) : 0};
+        total += fold_blocks(jobs[t]);
         if (total >= (1ull << 31)) {
             release();
             return fail(LVM_ERR_ARG, "batched fold exceeds 2^31 blocks");
@@ -357,7 +415,7 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
     hipError_t e = stage_upload(arena, blob.data(), blob.size(), st);
     if (e == hipSuccess) {
         ProfScope ps(commit ? "fri_fold_leaves" : "fri_fold", st);
-        hipLaunchKernelGGL(fri_fold_batched_kernel, dim3((unsigned)total), dim3(256), 0, st,
+        hipLaunchKernelGGL(fri_fold_batched_kernel, dim3((unsigned)total), dim3(FOLD_THREADS), 0, st,
                            (const FoldJob *)(arena + o_jobs), (const uint32_t *)(arena + o_prefix), (uint32_t)count,
                            d->tb.inv_lo, d->tb.inv_hi);
     }

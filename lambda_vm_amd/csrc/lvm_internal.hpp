@@ -135,11 +135,14 @@ int ntt_coset_expand(const uint64_t *coef, uint32_t coef_pitch, uint64_t *lde, u
 
 // ---- Keccak / Merkle (merkle.hip) ----
 // Row-pair leaves over words [w0, w1) of each row of a row-major table whose
-// rows are already stored in bit-reversed order: leaf i hashes rows 2i, 2i+1.
-void keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t num_leaves,
-                            uint8_t *leaves_out, hipStream_t st);
-// inner nodes of a (2L-1)*32-byte tree whose leaves sit at [L-1, 2L-1)
-void merkle_build_inner(uint8_t *nodes, uint64_t L, hipStream_t st);
+// rows are already stored in bit-reversed order: leaf i hashes rows 2i, 2i+1,
+// into node L-1+i of the tree. Small tables' blocks go on to the levels above
+// their leaves; returns the nodes C of the topmost level written, which lie at
+// [C-1, 2C-1): what merkle_build_inner goes on from.
+uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
+                                uint8_t *nodes, hipStream_t st);
+// the levels above the C nodes (a power of two) at [C-1, 2C-1) of a tree
+void merkle_build_inner(uint8_t *nodes, uint64_t C, hipStream_t st);
 // Keccak(BE24(e[2j]) || BE24(e[2j+1])) over an Fp3 array of `len` elements
 void keccak_fp3_pair_leaves(const uint64_t *evals, uint64_t len, uint8_t *leaves_out, hipStream_t st);
 
@@ -194,7 +197,9 @@ struct LeafJob {
     const uint64_t *rows;  // bit-reversed row-major LDE, `pitch` words per row
     uint64_t pitch;
     uint64_t num_leaves;
-    uint64_t *leaves;      // num_leaves x 32 bytes
+    uint64_t *nodes;       // the table's tree
+    uint32_t span;         // leaves per block of a small table (leaf_top_span), 0: TREE_THREADS of them, no levels
+    uint32_t pad;
 };
 struct TreeStep {
     uint64_t *nodes;
@@ -208,6 +213,10 @@ struct TreeStep {
 constexpr uint64_t TREE_TOP_CHILDREN = 1u << 14;
 constexpr uint32_t TREE_TOP_SPAN = 32;
 constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
+// Trees of at most this many leaves hash them one permutation per 16 lanes
+// too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch.
+constexpr uint64_t LEAF_TOP_LEAVES = 1u << 13;
+inline uint32_t leaf_top_span(uint64_t L) { return (uint32_t)(L < TREE_TOP_SPAN ? L : TREE_TOP_SPAN); }
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
                            hipStream_t st);
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
@@ -216,8 +225,8 @@ void launch_gather_roots(uint64_t *const *d_trees, uint32_t count, uint64_t *d_r
 // One FRI fold of each of count codewords in shared launches (fri.hip);
 // zetas: count x 3; roots_out (count x 32) when committing.
 int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool commit, uint8_t *roots_out);
-// the launches of one tree of L leaves (a power of two) at `nodes`: (step, blocks)
-std::vector<std::pair<TreeStep, uint32_t>> tree_steps(uint8_t *nodes, uint64_t L);
+// the launches above the C nodes (a power of two) at [C-1, 2C-1) of a tree: (step, blocks)
+std::vector<std::pair<TreeStep, uint32_t>> tree_steps(uint8_t *nodes, uint64_t C);
 
 // Constraint programs (compose.hip interpreter, compose_jit.cpp compiled form).
 struct CompArgs;

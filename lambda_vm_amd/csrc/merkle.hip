@@ -11,8 +11,8 @@
 // Tree layout (crypto/crypto/src/merkle_tree/merkle.rs:201-224, utils.rs:
 // 68-96): nodes[0..L-1) inner with the root at 0, leaves at [L-1, 2L-1),
 // parent(i) = Keccak(node[2i+1] || node[2i+2]).
-#include "keccak.hpp"
 #include "lvm_internal.hpp"
+#include "tree_top.hpp"
 
 namespace lvm {
 
@@ -80,6 +80,58 @@ __device__ __forceinline__ void row_pair_leaf(const uint64_t *__restrict__ rows,
     for (int k = 0; k < 4; k++) o[k] = ((uint64_t)h[k] << 32) | l[k];
 }
 
+// Leaves [span*b, span*b + span) of a small table, one permutation per 16
+// lanes, and the tree levels above them in the same launch. A table of up to
+// LEAF_TOP_LEAVES leaves would fill at most an eighth of the chip's lanes with
+// one leaf each, at 7.2 us per absorbed block; nodes is the whole tree.
+__device__ __forceinline__ void row_pair_leaf_top(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1,
+                                                  uint64_t L, uint32_t span, uint64_t b, uint64_t *nodes) {
+    __shared__ TreeTopLds s;
+    const TreeTop t(s);
+    const uint64_t first = (uint64_t)span * b;
+    if (t.wave_on(span)) {
+        const bool on = t.g < span;
+        const uint64_t width = w1 - w0, total = 2 * width, blocks = total / 17 + 1;
+        // the leaf's rows 2i and 2i+1; word e of the message is word e of row
+        // 2i, or word e - width of row 2i+1 (pitch - width words further on)
+        const gmem_u64 *row = LVM_GLOBAL_CONST(rows) + 2 * (first + (on ? t.g : 0)) * pitch + w0;
+        const uint64_t skip = pitch - width;
+        uint64_t v[5];
+        auto fetch = [&](uint64_t blk) {
+#pragma unroll
+            for (int x = 0; x < 5; x++) {
+                const uint32_t i = 5 * t.y + x;
+                const uint64_t e = blk * 17 + i;
+                v[x] = on && i < 17 && e < total ? row[e + (e >= width ? skip : 0)] : 0;
+            }
+        };
+        uint32_t a[5] = {0, 0, 0, 0, 0};
+        fetch(0);
+        for (uint64_t blk = 0; blk < blocks; blk++) {
+            const bool last = blk + 1 == blocks;
+            const uint64_t rem = total - blk * 17;  // first padding word of the last block
+#pragma unroll
+            for (int x = 0; x < 5; x++) {
+                const uint32_t i = 5 * t.y + x;
+                const uint64_t c = canon(v[x]);
+                a[x] ^= __builtin_bswap32(t.half ? (uint32_t)c : (uint32_t)(c >> 32));
+                if (last && i == rem && t.half == 0) a[x] ^= 0x01;
+                if (last && i == 16 && t.half == 1) a[x] ^= 0x80000000u;
+            }
+            if (!last) fetch(blk + 1);
+            t.permute(a);
+        }
+        if (on) t.put(a, nodes, L - 1 + first + t.g, s, 0);
+    }
+    tree_top_levels(t, s, nodes, L - 1 + first, span, 0);
+}
+
+__global__ __launch_bounds__(TREE_THREADS) void leaf_top_kernel(const uint64_t *rows, uint64_t pitch, uint64_t w0,
+                                                                uint64_t w1, uint64_t L, uint32_t span,
+                                                                uint64_t *nodes) {
+    row_pair_leaf_top(rows, pitch, w0, w1, L, span, blockIdx.x, nodes);
+}
+
 template <bool CONTIG>
 __global__ __launch_bounds__(256) void keccak_row_pair_leaves_kernel(const uint64_t *__restrict__ rows,
                                                                     uint64_t pitch, uint64_t w0, uint64_t w1,
@@ -91,16 +143,21 @@ __global__ __launch_bounds__(256) void keccak_row_pair_leaves_kernel(const uint6
 }
 
 // Leaves of several tables in one launch: blocks [prefix[t], prefix[t+1])
-// hash table t's leaves, 256 per block.
-__global__ __launch_bounds__(256) void keccak_leaves_batched_kernel(const LeafJob *__restrict__ jobs,
-                                                                   const uint32_t *__restrict__ prefix,
-                                                                   uint32_t count) {
+// hash table t's leaves, TREE_THREADS per block, or job.span of them with the
+// levels above for a small table.
+__global__ __launch_bounds__(TREE_THREADS) void keccak_leaves_batched_kernel(const LeafJob *__restrict__ jobs,
+                                                                            const uint32_t *__restrict__ prefix,
+                                                                            uint32_t count) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const LeafJob j = jobs[t];
-    const uint64_t i = (uint64_t)(b - prefix[t]) * 256 + threadIdx.x;
+    if (j.span) {
+        row_pair_leaf_top(j.rows, j.pitch, 0, j.pitch, j.num_leaves, j.span, b - prefix[t], j.nodes);
+        return;
+    }
+    const uint64_t i = (uint64_t)(b - prefix[t]) * TREE_THREADS + threadIdx.x;
     if (i >= j.num_leaves) return;
-    row_pair_leaf<true>(j.rows, j.pitch, 0, j.pitch, i, j.leaves);
+    row_pair_leaf<true>(j.rows, j.pitch, 0, j.pitch, i, j.nodes + 4 * (j.num_leaves - 1));
 }
 
 // FRI layer leaves: Keccak(BE24(e[2j]) || BE24(e[2j+1])), 6 lanes, one permutation
@@ -152,42 +209,19 @@ __global__ __launch_bounds__(256) void merkle_level_kernel(uint64_t *nodes, uint
 // one: 512 threads hold 32 states (two waves per SIMD at the first level).
 // A tree of 2^11 leaves: 98 -> 48 us against one lane per node with its rounds
 // unrolled; 2^17 leaves (top of 2^14): 130 -> 62 us.
-constexpr uint32_t TREE_THREADS = 512;
 __device__ __forceinline__ void merkle_top_body(uint64_t *nodes, uint64_t cstart, uint64_t pstart, uint32_t span,
                                                 uint64_t b) {
-    __shared__ uint32_t s_pi[TREE_THREADS / 64][COOP_WORDS];
-    __shared__ uint32_t s_dig[2][TREE_TOP_SPAN][8];
-    uint32_t *ws = s_pi[threadIdx.x >> 6];
-    CoopKeccak k;
-    coop_setup(k, ws);
-    const uint32_t g = threadIdx.x >> 4, lane = threadIdx.x & 15, y = lane & 7, half = lane >> 3;
-    uint32_t *nodes32 = (uint32_t *)nodes;
-    uint64_t pbase = pstart + (uint64_t)span * b;  // first parent of this block at the current level
-    uint32_t cur = 0;
-    for (uint32_t cnt = span;; cnt >>= 1) {
-        // waves with no state at this level have nothing to do (uniform per wave)
-        if ((threadIdx.x >> 6) * 4 < cnt) {
-            const bool on = g < cnt;
-            uint32_t a[5];
-            if (cnt == span)
-                coop_load_pair(a, (const gmem_u32 *)nodes32 + 8 * (cstart + 2 * ((uint64_t)span * b + g)), on);
-            else
-                coop_load_pair(a, s_dig[cur ^ 1][2 * (on ? g : 0)], on);
-            keccak_f1600_coop(a, k, ws);
-            if (on && y == 0) {
-                gmem_u32 *d = (gmem_u32 *)nodes32 + 8 * (pbase + g);
-#pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    d[2 * x + half] = a[x];
-                    s_dig[cur][g][2 * x + half] = a[x];
-                }
-            }
-        }
-        if (cnt == 1) break;
-        __syncthreads();
-        cur ^= 1;
-        pbase = (pbase - 1) / 2;  // the parent of node x is (x - 1) / 2; a block's nodes stay contiguous
+    __shared__ TreeTopLds s;
+    const TreeTop t(s);
+    const uint64_t pbase = pstart + (uint64_t)span * b;  // first parent of this block
+    if (t.wave_on(span)) {
+        const bool on = t.g < span;
+        uint32_t a[5];
+        coop_load_pair(a, (const gmem_u32 *)nodes + 8 * (cstart + 2 * ((uint64_t)span * b + t.g)), on);
+        t.permute(a);
+        if (on) t.put(a, nodes, pbase + t.g, s, 0);
     }
+    tree_top_levels(t, s, nodes, pbase, span, 0);
 }
 
 __global__ __launch_bounds__(TREE_THREADS) void merkle_top_kernel(uint64_t *nodes, uint64_t cstart, uint64_t pstart,
@@ -224,16 +258,23 @@ size_t padded_leaves(size_t n) {
     return p;
 }
 
-void keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t num_leaves,
-                            uint8_t *leaves_out, hipStream_t st) {
-    if (num_leaves == 0) return;
-    dim3 grid((unsigned)((num_leaves + 255) / 256));
+uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
+                                uint8_t *nodes, hipStream_t st) {
+    if (L <= LEAF_TOP_LEAVES) {
+        const uint32_t span = leaf_top_span(L);
+        hipLaunchKernelGGL(leaf_top_kernel, dim3((unsigned)(L / span)), dim3(TREE_THREADS), 0, st, rows, pitch, w0, w1,
+                           L, span, (uint64_t *)nodes);
+        return L / span;
+    }
+    uint64_t *leaves = (uint64_t *)(nodes + (L - 1) * 32);
+    dim3 grid((unsigned)((L + 255) / 256));
     if (w0 == 0 && w1 == pitch)
-        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<true>, grid, dim3(256), 0, st, rows, pitch, w0, w1,
-                           num_leaves, (uint64_t *)leaves_out);
+        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<true>, grid, dim3(256), 0, st, rows, pitch, w0, w1, L,
+                           leaves);
     else
-        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<false>, grid, dim3(256), 0, st, rows, pitch, w0, w1,
-                           num_leaves, (uint64_t *)leaves_out);
+        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<false>, grid, dim3(256), 0, st, rows, pitch, w0, w1, L,
+                           leaves);
+    return L;
 }
 
 void keccak_fp3_pair_leaves(const uint64_t *evals, uint64_t len, uint8_t *leaves_out, hipStream_t st) {
@@ -243,10 +284,8 @@ void keccak_fp3_pair_leaves(const uint64_t *evals, uint64_t len, uint8_t *leaves
     hipLaunchKernelGGL(keccak_fp3_pair_leaves_kernel, grid, dim3(256), 0, st, evals, nl, (uint64_t *)leaves_out);
 }
 
-void merkle_build_inner(uint8_t *nodes_b, uint64_t L, hipStream_t st) {
+void merkle_build_inner(uint8_t *nodes_b, uint64_t C, hipStream_t st) {
     uint64_t *nodes = (uint64_t *)nodes_b;
-    // children of the current level: C nodes starting at C - 1 (C a power of two)
-    uint64_t C = L;
     // wide levels: one fully parallel launch per level
     while (C > TREE_TOP_CHILDREN) {
         const uint64_t count = C / 2;
@@ -266,7 +305,9 @@ void merkle_build_inner(uint8_t *nodes_b, uint64_t L, hipStream_t st) {
 
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
                            hipStream_t st) {
-    if (blocks) hipLaunchKernelGGL(keccak_leaves_batched_kernel, dim3(blocks), dim3(256), 0, st, d_jobs, d_prefix, count);
+    if (blocks)
+        hipLaunchKernelGGL(keccak_leaves_batched_kernel, dim3(blocks), dim3(TREE_THREADS), 0, st, d_jobs, d_prefix,
+                           count);
 }
 
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
