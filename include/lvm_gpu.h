@@ -400,11 +400,11 @@ int lvm_generate_nonce(const uint8_t seed[32], uint8_t grinding_factor, uint64_t
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). Same arguments, result and status
  * codes; it calls no hipMalloc/hipFree and creates no stream. Its scratch (the
- * block minima of one batch of 2^24 candidates, 512 KiB + 8 B) is a fixed
- * device array each GPU holds until the process ends; searches of any length
- * run batch by batch through it, so no input size exceeds it. Needs lvm_init
- * on the current device first (LVM_ERR_STATE otherwise). Calls that overlap
- * on one device share that array and race. */
+ * smallest nonce found so far) is a fixed device word each GPU holds until the
+ * process ends; searches of any length run batch by batch through it, so no
+ * input size exceeds it. Needs lvm_init on the current device first
+ * (LVM_ERR_STATE otherwise). Calls that overlap on one device share that word
+ * and race. */
 int lvm_generate_nonce_noalloc(const uint8_t seed[32], uint8_t grinding_factor, uint64_t max_nonce,
                                uint64_t *nonce_out);
 

@@ -9,17 +9,22 @@
 // reference's sequential search. One thread per candidate; the 40-byte
 // message fits one Keccak-f (lanes 0-3 the inner digest, lane 4 the nonce,
 // padding in lanes 5 and 16). Batches of candidates are searched in
-// increasing order; each block reduces its smallest hit through LDS and
-// writes it with a plain store, so the first batch with a hit gives the
-// answer without atomics.
+// increasing order; a wave lowers one word of device memory, `best`, to its
+// smallest hit, and a wave whose candidates all lie above `best` leaves at
+// once: no smaller hit can be lost, and once one is found the rest of the
+// batch costs its dispatch alone.
 //
-// lvm_generate_nonce_noalloc runs the same kernels with its block minima in a
-// fixed device array (`scratch` below) and reduces them on the device, so a
-// search allocates no memory.
+// The expected search is 2^g candidates, VALU-bound (one permutation each,
+// 2^24 take 1.7 ms). A batch holds 2^(g+2), so that one batch in fifty misses
+// (e^-4), bounded below by one block per CU and above by 2^24. Mean over 24
+// seeds, batches of 2^24 searched in full before: g = 16 1.74 -> 0.058 ms,
+// g = 20 1.67 -> 0.16 ms, g = 22 1.81 -> 0.54 ms.
+//
+// lvm_generate_nonce_noalloc runs the same kernels with `best` in a fixed
+// device word (`scratch` below), so a search allocates no memory.
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <vector>
 
 #include "keccak.hpp"
 #include "lvm_internal.hpp"
@@ -30,27 +35,31 @@ namespace lvm {
 void host_keccak256(const uint8_t *p, size_t n, uint8_t out[32]);
 
 constexpr int GRIND_BLOCK = 256;
-// candidates per launch, and the blocks that take them
-constexpr uint64_t GRIND_BATCH = 1ull << 24;
-constexpr uint64_t GRIND_BLOCKS = GRIND_BATCH / GRIND_BLOCK;
+
+// candidates per launch
+uint64_t grind_batch(unsigned g) { return 1ull << (g + 2 < 16 ? 16 : g + 2 > 24 ? 24 : g + 2); }
 
 // the inner digest as four little-endian lanes, passed by value
 struct GrindDigest {
     uint64_t w[4];
 };
 
-// Scratch of the allocation-free search: words [0, GRIND_BLOCKS) the block
-// minima of one batch, word GRIND_BLOCKS the batch minimum (512 KiB + 8 B per
-// device, held until the process ends). Host code never names it outside
+// `best` of the allocation-free search. Host code never names it outside
 // HIP_SYMBOL(): kernels get its device address from g_scratch_dev.
-static __device__ __align__(256) uint64_t scratch[GRIND_BLOCKS + 1];
+static __device__ __align__(256) uint64_t scratch[1];
+
+__global__ void grind_start_kernel(uint64_t *best) { *best = ~0ull; }
 
 __global__ __launch_bounds__(GRIND_BLOCK) void grind_kernel(GrindDigest inner, uint64_t base, uint64_t count,
-                                                            uint64_t limit, uint64_t *__restrict__ block_min) {
-    __shared__ uint64_t s_min[GRIND_BLOCK];
+                                                            uint64_t limit, uint64_t *best) {
     const uint64_t i = (uint64_t)blockIdx.x * GRIND_BLOCK + threadIdx.x;
     const uint64_t nonce = base + i;
-    uint64_t found = ~0ull;
+    // one load per wave, and one answer for it
+    const uint64_t seen = __hip_atomic_load(best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t cur = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(seen >> 32)) << 32) |
+                         (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)seen);
+    if (cur < nonce - (threadIdx.x & 63)) return;
+    bool hit = false;
     if (i < count) {
         uint32_t l[25], h[25];
 #pragma unroll
@@ -69,36 +78,12 @@ __global__ __launch_bounds__(GRIND_BLOCK) void grind_kernel(GrindDigest inner, u
         h[16] = 0x80000000u;   // byte 135: last padding byte
         keccak_f1600_32(l, h);
         const uint64_t lane0 = ((uint64_t)h[0] << 32) | l[0];
-        if (bswap64(lane0) < limit) found = nonce;
+        hit = bswap64(lane0) < limit;
     }
-    s_min[threadIdx.x] = found;
-    __syncthreads();
-    for (int off = GRIND_BLOCK / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < (unsigned)off) {
-            const uint64_t o = s_min[threadIdx.x + off];
-            if (o < s_min[threadIdx.x]) s_min[threadIdx.x] = o;
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) block_min[blockIdx.x] = s_min[0];
-}
-
-// out[0] = min(block_min[0..blocks)); one block of 1024 threads
-__global__ __launch_bounds__(1024) void grind_min_kernel(const uint64_t *__restrict__ block_min, uint32_t blocks,
-                                                         uint64_t *__restrict__ out) {
-    __shared__ uint64_t s_min[1024];
-    uint64_t m = ~0ull;
-    for (uint32_t b = threadIdx.x; b < blocks; b += 1024) m = block_min[b] < m ? block_min[b] : m;
-    s_min[threadIdx.x] = m;
-    __syncthreads();
-    for (int off = 512; off > 0; off >>= 1) {
-        if (threadIdx.x < (unsigned)off) {
-            const uint64_t o = s_min[threadIdx.x + off];
-            if (o < s_min[threadIdx.x]) s_min[threadIdx.x] = o;
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = s_min[0];
+    // the wave's smallest hit is its lowest lane's
+    const uint64_t mask = __ballot(hit);
+    if (hit && (mask & ((1ull << (threadIdx.x & 63)) - 1)) == 0)
+        __hip_atomic_fetch_min(best, nonce, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 namespace {
@@ -146,40 +131,36 @@ extern "C" int lvm_generate_nonce(const uint8_t seed[32], uint8_t grinding_facto
     hipStream_t st = lib_stream();
     const GrindDigest inner = inner_digest(seed, grinding_factor);
     const uint64_t limit = grinding_factor == 64 ? 1 : (1ull << (64 - grinding_factor));
-    constexpr uint64_t BATCH = GRIND_BATCH;
-    constexpr uint64_t BLOCKS = GRIND_BLOCKS;
-    uint64_t *d_min = nullptr;
-    if (lvm_malloc(&d_min, BLOCKS * 8) != hipSuccess)
+    const uint64_t batch = grind_batch(grinding_factor);
+    uint64_t *d_best = nullptr;
+    if (lvm_malloc(&d_best, 8) != hipSuccess)
         return fail(LVM_ERR_NOMEM, "device allocation for the nonce search failed");
-    std::vector<uint64_t> mins(BLOCKS);
     StageScope ss(st);
     hipError_t e = hipSuccess;
     uint64_t best = ~0ull;
-    for (uint64_t base = 0; e == hipSuccess && base < max_nonce; base += BATCH) {
-        const uint64_t count = max_nonce - base < BATCH ? max_nonce - base : BATCH;
-        const uint64_t blocks = (count + GRIND_BLOCK - 1) / GRIND_BLOCK;
+    hipLaunchKernelGGL(grind_start_kernel, dim3(1), dim3(1), 0, st, d_best);
+    for (uint64_t base = 0; e == hipSuccess && base < max_nonce; base += batch) {
+        const uint64_t count = max_nonce - base < batch ? max_nonce - base : batch;
         {
             ProfScope ps("grinding", st);
-            hipLaunchKernelGGL(grind_kernel, dim3((unsigned)blocks), dim3(GRIND_BLOCK), 0, st, inner, base, count,
-                               limit, d_min);
+            hipLaunchKernelGGL(grind_kernel, dim3((unsigned)((count + GRIND_BLOCK - 1) / GRIND_BLOCK)),
+                               dim3(GRIND_BLOCK), 0, st, inner, base, count, limit, d_best);
         }
         e = hipGetLastError();
-        if (e == hipSuccess) e = stage_download(mins.data(), d_min, blocks * 8, st);
+        if (e == hipSuccess) e = stage_download(&best, d_best, 8, st);
         if (e == hipSuccess) e = stage_sync(st);
-        if (e != hipSuccess) break;
-        for (uint64_t b = 0; b < blocks; b++) best = mins[b] < best ? mins[b] : best;
-        if (best != ~0ull) break;
-        if (base + BATCH < base) break;  // wrapped
+        if (e != hipSuccess || best != ~0ull) break;
+        if (base + batch < base) break;  // wrapped
     }
-    lvm_free(d_min);
+    lvm_free(d_best);
     if (e != hipSuccess) return fail(LVM_ERR_DEVICE, std::string("nonce search failed: ") + hipGetErrorString(e));
     if (best == ~0ull) return fail(LVM_ERR_STATE, "no valid nonce below the search limit");
     *nonce_out = best;
     return LVM_OK;
 }
 
-// The same search with no allocation: block minima in the device's `scratch`
-// array, reduced on the device; one 8-byte copy per batch to the host. Needs
+// The same search with no allocation: `best` in the device's `scratch` word;
+// one 8-byte copy per batch to the host. Needs
 // lvm_init on this device first (it resolves the scratch address). Calls that
 // overlap on one device share its scratch and race.
 extern "C" int lvm_generate_nonce_noalloc(const uint8_t seed[32], uint8_t grinding_factor, uint64_t max_nonce,
@@ -202,18 +183,17 @@ extern "C" int lvm_generate_nonce_noalloc(const uint8_t seed[32], uint8_t grindi
     const uint64_t limit = grinding_factor == 64 ? 1 : (1ull << (64 - grinding_factor));
     hipError_t e = hipSuccess;
     uint64_t best = ~0ull;
-    for (uint64_t base = 0; base < max_nonce; base += GRIND_BATCH) {
-        const uint64_t count = max_nonce - base < GRIND_BATCH ? max_nonce - base : GRIND_BATCH;
-        const uint64_t blocks = (count + GRIND_BLOCK - 1) / GRIND_BLOCK;  // <= GRIND_BLOCKS
-        hipLaunchKernelGGL(grind_kernel, dim3((unsigned)blocks), dim3(GRIND_BLOCK), 0, st, inner, base, count, limit,
-                           sc);
-        hipLaunchKernelGGL(grind_min_kernel, dim3(1), dim3(1024), 0, st, (const uint64_t *)sc, (uint32_t)blocks,
-                           sc + GRIND_BLOCKS);
+    const uint64_t batch = grind_batch(grinding_factor);
+    hipLaunchKernelGGL(grind_start_kernel, dim3(1), dim3(1), 0, st, sc);
+    for (uint64_t base = 0; base < max_nonce; base += batch) {
+        const uint64_t count = max_nonce - base < batch ? max_nonce - base : batch;
+        hipLaunchKernelGGL(grind_kernel, dim3((unsigned)((count + GRIND_BLOCK - 1) / GRIND_BLOCK)), dim3(GRIND_BLOCK),
+                           0, st, inner, base, count, limit, sc);
         e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(&best, sc + GRIND_BLOCKS, 8, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(&best, sc, 8, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess || best != ~0ull) break;
-        if (base + GRIND_BATCH < base) break;  // wrapped
+        if (base + batch < base) break;  // wrapped
     }
     if (e != hipSuccess) return fail(LVM_ERR_DEVICE, std::string("nonce search failed: ") + hipGetErrorString(e));
     if (best == ~0ull) return fail(LVM_ERR_STATE, "no valid nonce below the search limit");
