@@ -354,6 +354,26 @@ LVM_HD void acc_mad(acc128 &a, uint64_t x, uint64_t y) {
 #endif
 }
 
+// the same with a factor x that every lane of the wave shares (scalar registers)
+__device__ __forceinline__ void acc_mad_uniform(acc128 &a, uint64_t x, uint64_t y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t a0 = (uint32_t)x, a1 = (uint32_t)(x >> 32), b0 = (uint32_t)y, b1 = (uint32_t)(y >> 32);
+    uint64_t cy;
+    asm("v_mad_u64_u32 %0, %6, %7, %9, %0\n\t"
+        "v_addc_co_u32 %3, %6, 0, %3, %6\n\t"
+        "v_mad_u64_u32 %1, %6, %7, %10, %1\n\t"
+        "v_addc_co_u32 %4, %6, 0, %4, %6\n\t"
+        "v_mad_u64_u32 %1, %6, %8, %9, %1\n\t"
+        "v_addc_co_u32 %4, %6, 0, %4, %6\n\t"
+        "v_mad_u64_u32 %2, %6, %8, %10, %2\n\t"
+        "v_addc_co_u32 %5, %6, 0, %5, %6"
+        : "+v"(a.s0), "+v"(a.s1), "+v"(a.s2), "+v"(a.c0), "+v"(a.c1), "+v"(a.c2), "=&s"(cy)
+        : "s"(a0), "s"(a1), "v"(b0), "v"(b1));
+#else
+    acc_mad(a, x, y);
+#endif
+}
+
 // value = s0 + c0*2^64 + s1*2^32 + c1*2^96 + s2*2^64 + c2*2^128 (mod p), with
 // 2^64 = EPS, 2^96 = -1, 2^128 = EPS^2
 LVM_HD uint64_t acc_reduce(const acc128 &a) {

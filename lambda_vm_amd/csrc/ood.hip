@@ -175,73 +175,85 @@ static void launch_pole_inverse(uint64_t *out, uint64_t rows, uint32_t log_N, ui
 }
 
 constexpr int BARY_MAX_K = 8;
-constexpr uint64_t BARY_MAX_ROWS_PER_BLOCK = 1024;
-
 // partial[chunk][k][c] = sum over the chunk's rows p of lde[p][c] * scale[k][p]
-// block: 256 threads = 4 row lanes x 64 columns; grid (chunks, column groups),
-// a chunk being `rpb` consecutive rows (fewer for small tables, so that the
-// grid still has enough blocks; each thread walks rpb/4 rows, loads of four
-// rows issued together). The three components of each point's sum are
-// delayed-reduction dot products (one 128-bit accumulate per product, one
-// reduction per thread).
+// block: 256 threads over min(w, 256) adjacent columns and as many rows RB at
+// once as fit (thread = row * columns + column, so a block's loads are runs of
+// whole rows and no lane idles on a narrow table: with 64 lanes a row, 17
+// columns used 17 of them); grid (chunks of rpb rows, groups of 256 columns).
+// The three components of each point's sum are delayed-reduction dot products
+// (one 128-bit accumulate per product, one reduction per thread), loads of U
+// rows issued together; the RB partial sums of a column meet in LDS.
+__host__ __device__ inline uint32_t bary_cols(uint64_t w) { return w < 256 ? (uint32_t)w : 256u; }
+
 template <int K>
-__global__ __launch_bounds__(256) void bary_partial_kernel(const uint64_t *__restrict__ lde, uint64_t pitch,
-                                                           uint64_t w, uint64_t n, uint64_t rpb,
-                                                           const uint64_t *__restrict__ scale,
+__global__ __launch_bounds__(256) void bary_partial_kernel(const uint64_t *__restrict__ lde, uint64_t w, uint64_t n,
+                                                           uint64_t rpb, const uint64_t *__restrict__ scale,
                                                            uint64_t *__restrict__ partial) {
-    __shared__ uint64_t red[4][K][64][3];
-    const int lane = threadIdx.x & 63, rl = threadIdx.x >> 6;
-    const uint64_t c = (uint64_t)blockIdx.y * 64 + lane;
-    const uint64_t p0 = (uint64_t)blockIdx.x * rpb;
+    constexpr int U = K <= 2 ? 4 : 2;
+    __shared__ uint64_t red[256][3];
+    const uint32_t t = threadIdx.x;
+    const uint64_t c0 = (uint64_t)blockIdx.y * 256;
+    const uint32_t wc = bary_cols(w - c0), RB = 256 / wc;
+    const uint32_t r = t / wc, c = t - r * wc;
+    const uint64_t p0 = (uint64_t)blockIdx.x * rpb, pend = p0 + rpb < n ? p0 + rpb : n;
     acc128 acc[K][3];
 #pragma unroll
     for (int k = 0; k < K; k++)
 #pragma unroll
         for (int j = 0; j < 3; j++) acc_zero(acc[k][j]);
-    if (c < w) {
-        const uint64_t pend = p0 + rpb < n ? p0 + rpb : n;
-        auto row = [&](uint64_t p, uint64_t f) {
-            // p is the same for the 64 lanes of a wave: read the scales through
-            // the scalar path once per wave instead of 64 identical vector loads
-            const uint64_t pu = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(p >> 32)) << 32) |
-                                __builtin_amdgcn_readfirstlane((uint32_t)p);
+    if (r < RB) {
+        const gmem_u64 *f = LVM_GLOBAL_CONST(lde) + c0 + c;
+        const gmem_u64 *sc = LVM_GLOBAL_CONST(scale);
+        uint64_t p = p0 + r;
+        for (; p + (U - 1) * RB < pend; p += U * RB) {
+            uint64_t v[U], s[U][K][3];
 #pragma unroll
-            for (int k = 0; k < K; k++) {
-                const uint64_t *s = scale + 3 * (k * n + pu);
-                acc_mad(acc[k][0], s[0], f);
-                acc_mad(acc[k][1], s[1], f);
-                acc_mad(acc[k][2], s[2], f);
+            for (int u = 0; u < U; u++) {
+                const uint64_t q = p + u * RB;
+                v[u] = f[q * w];
+#pragma unroll
+                for (int k = 0; k < K; k++)
+#pragma unroll
+                    for (int j = 0; j < 3; j++) s[u][k][j] = sc[3 * (k * n + q) + j];
             }
-        };
-        uint64_t p = p0 + rl;
-        for (; p + 12 < pend; p += 16) {
-            const uint64_t f0 = lde[p * pitch + c], f1 = lde[(p + 4) * pitch + c];
-            const uint64_t f2 = lde[(p + 8) * pitch + c], f3 = lde[(p + 12) * pitch + c];
-            row(p, f0);
-            row(p + 4, f1);
-            row(p + 8, f2);
-            row(p + 12, f3);
+            __builtin_amdgcn_sched_barrier(0);  // all U rows' loads before the first product
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int k = 0; k < K; k++)
+#pragma unroll
+                    for (int j = 0; j < 3; j++) acc_mad(acc[k][j], s[u][k][j], v[u]);
         }
-        for (; p < pend; p += 4) row(p, lde[p * pitch + c]);
+        for (; p < pend; p += RB) {
+            const uint64_t v = f[p * w];
+#pragma unroll
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) acc_mad(acc[k][j], sc[3 * (k * n + p) + j], v);
+        }
     }
 #pragma unroll
-    for (int k = 0; k < K; k++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) red[rl][k][lane][j] = acc_reduce(acc[k][j]);
-    __syncthreads();
-    if (rl == 0 && c < w) {
-        for (int k = 0; k < K; k++) {
-            fp3 s = fp3{red[0][k][lane][0], red[0][k][lane][1], red[0][k][lane][2]};
-            for (int r = 1; r < 4; r++) s = f3_add(s, fp3{red[r][k][lane][0], red[r][k][lane][1], red[r][k][lane][2]});
-            st3(partial + 3 * (((uint64_t)blockIdx.x * K + k) * w + c), s);
+    for (int k = 0; k < K; k++) {
+        fp3 v = fp3{acc_reduce(acc[k][0]), acc_reduce(acc[k][1]), acc_reduce(acc[k][2])};
+        st3(red[t], v);
+        for (uint32_t left = RB; left > 1;) {
+            const uint32_t half = (left + 1) / 2;
+            __syncthreads();
+            if (r + half < left) {
+                v = f3_add(v, ld3(red[t + half * wc]));
+                st3(red[t], v);
+            }
+            left = half;
         }
+        if (r == 0) st3(partial + 3 * (((uint64_t)blockIdx.x * K + k) * w + c0 + c), v);
+        __syncthreads();  // the sums are rewritten for the next point
     }
 }
 
 template <int K>
 static void launch_bary_partial(dim3 grid, hipStream_t st, const uint64_t *lde, uint64_t w, uint64_t n,
                                 uint64_t rpb, const uint64_t *scale, uint64_t *partial) {
-    hipLaunchKernelGGL(bary_partial_kernel<K>, grid, dim3(256), 0, st, lde, w, w, n, rpb, scale, partial);
+    hipLaunchKernelGGL(bary_partial_kernel<K>, grid, dim3(256), 0, st, lde, w, n, rpb, scale, partial);
 }
 
 // out[k][c] = vf[k] * sum over chunks of partial[chunk][k][c]; one block per
@@ -277,104 +289,148 @@ __global__ __launch_bounds__(256) void bary_combine_kernel(const uint64_t *parti
 // computed once on the host, main columns are base words, aux and parts are
 // Fp3 (3 words each).
 constexpr int DEEP_MAX_K = 4;
-constexpr int DEEP_CHUNK = 16;  // main columns staged per LDS round
-// block: 256 consecutive physical rows. The main (base) columns of the block
-// are staged through LDS 16 at a time with coalesced row-segment loads; each
-// thread accumulates sum_j gt_{j,k} * t_j[p] as 3*KA delayed-reduction dot
-// products. KA < K when the trace-term weights are geometric in k past the
-// first KA - 1 points (gt_{j,k} = gt_{j,KA-1} * r^(k-KA+1) for every column j,
-// which the reference's weights are: gamma^(W + j(K-1) + k - 1) for k >= 1,
-// crypto/stark/src/prover.rs:2400-2460): then sum_j gt_{j,k} t_j = r^(k-KA+1)
-// * sum_j gt_{j,KA-1} t_j, and rpow[k] holds r^(k-KA+1).
+constexpr int DEEP_CHUNK = 16;  // most columns staged per LDS round
+
+// An Fp3 column a = a0 + a1 w + a2 w^2 weighted by g is three base columns
+// weighted by g, w g and w^2 g, so every table is a segment of base columns.
+struct DeepSegment {
+    const uint64_t *rows;
+    uint64_t cols;  // words per row
+};
+struct DeepArgs {
+    uint64_t N;
+    DeepSegment trace[2], parts;  // main and aux trace words, composition parts words
+    const uint64_t *gtr;          // [trace word][KA][3]
+    const uint64_t *gh;           // [parts word][3]
+    const uint64_t *consts;       // ct_k, then ch
+    const uint64_t *rpow;
+    const uint64_t *inv_den;      // [pole][N][3]
+    uint64_t *out;
+};
+
+// block: 256 consecutive physical rows. A chunk of columns of those rows goes
+// through LDS with coalesced row-segment loads (the next chunk's loads are
+// issued before the current chunk is accumulated); each thread accumulates
+// its row's sum_j gt_{j,k} * t_j[p] as 3*KA delayed-reduction dot products.
+// The weights are the same for every row: scalar loads and scalar operands.
+// A zero weight is skipped (a bus table opens one column at its next row, so
+// all its other weights of k = 1 are zero). KA < K when the trace-term weights
+// are geometric in k past the first KA - 1 points (gt_{j,k} = gt_{j,KA-1} *
+// r^(k-KA+1) for every column j, which the reference's weights are: gamma^(W +
+// j(K-1) + k - 1) for k >= 1, crypto/stark/src/prover.rs:2400-2460): then
+// sum_j gt_{j,k} t_j = r^(k-KA+1) * sum_j gt_{j,KA-1} t_j, and rpow[k] holds
+// r^(k-KA+1).
 template <int K, int KA>
-__global__ __launch_bounds__(256) void deep_kernel(uint64_t N, const uint64_t *__restrict__ main_lde, uint64_t wm,
-                                                   const uint64_t *__restrict__ aux_lde, uint64_t wa,
-                                                   const uint64_t *__restrict__ parts_lde, uint64_t np,
-                                                   const uint64_t *__restrict__ gtr, const uint64_t *__restrict__ gh,
-                                                   const uint64_t *__restrict__ consts,
-                                                   const uint64_t *__restrict__ rpow,
-                                                   const uint64_t *__restrict__ inv_den, uint64_t *__restrict__ out) {
+__global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
     __shared__ uint64_t tile[256][DEEP_CHUNK + 1];
-    __shared__ uint64_t sg[DEEP_CHUNK][KA][3];
     const int t = threadIdx.x;
-    const uint64_t r0 = (uint64_t)blockIdx.x * 256;
-    const uint64_t p = r0 + t;
+    const uint64_t N = a.N, r0 = (uint64_t)blockIdx.x * 256, p = r0 + t;
+    uint64_t nv[DEEP_CHUNK];
+    // columns [j0, j0 + cw) of the block's rows: thread t loads column t % 16 of
+    // rows t / 16, t / 16 + 16, ... (16 lanes per row segment)
+    const uint32_t lc = t & 15, lr = t >> 4;
+    const uint32_t rows = N - r0 < 256 ? (uint32_t)(N - r0) : 256u;  // a power of two
+    auto fetch = [&](const DeepSegment &s, uint32_t j0, uint32_t cw) {
+        if (lc >= cw || lr >= rows) return;
+        const gmem_u64 *src = LVM_GLOBAL_CONST(s.rows) + (r0 + lr) * s.cols + j0 + lc;
+        const uint64_t step = 16 * s.cols;
+        if (rows == 256) {
+#pragma unroll
+            for (int q = 0; q < 16; q++) nv[q] = src[q * step];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                if (16u * q < rows) nv[q] = src[q * step];
+        }
+    };
+    auto stage = [&]() {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 16; q++) tile[lr + 16 * q][lc] = nv[q];
+        __syncthreads();
+    };
+    // acc[k] += w_k * (the thread's value) over the chunk's columns; a column's
+    // weights are loaded while the previous one is accumulated
+    auto accumulate = [&](auto &acc, const uint64_t *w, uint32_t cw) {
+        constexpr int NK = sizeof(acc) / sizeof(acc[0]);
+        uint64_t g[3 * NK];
+#pragma unroll
+        for (int i = 0; i < 3 * NK; i++) g[i] = w[i];
+        for (uint32_t cc = 0; cc < cw; cc++) {
+            const uint64_t v = tile[t][cc];
+            uint64_t cur[3 * NK];
+#pragma unroll
+            for (int i = 0; i < 3 * NK; i++) cur[i] = g[i];
+            w += cc + 1 < cw ? 3 * NK : 0;
+#pragma unroll
+            for (int i = 0; i < 3 * NK; i++) g[i] = w[i];
+#pragma unroll
+            for (int k = 0; k < NK; k++) {
+                if (cur[3 * k] | cur[3 * k + 1] | cur[3 * k + 2]) {
+#pragma unroll
+                    for (int j = 0; j < 3; j++) acc_mad_uniform(acc[k][j], cur[3 * k + j], v);
+                }
+            }
+        }
+    };
+    // equal chunks of at most DEEP_CHUNK columns
+    auto width = [](uint64_t cols) -> uint32_t {
+        const uint32_t n = (uint32_t)((cols + DEEP_CHUNK - 1) / DEEP_CHUNK);
+        return n ? (uint32_t)((cols + n - 1) / n) : 0;
+    };
     acc128 acc[KA][3];
 #pragma unroll
     for (int k = 0; k < KA; k++)
 #pragma unroll
         for (int j = 0; j < 3; j++) acc_zero(acc[k][j]);
-    // the block's 256 rows x DEEP_CHUNK columns are DEEP_CHUNK values per
-    // thread; the next chunk's loads are issued before the current chunk is
-    // accumulated, so they are in flight during the products
-    uint64_t nv[DEEP_CHUNK];
-    auto fetch = [&](uint64_t j0) {
-        const int cw = (int)(wm - j0 < DEEP_CHUNK ? wm - j0 : DEEP_CHUNK);
-#pragma unroll
-        for (int q = 0; q < DEEP_CHUNK; q++) {
-            const int e = t + 256 * q, rr = e / DEEP_CHUNK, cc = e % DEEP_CHUNK;
-            nv[q] = (cc < cw && r0 + rr < N) ? main_lde[(r0 + rr) * wm + j0 + cc] : 0;
-        }
-    };
-    if (wm) fetch(0);
-    for (uint64_t j0 = 0; j0 < wm; j0 += DEEP_CHUNK) {
-        const int cw = (int)(wm - j0 < DEEP_CHUNK ? wm - j0 : DEEP_CHUNK);
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < DEEP_CHUNK; q++) {
-            const int e = t + 256 * q;
-            tile[e / DEEP_CHUNK][e % DEEP_CHUNK] = nv[q];
-        }
-        for (int e = t; e < DEEP_CHUNK * KA * 3; e += 256) {
-            const int cc = e / (KA * 3), rem = e % (KA * 3);
-            sg[cc][rem / 3][rem % 3] = cc < cw ? gtr[3 * ((j0 + cc) * K + rem / 3) + rem % 3] : 0;
-        }
-        __syncthreads();
-        if (j0 + DEEP_CHUNK < wm) fetch(j0 + DEEP_CHUNK);
-#pragma unroll 4
-        for (int cc = 0; cc < DEEP_CHUNK; cc++) {
-            const uint64_t v = tile[t][cc];
-#pragma unroll
-            for (int k = 0; k < KA; k++) {
-                acc_mad(acc[k][0], sg[cc][k][0], v);
-                acc_mad(acc[k][1], sg[cc][k][1], v);
-                acc_mad(acc[k][2], sg[cc][k][2], v);
-            }
+    const uint64_t *w = a.gtr;
+    for (int sgi = 0; sgi < 2; sgi++) {
+        const DeepSegment s = a.trace[sgi];
+        const uint32_t cols = (uint32_t)s.cols, cm = width(cols);
+        if (!cols) continue;
+        fetch(s, 0, cm);
+        for (uint32_t j0 = 0; j0 < cols; j0 += cm) {
+            const uint32_t cw = cols - j0 < cm ? cols - j0 : cm;
+            stage();
+            const uint32_t next = j0 + cm;
+            if (next < cols) fetch(s, next, cols - next < cm ? cols - next : cm);
+            accumulate(acc, w, cw);
+            w += (uint64_t)cw * 3 * KA;
         }
     }
-    if (p >= N) return;
     fp3 tk[K];
 #pragma unroll
     for (int k = 0; k < KA; k++) tk[k] = fp3{acc_reduce(acc[k][0]), acc_reduce(acc[k][1]), acc_reduce(acc[k][2])};
-    if (aux_lde) {
-        const uint64_t *arow = aux_lde + p * 3 * wa;
-        for (uint64_t j = 0; j < wa; j++) {
-            fp3 v = ld3(arow + 3 * j);
 #pragma unroll
-            for (int k = 0; k < KA; k++) tk[k] = f3_add(tk[k], f3_mul(ld3(gtr + 3 * ((wm + j) * K + k)), v));
+    for (int k = KA; k < K; k++) tk[k] = f3_mul(ld3(a.rpow + 3 * k), tk[KA - 1]);
+    fp3 r = fp3{0, 0, 0};
+    if (p < N) {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            r = f3_add(r, f3_mul(ld3(a.inv_den + 3 * (k * N + p)), f3_sub(tk[k], ld3(a.consts + 3 * k))));
+    }
+    if (a.parts.cols) {
+        const uint32_t cols = (uint32_t)a.parts.cols, cm = width(cols);
+        acc128 ha[1][3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) acc_zero(ha[0][j]);
+        for (uint32_t j0 = 0; j0 < cols; j0 += cm) {
+            const uint32_t cw = cols - j0 < cm ? cols - j0 : cm;
+            fetch(a.parts, j0, cw);
+            stage();
+            accumulate(ha, a.gh + 3 * j0, cw);
+        }
+        if (p < N) {
+            const fp3 hs = fp3{acc_reduce(ha[0][0]), acc_reduce(ha[0][1]), acc_reduce(ha[0][2])};
+            r = f3_add(r, f3_mul(ld3(a.inv_den + 3 * (K * N + p)), f3_sub(hs, ld3(a.consts + 3 * K))));
         }
     }
-#pragma unroll
-    for (int k = KA; k < K; k++) tk[k] = f3_mul(ld3(rpow + 3 * k), tk[KA - 1]);
-    fp3 r = fp3{0, 0, 0};
-#pragma unroll
-    for (int k = 0; k < K; k++)
-        r = f3_add(r, f3_mul(ld3(inv_den + 3 * (k * N + p)), f3_sub(tk[k], ld3(consts + 3 * k))));
-    if (parts_lde && np) {
-        fp3 hs = fp3{0, 0, 0};
-        const uint64_t *prow = parts_lde + p * 3 * np;
-        for (uint64_t j = 0; j < np; j++) hs = f3_add(hs, f3_mul(ld3(gh + 3 * j), ld3(prow + 3 * j)));
-        r = f3_add(r, f3_mul(ld3(inv_den + 3 * (K * N + p)), f3_sub(hs, ld3(consts + 3 * K))));
-    }
-    st3(out + 3 * p, r);
+    if (p < N) st3(a.out + 3 * p, r);
 }
 
 template <int K, int KA>
-static void launch_deep(hipStream_t st, uint64_t N, const uint64_t *main_lde, uint64_t wm, const uint64_t *aux_lde,
-                        uint64_t wa, const uint64_t *parts_lde, uint64_t np, const uint64_t *gtr, const uint64_t *gh,
-                        const uint64_t *consts, const uint64_t *rpow, const uint64_t *inv_den, uint64_t *out) {
-    hipLaunchKernelGGL((deep_kernel<K, KA>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, N, main_lde, wm,
-                       aux_lde, wa, parts_lde, np, gtr, gh, consts, rpow, inv_den, out);
+static void launch_deep(hipStream_t st, const DeepArgs &a) {
+    hipLaunchKernelGGL((deep_kernel<K, KA>), dim3((unsigned)((a.N + 255) / 256)), dim3(256), 0, st, a);
 }
 }  // namespace lvm
 
@@ -469,11 +525,10 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
     const unsigned logN = log2u(h->N);
     Scratch s;
     uint64_t *dz, *scale, *partial, *vfd, *dout;
-    // rows per block: 1024, fewer (down to 64) when the grid would have under
-    // ~1024 blocks
-    const uint64_t cgroups = (w + 63) / 64;
-    uint64_t rpb = BARY_MAX_ROWS_PER_BLOCK;
-    while (rpb > 64 && ((n + rpb - 1) / rpb) * cgroups < 1024) rpb /= 2;
+    // 64 rows per thread, fewer (down to 4) when the grid would have under 1024 blocks
+    const uint64_t cgroups = (w + 255) / 256, RB = 256 / bary_cols(w);
+    uint64_t rpb = 64 * RB;
+    while (rpb > 4 * RB && ((n + rpb - 1) / rpb) * cgroups < 1024) rpb /= 2;
     const uint64_t chunks = (n + rpb - 1) / rpb;
     TRYS(s.get(&dz, K * 24));
     TRYS(s.get(&scale, K * n * 24));
@@ -500,7 +555,7 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
     }
     {
         ProfScope ps("bary_sum", st);
-        dim3 grid((unsigned)chunks, (unsigned)((w + 63) / 64));
+        dim3 grid((unsigned)chunks, (unsigned)cgroups);
         switch (K) {
         case 1: launch_bary_partial<1>(grid, st, h->lde, w, n, rpb, scale, partial); break;
         case 2: launch_bary_partial<2>(grid, st, h->lde, w, n, rpb, scale, partial); break;
@@ -581,22 +636,49 @@ int lvm_deep_composition(const lvm_lde *main, const lvm_lde *aux, const lvm_lde 
                 }
         }
     }
+    // the weights by base word: an Fp3 column's three words weigh g, w g, w^2 g
+    const uint32_t KA = geo ? 2 : (uint32_t)K;
+    const uint64_t words = wm + 3 * wa;
+    std::vector<uint64_t> wt(3 * KA * words), wh(9 * np);
+    auto times_w = [](const uint64_t *g, uint64_t *o) {  // w g (w^3 = 2)
+        const uint64_t g0 = g[0], g1 = g[1], g2 = g[2];
+        o[0] = dbl(g2);
+        o[1] = g0;
+        o[2] = g1;
+    };
+    for (uint64_t j = 0; j < cols; j++)
+        for (uint32_t k = 0; k < KA; k++) {
+            const uint64_t *g = gammas_tr + 3 * (j * K + k);
+            const uint64_t w0 = j < wm ? j : wm + 3 * (j - wm);
+            std::memcpy(&wt[3 * (w0 * KA + k)], g, 24);
+            if (j >= wm) {
+                times_w(&wt[3 * (w0 * KA + k)], &wt[3 * ((w0 + 1) * KA + k)]);
+                times_w(&wt[3 * ((w0 + 1) * KA + k)], &wt[3 * ((w0 + 2) * KA + k)]);
+            }
+        }
+    for (uint64_t j = 0; j < np; j++) {
+        std::memcpy(&wh[9 * j], gammas_h + 3 * j, 24);
+        times_w(&wh[9 * j], &wh[9 * j + 3]);
+        times_w(&wh[9 * j + 3], &wh[9 * j + 6]);
+    }
     Scratch s;
-    uint64_t *dpoles, *inv_den, *dconsts, *dgtr, *drp, *dgh = nullptr;
+    uint64_t *dpoles, *inv_den, *dargs;
     TRYS(s.get(&dpoles, npoles * 24));
     TRYS(s.get(&inv_den, (uint64_t)npoles * N * 24));
-    TRYS(s.get(&dconsts, (K + 1) * 24));
-    TRYS(s.get(&dgtr, cols * K * 24));
-    TRYS(s.get(&drp, K * 24));
+    // consts, powers and weights in one upload
+    std::vector<uint64_t> blob;
+    auto put = [&](const void *p, size_t bytes) {
+        const size_t at = blob.size();
+        blob.resize(at + (bytes + 7) / 8);
+        if (bytes) std::memcpy(&blob[at], p, bytes);
+        return at;
+    };
+    const size_t o_consts = put(consts.data(), (K + 1) * 24), o_rp = put(rp.data(), K * 24);
+    const size_t o_wt = put(wt.data(), wt.size() * 8), o_wh = put(wh.data(), wh.size() * 8);
+    TRYS(s.get(&dargs, blob.size() * 8));
     StageScope ss(st);
     LVM_HIP(stage_upload(dpoles, poles.data(), npoles * 24, st));
-    LVM_HIP(stage_upload(dconsts, consts.data(), (K + 1) * 24, st));
-    LVM_HIP(stage_upload(dgtr, gammas_tr, cols * K * 24, st));
-    LVM_HIP(stage_upload(drp, rp.data(), K * 24, st));
-    if (parts) {
-        TRYS(s.get(&dgh, np * 24));
-        LVM_HIP(stage_upload(dgh, gammas_h, np * 24, st));
-    }
+    LVM_HIP(stage_upload(dargs, blob.data(), blob.size() * 8, st));
     {
         ProfScope ps("deep_denoms", st);
         // 1 / (x - z) (XMinusZ, crypto/math-cuda/src/inverse.rs:241-300)
@@ -604,15 +686,18 @@ int lvm_deep_composition(const lvm_lde *main, const lvm_lde *aux, const lvm_lde 
     }
     {
         ProfScope ps("deep_rows", st);
-        const uint64_t *al = aux ? aux->lde : nullptr, *pl = parts ? parts->lde : nullptr;
-        const uint64_t *m = main->lde;
+        const DeepArgs a{N,
+                         {{main->lde, wm}, {aux ? aux->lde : nullptr, 3 * wa}},
+                         {parts ? parts->lde : nullptr, 3 * np},
+                         dargs + o_wt, dargs + o_wh, dargs + o_consts,
+                         dargs + o_rp, inv_den, dev_out};
         switch (K * 2 + (geo ? 1 : 0)) {
-        case 2: launch_deep<1, 1>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
-        case 4: launch_deep<2, 2>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
-        case 6: launch_deep<3, 3>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
-        case 7: launch_deep<3, 2>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
-        case 8: launch_deep<4, 4>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
-        default: launch_deep<4, 2>(st, N, m, wm, al, wa, pl, np, dgtr, dgh, dconsts, drp, inv_den, dev_out); break;
+        case 2: launch_deep<1, 1>(st, a); break;
+        case 4: launch_deep<2, 2>(st, a); break;
+        case 6: launch_deep<3, 3>(st, a); break;
+        case 7: launch_deep<3, 2>(st, a); break;
+        case 8: launch_deep<4, 4>(st, a); break;
+        default: launch_deep<4, 2>(st, a); break;
         }
     }
     LVM_HIP(hipGetLastError());
