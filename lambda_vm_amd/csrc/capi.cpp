@@ -114,8 +114,8 @@ int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blow
     uint64_t C;
     {
         ProfScope ps("keccak_leaves", st);
-        C = keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, nodes.as<uint8_t>(), st);
-        if (split) keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, pre.as<uint8_t>(), st);
+        C = keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, true, nodes.as<uint8_t>(), st);
+        if (split) keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, true, pre.as<uint8_t>(), st);
     }
     {
         ProfScope ps("merkle_inner", st);
@@ -353,7 +353,7 @@ int commit_owned_rows(Device *d, hipStream_t st, DevBuf &rows, size_t N, size_t 
     uint64_t C;
     {
         ProfScope ps("keccak_leaves", st);
-        C = keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, nodes.as<uint8_t>(), st);
+        C = keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, false, nodes.as<uint8_t>(), st);
     }
     {
         ProfScope ps("merkle_inner", st);

@@ -82,7 +82,7 @@ __device__ __forceinline__ void fri_fold_body(const FoldJob &j, uint64_t t, cons
         }
         l[6] = 0x01;
         h[16] = 0x80000000u;
-        keccak_f1600_32<true>(l, h);  // small layers are latency-bound: rounds unrolled
+        keccak_f1600_32_digest<true>(l, h);
         uint64_t *o = leaves + 4 * t;
 #pragma unroll
         for (int k = 0; k < 4; k++) o[k] = ((uint64_t)h[k] << 32) | l[k];

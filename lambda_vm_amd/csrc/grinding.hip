@@ -76,7 +76,7 @@ __global__ __launch_bounds__(GRIND_BLOCK) void grind_kernel(GrindDigest inner, u
         h[4] = (uint32_t)(nb >> 32);
         l[5] = 0x01;           // byte 40: first padding byte
         h[16] = 0x80000000u;   // byte 135: last padding byte
-        keccak_f1600_32(l, h);
+        keccak_f1600_32_digest<true>(l, h);
         const uint64_t lane0 = ((uint64_t)h[0] << 32) | l[0];
         hit = bswap64(lane0) < limit;
     }

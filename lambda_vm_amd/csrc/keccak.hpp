@@ -2,7 +2,10 @@
 // for gfx950. Each 64-bit lane is held as two 32-bit VGPRs (lo, hi):
 //  - column parities and theta use v_bitop3_b32 as a 3-input XOR (LUT 0x96),
 //    and the theta term D[x] is folded into the per-lane XOR (A ^ C[x-1] ^
-//    rot(C[x+1], 1) is one 3-input XOR per half);
+//    rot(C[x+1], 1) is one 3-input XOR per half). v_xor_b32 alone issues every
+//    2.9 cycles per wave against 4.7 for v_bitop3_b32, but not in this mix:
+//    parities of two-input XORs measured slower (row-pair leaves of 2^24 x 64:
+//    8.27 against 7.7-7.9 ms), D[x] formed first and XORed in the same;
 //  - a 64-bit rotate is two v_alignbit_b32 (funnel shifts of the halves);
 //  - chi, a ^ (~b & c), is one v_bitop3_b32 per half (LUT 0xD2 for
 //    operands (a, b, c), i.e. f(0xF0, 0xCC, 0xAA)).
@@ -26,6 +29,10 @@ __constant__ static const uint32_t KECCAK_RC_HI[24] = {
     0x80000000u, 0x80000000u, 0x00000000u, 0x80000000u, 0x80000000u, 0x80000000u, 0x00000000u, 0x80000000u};
 
 __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    // lanes known to be zero (the first round of a one-block message) drop out
+    if (__builtin_constant_p(a) && a == 0) return b ^ c;
+    if (__builtin_constant_p(b) && b == 0) return a ^ c;
+    if (__builtin_constant_p(c) && c == 0) return a ^ b;
     return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
 }
 // a ^ (~b & c)
@@ -51,6 +58,18 @@ __device__ __forceinline__ void rotl(uint32_t hi, uint32_t lo, uint32_t &oh, uin
     }
 }
 
+// C[x] and rot(C[x], 1) of theta
+__device__ __forceinline__ void theta_c(const uint32_t l[25], const uint32_t h[25], uint32_t Cl[5], uint32_t Ch[5],
+                                        uint32_t Rl[5], uint32_t Rh[5]) {
+#pragma unroll
+    for (int x = 0; x < 5; x++) {
+        Cl[x] = xor3(xor3(l[x], l[x + 5], l[x + 10]), l[x + 15], l[x + 20]);
+        Ch[x] = xor3(xor3(h[x], h[x + 5], h[x + 10]), h[x + 15], h[x + 20]);
+    }
+#pragma unroll
+    for (int x = 0; x < 5; x++) rotl<1>(Ch[x], Cl[x], Rh[x], Rl[x]);
+}
+
 // B[dst] = rot(A[src] ^ C[x-1] ^ rot(C[x+1], 1), R) where x = src % 5
 #define LVM_KB(dst, src, R)                                                                      \
     rotl<R>(xor3(h[src], Ch[((src) + 4) % 5], Rh[((src) + 1) % 5]),                             \
@@ -59,13 +78,7 @@ __device__ __forceinline__ void rotl(uint32_t hi, uint32_t lo, uint32_t &oh, uin
 // one round (theta, rho, pi, chi, iota) on the 32-bit halves
 __device__ __forceinline__ void keccak_round_32(uint32_t l[25], uint32_t h[25], int round) {
     uint32_t Cl[5], Ch[5], Rl[5], Rh[5];
-#pragma unroll
-    for (int x = 0; x < 5; x++) {
-        Cl[x] = xor3(xor3(l[x], l[x + 5], l[x + 10]), l[x + 15], l[x + 20]);
-        Ch[x] = xor3(xor3(h[x], h[x + 5], h[x + 10]), h[x + 15], h[x + 20]);
-    }
-#pragma unroll
-    for (int x = 0; x < 5; x++) rotl<1>(Ch[x], Cl[x], Rh[x], Rl[x]);
+    theta_c(l, h, Cl, Ch, Rl, Rh);
     uint32_t bl[25], bh[25];
     // theta + rho + pi: B[y, 2x+3y] = rot(A[x,y] ^ D[x], r[x,y]), lane index x + 5y
     LVM_KB(0, 0, 0);
@@ -107,37 +120,46 @@ __device__ __forceinline__ void keccak_round_32(uint32_t l[25], uint32_t h[25], 
     h[0] ^= KECCAK_RC_HI[round];
 }
 
-// The 24 rounds as a loop (throughput kernels: one copy of the round body
-// keeps the code small), or fully unrolled (latency-bound tree tops: no loop
-// overhead, round constants as literals).
-template <bool UNROLL = false>
-__device__ __forceinline__ void keccak_f1600_32(uint32_t l[25], uint32_t h[25]) {
-    if constexpr (UNROLL) {
+// The last round as far as a 32-byte digest needs it: row 0 of its B, lanes 0..3.
+__device__ __forceinline__ void keccak_last_round_digest(uint32_t l[25], uint32_t h[25]) {
+    uint32_t Cl[5], Ch[5], Rl[5], Rh[5];
+    theta_c(l, h, Cl, Ch, Rl, Rh);
+    uint32_t bl[5], bh[5];
+    LVM_KB(0, 0, 0);
+    LVM_KB(1, 6, 44);
+    LVM_KB(2, 12, 43);
+    LVM_KB(3, 18, 21);
+    LVM_KB(4, 24, 14);
 #pragma unroll
-        for (int round = 0; round < 24; round++) keccak_round_32(l, h, round);
-    } else {
-#pragma unroll 1
-        for (int round = 0; round < 24; round++) keccak_round_32(l, h, round);
+    for (int x = 0; x < 4; x++) {
+        l[x] = chi(bl[x], bl[(x + 1) % 5], bl[(x + 2) % 5]);
+        h[x] = chi(bh[x], bh[(x + 1) % 5], bh[(x + 2) % 5]);
     }
+    l[0] ^= KECCAK_RC_LO[23];
+    h[0] ^= KECCAK_RC_HI[23];
 }
 #undef LVM_KB
 
-// 64-bit-lane interface over the 32-bit-half permutation
-__device__ __forceinline__ void keccak_f1600(uint64_t s[25]) {
-    uint32_t l[25], h[25];
-#pragma unroll
-    for (int i = 0; i < 25; i++) {
-        l[i] = (uint32_t)s[i];
-        h[i] = (uint32_t)(s[i] >> 32);
-    }
-    keccak_f1600_32(l, h);
-#pragma unroll
-    for (int i = 0; i < 25; i++) s[i] = ((uint64_t)h[i] << 32) | l[i];
+// The 24 rounds as a loop (one copy of the round body keeps the code small).
+__device__ __forceinline__ void keccak_f1600_32(uint32_t l[25], uint32_t h[25]) {
+#pragma unroll 1
+    for (int round = 0; round < 24; round++) keccak_round_32(l, h, round);
+}
+
+// The permutation that ends a Keccak-256: only lanes 0..3 (the digest) come
+// out, the last round's other lanes are not formed. FIRST: the first round is
+// a copy of its own, for states whose zero lanes are known at compile time
+// (one-block messages). Together 3.5 % of a permutation.
+template <bool FIRST>
+__device__ __forceinline__ void keccak_f1600_32_digest(uint32_t l[25], uint32_t h[25]) {
+    if constexpr (FIRST) keccak_round_32(l, h, 0);
+#pragma unroll 1
+    for (int round = FIRST ? 1 : 0; round < 23; round++) keccak_round_32(l, h, round);
+    keccak_last_round_digest(l, h);
 }
 
 // Keccak-256 of exactly two 32-byte nodes (one permutation): lanes 0..7 hold
 // left || right, pad byte 0x01 at lane 8, 0x80 at the top of lane 16.
-template <bool UNROLL = false>
 __device__ __forceinline__ void keccak_pair_node(const uint64_t lft[4], const uint64_t rgt[4], uint64_t out[4]) {
     uint32_t l[25], h[25];
 #pragma unroll
@@ -151,7 +173,7 @@ __device__ __forceinline__ void keccak_pair_node(const uint64_t lft[4], const ui
     }
     l[8] = 0x01;
     h[16] = 0x80000000u;
-    keccak_f1600_32<UNROLL>(l, h);
+    keccak_f1600_32_digest<true>(l, h);
 #pragma unroll
     for (int i = 0; i < 4; i++) out[i] = ((uint64_t)h[i] << 32) | l[i];
 }

@@ -138,13 +138,12 @@ int ntt_coset_expand(const uint64_t *coef, uint32_t coef_pitch, uint64_t *lde, u
 // rows are already stored in bit-reversed order: leaf i hashes rows 2i, 2i+1,
 // into node L-1+i of the tree. Small tables' blocks go on to the levels above
 // their leaves; returns the nodes C of the topmost level written, which lie at
-// [C-1, 2C-1): what merkle_build_inner goes on from.
+// [C-1, 2C-1): what merkle_build_inner goes on from. canonical: every word is
+// known to be below p (the NTT's output).
 uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
-                                uint8_t *nodes, hipStream_t st);
+                                bool canonical, uint8_t *nodes, hipStream_t st);
 // the levels above the C nodes (a power of two) at [C-1, 2C-1) of a tree
 void merkle_build_inner(uint8_t *nodes, uint64_t C, hipStream_t st);
-// Keccak(BE24(e[2j]) || BE24(e[2j+1])) over an Fp3 array of `len` elements
-void keccak_fp3_pair_leaves(const uint64_t *evals, uint64_t len, uint8_t *leaves_out, hipStream_t st);
 
 size_t padded_leaves(size_t n);
 

@@ -16,10 +16,9 @@
 
 namespace lvm {
 
-// XOR the big-endian encoding of a canonicalised element into a lane held as
-// 32-bit halves: the little-endian lane of BE(v) is bswap64(v).
+// XOR the big-endian encoding of an element into a lane held as 32-bit
+// halves: the little-endian lane of BE(v) is bswap64(v), v canonical.
 __device__ __forceinline__ void absorb_be(uint32_t &l, uint32_t &h, uint64_t v) {
-    v = canon(v);
     l ^= __builtin_bswap32((uint32_t)(v >> 32));
     h ^= __builtin_bswap32((uint32_t)v);
 }
@@ -27,54 +26,43 @@ __device__ __forceinline__ void absorb_be(uint32_t &l, uint32_t &h, uint64_t v) 
 // One thread per leaf. Words [w0, w1) of rows 2i and 2i+1 (row stride
 // `pitch` words) are absorbed in order, 17 lanes per permutation. CONTIG:
 // the committed words are whole rows, so the leaf's data is one contiguous
-// run of 2*pitch words.
-template <bool CONTIG>
+// run of 2*pitch words. CANON: the words may lie in [p, 2^64) (rows handed in
+// by a caller; this library's own LDE rows are canonical).
+// VALU-bound (0.96 of the issue rate on wide tables): what counts is
+// instructions. The last block masks the words past the message instead of
+// branching per word, which had the compiler copy the 50-register state at
+// each of 17 joins (1300 cycles, 7 % of a permutation).
+template <bool CONTIG, bool CANON>
 __device__ __forceinline__ void row_pair_leaf(const uint64_t *__restrict__ rows, uint64_t pitch, uint64_t w0,
                                               uint64_t w1, uint64_t i, uint64_t *__restrict__ leaves) {
     const uint64_t width = w1 - w0;
     const uint64_t total = 2 * width;
-    const uint64_t *r0 = rows + (2 * i) * pitch + w0;
-    const uint64_t *r1 = rows + (2 * i + 1) * pitch + w0;
+    const uint64_t skip = pitch - width;  // row 2i's end to row 2i+1's start
+    const gmem_u64 *row = LVM_GLOBAL_CONST(rows) + (2 * i) * pitch + w0;
+    auto word = [&](uint64_t e) -> uint64_t {
+        const uint64_t v = row[CONTIG ? e : e + (e >= width ? skip : 0)];
+        return CANON ? canon(v) : v;
+    };
     uint32_t l[25], h[25];
 #pragma unroll
     for (int k = 0; k < 25; k++) l[k] = h[k] = 0;
-    const uint64_t *cur = r0;
-    uint64_t left_in_row = width;
-    bool second = false;
     uint64_t e = 0;
-    while (e + 17 <= total) {
+    for (; e + 17 <= total; e += 17) {
 #pragma unroll
-        for (int j = 0; j < 17; j++) {
-            absorb_be(l[j], h[j], *cur++);
-            if (!CONTIG) {
-                if (--left_in_row == 0 && !second) {
-                    second = true;
-                    cur = r1;
-                    left_in_row = width;
-                }
-            }
-        }
+        for (int j = 0; j < 17; j++) absorb_be(l[j], h[j], word(e + j));
         keccak_f1600_32(l, h);
-        e += 17;
     }
-    const uint64_t rem = total - e;
+    const uint32_t rem = (uint32_t)(total - e);  // 0..16 words, then the padding byte
 #pragma unroll
     for (int j = 0; j < 17; j++) {
-        if ((uint64_t)j < rem) {
-            absorb_be(l[j], h[j], *cur++);
-            if (!CONTIG) {
-                if (--left_in_row == 0 && !second) {
-                    second = true;
-                    cur = r1;
-                    left_in_row = width;
-                }
-            }
-        } else if ((uint64_t)j == rem) {
-            l[j] ^= 0x01;
-        }
+        const bool in = (uint32_t)j < rem;
+        const uint64_t v = word(in ? e + j : 0);
+        const uint32_t mask = in ? ~0u : 0u;
+        l[j] ^= (__builtin_bswap32((uint32_t)(v >> 32)) & mask) | ((uint32_t)j == rem ? 0x01u : 0u);
+        h[j] ^= __builtin_bswap32((uint32_t)v) & mask;
     }
     h[16] ^= 0x80000000u;
-    keccak_f1600_32(l, h);
+    keccak_f1600_32_digest<false>(l, h);
     uint64_t *o = leaves + 4 * i;
 #pragma unroll
     for (int k = 0; k < 4; k++) o[k] = ((uint64_t)h[k] << 32) | l[k];
@@ -132,14 +120,14 @@ __global__ __launch_bounds__(TREE_THREADS) void leaf_top_kernel(const uint64_t *
     row_pair_leaf_top(rows, pitch, w0, w1, L, span, blockIdx.x, nodes);
 }
 
-template <bool CONTIG>
+template <bool CONTIG, bool CANON>
 __global__ __launch_bounds__(256) void keccak_row_pair_leaves_kernel(const uint64_t *__restrict__ rows,
                                                                     uint64_t pitch, uint64_t w0, uint64_t w1,
                                                                     uint64_t num_leaves,
                                                                     uint64_t *__restrict__ leaves) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= num_leaves) return;
-    row_pair_leaf<CONTIG>(rows, pitch, w0, w1, i, leaves);
+    row_pair_leaf<CONTIG, CANON>(rows, pitch, w0, w1, i, leaves);
 }
 
 // Leaves of several tables in one launch: blocks [prefix[t], prefix[t+1])
@@ -157,28 +145,7 @@ __global__ __launch_bounds__(TREE_THREADS) void keccak_leaves_batched_kernel(con
     }
     const uint64_t i = (uint64_t)(b - prefix[t]) * TREE_THREADS + threadIdx.x;
     if (i >= j.num_leaves) return;
-    row_pair_leaf<true>(j.rows, j.pitch, 0, j.pitch, i, j.nodes + 4 * (j.num_leaves - 1));
-}
-
-// FRI layer leaves: Keccak(BE24(e[2j]) || BE24(e[2j+1])), 6 lanes, one permutation
-// (crypto/crypto/src/merkle_tree/backends/field_element_vector.rs:129-134).
-__global__ __launch_bounds__(256) void keccak_fp3_pair_leaves_kernel(const uint64_t *__restrict__ evals,
-                                                                    uint64_t num_leaves,
-                                                                    uint64_t *__restrict__ leaves) {
-    const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= num_leaves) return;
-    uint32_t l[25], h[25];
-#pragma unroll
-    for (int k = 0; k < 25; k++) l[k] = h[k] = 0;
-    const uint64_t *p = evals + 6 * j;
-#pragma unroll
-    for (int k = 0; k < 6; k++) absorb_be(l[k], h[k], p[k]);
-    l[6] = 0x01;
-    h[16] = 0x80000000u;
-    keccak_f1600_32(l, h);
-    uint64_t *o = leaves + 4 * j;
-#pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = ((uint64_t)h[k] << 32) | l[k];
+    row_pair_leaf<true, false>(j.rows, j.pitch, 0, j.pitch, i, j.nodes + 4 * (j.num_leaves - 1));
 }
 
 // parent p = Keccak(node[2p+1] || node[2p+2]), one lane per node
@@ -259,7 +226,7 @@ size_t padded_leaves(size_t n) {
 }
 
 uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
-                                uint8_t *nodes, hipStream_t st) {
+                                bool canonical, uint8_t *nodes, hipStream_t st) {
     if (L <= LEAF_TOP_LEAVES) {
         const uint32_t span = leaf_top_span(L);
         hipLaunchKernelGGL(leaf_top_kernel, dim3((unsigned)(L / span)), dim3(TREE_THREADS), 0, st, rows, pitch, w0, w1,
@@ -268,20 +235,17 @@ uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w
     }
     uint64_t *leaves = (uint64_t *)(nodes + (L - 1) * 32);
     dim3 grid((unsigned)((L + 255) / 256));
-    if (w0 == 0 && w1 == pitch)
-        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<true>, grid, dim3(256), 0, st, rows, pitch, w0, w1, L,
+    const bool contig = w0 == 0 && w1 == pitch;
+    if (contig && canonical)
+        hipLaunchKernelGGL((keccak_row_pair_leaves_kernel<true, false>), grid, dim3(256), 0, st, rows, pitch, w0, w1,
+                           L, leaves);
+    else if (contig)
+        hipLaunchKernelGGL((keccak_row_pair_leaves_kernel<true, true>), grid, dim3(256), 0, st, rows, pitch, w0, w1, L,
                            leaves);
     else
-        hipLaunchKernelGGL(keccak_row_pair_leaves_kernel<false>, grid, dim3(256), 0, st, rows, pitch, w0, w1, L,
-                           leaves);
+        hipLaunchKernelGGL((keccak_row_pair_leaves_kernel<false, true>), grid, dim3(256), 0, st, rows, pitch, w0, w1,
+                           L, leaves);
     return L;
-}
-
-void keccak_fp3_pair_leaves(const uint64_t *evals, uint64_t len, uint8_t *leaves_out, hipStream_t st) {
-    uint64_t nl = len / 2;
-    if (nl == 0) return;
-    dim3 grid((unsigned)((nl + 255) / 256));
-    hipLaunchKernelGGL(keccak_fp3_pair_leaves_kernel, grid, dim3(256), 0, st, evals, nl, (uint64_t *)leaves_out);
 }
 
 void merkle_build_inner(uint8_t *nodes_b, uint64_t C, hipStream_t st) {
