@@ -128,6 +128,15 @@ LVM_HD uint64_t root_of_unity(unsigned k) {
 // stay in this set, which needs one conditional correction per add or sub
 // instead of two.
 
+// r - k * EPS mod 2^64 for k = 0, 1, 2: one 64-bit add of the words (k, -k)
+LVM_HD uint64_t sub_eps(uint64_t r, uint32_t k) {
+    uint64_t kk = ((uint64_t)(0u - k) << 32) | k;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(kk));  // one pair: otherwise the words are added one by one
+#endif
+    return r + kk;
+}
+
 LVM_HD uint64_t ccanon(uint64_t r) { return r >= P ? r + EPS : r; }  // any r -> [0, p)
 
 // a, b < p. A carry means a + b - p = s + EPS (< p, no second wrap); no
@@ -139,24 +148,28 @@ LVM_HD uint64_t cadd(uint64_t a, uint64_t b) {
 }
 
 // a, b < p. A borrow means a - b + p = d - EPS with d = a - b + 2^64 > EPS.
+// The borrow is taken from the subtraction itself, word by word.
 LVM_HD uint64_t csub(uint64_t a, uint64_t b) {
-    const uint64_t d = a - b;
-    return a < b ? d - EPS : d;
+    uint32_t b0, b1;
+    const uint32_t lo = __builtin_subc((uint32_t)a, (uint32_t)b, 0u, &b0);
+    const uint32_t hi = __builtin_subc((uint32_t)(a >> 32), (uint32_t)(b >> 32), b0, &b1);
+    return sub_eps(((uint64_t)hi << 32) | lo, b1);
 }
 
 // canonical reduction of any 128-bit lo + 2^64 hi (2^64 = EPS, 2^96 = -1):
-// t0 = lo - hi_hi (mod p, in [0, 2^64)), t1 = hi_lo * EPS <= (2^32 - 1)^2,
-// t0 + t1 wraps at most once and its correction cannot wrap again.
+// with hi = hi_lo + 2^32 hi_hi the value is lo + EPS hi_lo - hi_hi. Since
+// EPS - hi_hi is the complement of hi_hi, u = EPS hi_lo + ~hi_hi (one
+// multiply-add, at most 2^64 - 2^32) is EPS too much: the value is s = lo + u
+// less EPS, plus 2^64 = EPS if lo + u wrapped. So a wrapped s is the answer (s <=
+// 2^64 - 2^32 - 2 < p), else s - EPS (< p), or s - EPS + p = s - 2 EPS mod 2^64
+// when that is negative: subtract k EPS with k = 0, 1, 2, two selects on one
+// word and its negative. A canonical product is 19 VALU instructions, 6 of them
+// cheap moves, where the borrow-and-correct form took 25: coset passes of 2^22 x
+// 64 4.46 -> 4.08 ms, 256-point passes 2.46 -> 2.36 ms (with csub below).
 LVM_HD uint64_t cred(uint64_t lo, uint64_t hi) {
-    const uint64_t hi_hi = hi >> 32, hi_lo = hi & EPS;
-    uint64_t t0, r;
-    // the borrow and carry as the operations' own flags (no 64-bit compare
-    // against a zero-extended word)
-    const bool borrow = __builtin_sub_overflow(lo, hi_hi, &t0);
-    t0 -= borrow ? EPS : 0;
-    const bool carry = __builtin_add_overflow(t0, (hi_lo << 32) - hi_lo, &r);
-    r += carry ? EPS : 0;
-    return ccanon(r);
+    const uint64_t u = (uint64_t)(uint32_t)hi * EPS + (uint32_t)~(uint32_t)(hi >> 32);
+    const uint64_t s = lo + u;
+    return sub_eps(s, s < lo ? 0u : s < EPS ? 2u : 1u);
 }
 
 // any a, b; canonical product
