@@ -22,6 +22,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "lvm_gpu.h"
@@ -44,7 +45,8 @@ struct lvm_batch {
     struct Launch {
         Kind kind;
         int r;
-        bool multi;
+        bool coset;
+        uint32_t rows;  // NTT: rows a window can span (the kernel's class)
         size_t args_off, prefix_off;
         uint32_t count, blocks;
         std::string name;  // profiler name of the launch
@@ -120,39 +122,44 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
     // NTT pass lists
     std::vector<std::vector<int>> R(T);
     std::vector<std::vector<PassArgs>> A(T);
-    std::vector<std::vector<uint32_t>> COS(T);
+    std::vector<std::vector<uint32_t>> NB(T);
     size_t max_steps = 0;
     for (size_t t = 0; t < T; t++) {
         const lvm_table_desc &d = b->in[t];
         int r[16];
         PassArgs a[16];
-        uint32_t cos[16];
+        uint32_t nb[16];
         const int k = lde_pass_list(d.trace, (uint32_t)d.m, log2u(d.n), log2u(d.blowup), d.weights, b->coef[t],
-                                    b->lde[t], tb, r, a, cos);
+                                    b->lde[t], tb, r, a, nb);
         if (k <= 0) return fail(LVM_ERR_ARG, "table too small for a coset LDE");
         R[t].assign(r, r + k);
         A[t].assign(a, a + k);
-        COS[t].assign(cos, cos + k);
+        NB[t].assign(nb, nb + k);
         max_steps = std::max(max_steps, (size_t)k);
     }
     for (size_t s = 0; s < max_steps; s++) {
-        // groups by (radix, multi) in order of first appearance
-        std::vector<std::pair<int, bool>> keys;
-        std::map<std::pair<int, bool>, std::vector<size_t>> groups;
+        // groups by (radix, coset pass, window class) in order of first appearance
+        using Key = std::tuple<int, bool, uint32_t>;
+        std::vector<Key> keys;
+        std::map<Key, std::vector<size_t>> groups;
         for (size_t t : b->order) {
             if (s >= R[t].size()) continue;
-            auto key = std::make_pair(R[t][s], COS[t][s] > 1);
+            const uint32_t rows = A[t][s].rows;
+            const Key key(R[t][s], A[t][s].weights != nullptr, rows <= 2 ? 2 : rows <= 4 ? 4 : rows);
             if (!groups.count(key)) keys.push_back(key);
             groups[key].push_back(t);
         }
         for (auto &key : keys) {
             const auto &ts = groups[key];
+            const int r = std::get<0>(key);
+            const bool coset = std::get<1>(key);
+            const uint32_t rows = std::get<2>(key);
             std::vector<PassArgs> args;
             std::vector<uint32_t> prefix(1, 0);
             uint64_t total = 0;
             for (size_t t : ts) {
                 args.push_back(A[t][s]);
-                total += pass_blocks(key.first, A[t][s]);
+                total += NB[t][s];
                 if (total >= (1ull << 31)) return fail(LVM_ERR_ARG, "batched launch exceeds 2^31 blocks");
                 prefix.push_back((uint32_t)total);
             }
@@ -162,14 +169,13 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
                 double bytes = 0;
                 for (size_t t : ts) {
                     const PassArgs &a = A[t][s];
-                    const double rows = (double)(a.total_groups << key.first);  // logical rows of the pass
-                    const double out_rows = a.cosets_per_block > 1 ? rows * a.cosets_per_block : rows;
-                    bytes += 8.0 * a.m * (rows + out_rows);
+                    const double in_rows = (double)(a.total_groups << r);  // logical rows of the pass
+                    bytes += 8.0 * a.m * in_rows * (coset ? 1.0 + b->in[t].blowup : 2.0);
                 }
-                std::string name = "batch_ntt_s" + std::to_string(s) + "_r" + std::to_string(key.first) +
-                                   (key.second ? "_coset" : "");
-                b->launches.push_back({lvm_batch::NTT, key.first, key.second, ao, po, (uint32_t)ts.size(),
-                                       (uint32_t)total, name, bytes});
+                std::string name = "batch_ntt_s" + std::to_string(s) + "_r" + std::to_string(r) +
+                                   (coset ? "_coset" : "") + (rows > 2 ? "_w" + std::to_string(rows) : "");
+                b->launches.push_back({lvm_batch::NTT, r, coset, rows, ao, po, (uint32_t)ts.size(), (uint32_t)total,
+                                       name, bytes});
             }
         }
     }
@@ -193,7 +199,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
             double bytes = 0;
             for (const LeafJob &j : jobs) bytes += 16.0 * j.pitch * j.num_leaves + 32.0 * j.num_leaves;
             b->launches.push_back(
-                {lvm_batch::LEAVES, 0, false, jo, po, (uint32_t)T, (uint32_t)total, "batch_leaves", bytes});
+                {lvm_batch::LEAVES, 0, false, 0, jo, po, (uint32_t)T, (uint32_t)total, "batch_leaves", bytes});
         }
     }
     // tree steps
@@ -225,7 +231,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
             const size_t so = w.put(steps.data(), steps.size());
             const size_t po = w.put(prefix.data(), prefix.size());
             if (record)
-                b->launches.push_back({lvm_batch::TREE, 0, false, so, po, (uint32_t)steps.size(), (uint32_t)total,
+                b->launches.push_back({lvm_batch::TREE, 0, false, 0, so, po, (uint32_t)steps.size(), (uint32_t)total,
                                        "batch_merkle_s" + std::to_string(s), bytes});
         }
     }
@@ -238,7 +244,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         if (record) {
             b->trees_off = to;
             b->roots_off = ro;
-            b->launches.push_back({lvm_batch::ROOTS, 0, false, to, ro, (uint32_t)T, 0, "batch_roots", 64.0 * T});
+            b->launches.push_back({lvm_batch::ROOTS, 0, false, 0, to, ro, (uint32_t)T, 0, "batch_roots", 64.0 * T});
         }
     }
     return LVM_OK;
@@ -250,8 +256,8 @@ void enqueue(lvm_batch *b, hipStream_t st, bool profile) {
         switch (l.kind) {
         case lvm_batch::NTT: {
             ProfScope ps(profile ? l.name.c_str() : nullptr, st);
-            launch_pass_batched(l.r, (const PassArgs *)(base + l.args_off), (const uint32_t *)(base + l.prefix_off),
-                                l.count, l.blocks, l.multi, st);
+            launch_pass_batched(l.r, l.coset, l.rows, (const PassArgs *)(base + l.args_off),
+                                (const uint32_t *)(base + l.prefix_off), l.count, l.blocks, st);
             break;
         }
         case lvm_batch::LEAVES: {

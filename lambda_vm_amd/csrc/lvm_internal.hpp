@@ -120,10 +120,19 @@ struct PassArgs {
     const uint64_t *shift_lo;      // forward tables for the coset shift
     const uint64_t *shift_hi;
     const uint64_t *tw_r;          // w_256^(+-e), e < 256
-    uint32_t cosets_per_block;     // cosets produced per block (grid.z = cosets / this)
+    uint32_t cosets_per_block;     // cosets produced per block
     uint32_t inverse;              // 1: inverse transform (tw_* hold inverse powers)
     uint32_t in_canonical;         // 1: input values are below p (an earlier pass wrote them)
+    // tiling (pass_tiling): runs of `run` words in `wins` windows of 16
+    uint32_t by_rows;              // 1: a run is the S*m words of a block's rows, 0: one row's m words
+    uint32_t run, wins, tiles;
+    uint32_t win_inv, m_inv;       // udiv multipliers of wins and m
+    uint32_t blocks;               // blocks that cover the tiles once
+    uint32_t rows;                 // rows a window can span
 };
+// A coset pass of fewer blocks than this has its cosets shared out over copies
+// of them (each reads the tile again).
+constexpr uint32_t COSET_SPLIT_BLOCKS = 512;
 
 void ntt_inverse_rows(const uint64_t *in, uint32_t in_pitch, uint64_t *out, uint32_t out_pitch, uint32_t m,
                       unsigned log_n, const Tables &tb, hipStream_t st);
@@ -184,13 +193,12 @@ __device__ __forceinline__ uint32_t find_slot(const uint32_t *__restrict__ prefi
 }
 int plan_passes(unsigned log_n, int *r);              // radices of a size-2^log_n transform
 bool set_ntt_plan(unsigned log_n, const int *r, int np);  // np = 0 restores the default
-uint32_t pass_blocks(int r, const PassArgs &a);       // blocks of one table's pass
-void launch_pass_batched(int r, const PassArgs *d_args, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
-                         bool multi, hipStream_t st);
+void launch_pass_batched(int r, bool coset, uint32_t rows, const PassArgs *d_args, const uint32_t *d_prefix,
+                         uint32_t count, uint32_t blocks, hipStream_t st);
 // One table's coset-LDE pass sequence (inverse passes into `coef`, then the
 // coset expansion into `lde`); returns the number of passes.
 int lde_pass_list(const uint64_t *trace, uint32_t m, unsigned log_n, unsigned log_blowup, const uint64_t *weights,
-                  uint64_t *coef, uint64_t *lde, const Tables &tb, int *r_out, PassArgs *a_out, uint32_t *cos_out);
+                  uint64_t *coef, uint64_t *lde, const Tables &tb, int *r_out, PassArgs *a_out, uint32_t *blocks_out);
 
 struct LeafJob {
     const uint64_t *rows;  // bit-reversed row-major LDE, `pitch` words per row
