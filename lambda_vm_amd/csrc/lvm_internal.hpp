@@ -129,6 +129,7 @@ struct PassArgs {
     uint32_t win_inv, m_inv;       // udiv multipliers of wins and m
     uint32_t blocks;               // blocks that cover the tiles once
     uint32_t rows;                 // rows a window can span
+    uint32_t units;                // runs packed into a tile (last pass of a narrow table), else 1
 };
 // A coset pass of fewer blocks than this has its cosets shared out over copies
 // of them (each reads the tile again).

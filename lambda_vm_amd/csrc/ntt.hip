@@ -66,11 +66,13 @@ static uint32_t udiv_inv(uint32_t d) { return d == 1 ? ~0u : (uint32_t)((1ull <<
 uint32_t pass_tiling(int r, uint32_t cosets, PassArgs &a) {
     const uint64_t S = 1ull << a.log_s, words = S * a.m;
     a.by_rows = words < (1ull << 31) ? 1u : 0u;
-    a.run = a.by_rows ? (uint32_t)words : a.m;
+    a.units = a.log_s == 0 && a.m <= PASS_C / 2 ? PASS_C / a.m : 1;
+    a.run = a.by_rows ? (uint32_t)words * a.units : a.m;
     a.wins = (uint32_t)(((uint64_t)a.run + PASS_C - 1) / PASS_C);
     a.win_inv = udiv_inv(a.wins);
     a.m_inv = udiv_inv(a.m);
-    a.tiles = (uint32_t)((a.by_rows ? a.total_groups >> a.log_s : a.total_groups) * a.wins);
+    const uint64_t runs = a.by_rows ? ((a.total_groups >> a.log_s) + a.units - 1) / a.units : a.total_groups;
+    a.tiles = (uint32_t)(runs * a.wins);
     const uint32_t per = pass_tiles_per_block(r);
     a.blocks = (a.tiles + per - 1) / per;
     // rows a window spans: its first word lies at most m - gcd(16, m) into a row

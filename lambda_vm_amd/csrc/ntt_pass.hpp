@@ -89,7 +89,8 @@ __device__ __forceinline__ uint32_t udiv(uint32_t n, uint32_t d, uint32_t inv) {
 // Tiles: run-major windows of PASS_C words. by_rows: a run is the S rows of one
 // block (run = S*m), lane c of window w takes word w*16 + c, i.e. row jlo = word
 // / m and column word % m; else (tables whose runs exceed 32 bits) a run is one
-// row's m words. NJ: rows a window can span, each with factors of its own in LDS
+// row's m words. In the last pass (S = 1) of a table of at most 8 columns a tile
+// packs `units` = 16 / m whole runs side by side. NJ: rows a window can span, each with factors of its own in LDS
 // (1 for m a multiple of 16, 2 for most m, 4 for m >= 4); 0: more than 4 (m <
 // 4), every lane forms its factors itself.
 // COSET: the first pass of a coset expansion (bit-reversed input rows,
@@ -126,11 +127,18 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs &a, uint32_t block)
     // unit: the tile's run; jb: its window's first row, jl: the lane's row past it
     const uint32_t unit = t_ok ? udiv(tile, a.wins, a.win_inv) : 0;
     const uint32_t w0 = t_ok ? (tile - unit * a.wins) * C : 0;
-    const bool c_ok = t_ok && w0 + c < a.run;
+    bool c_ok = t_ok && w0 + c < a.run;
     const uint32_t word = c_ok ? w0 + c : w0;  // a lane past the run reads its window's first word
     uint64_t blk;
     uint32_t jb, jlo, col, nj = 1;
-    if (a.by_rows) {
+    if (NJ && a.units > 1) {
+        const uint32_t u = udiv(word, a.m, a.m_inv);
+        blk = (uint64_t)unit * a.units + u;
+        c_ok = c_ok && blk < a.total_groups;
+        if (!c_ok) blk = 0;
+        jb = jlo = 0;
+        col = word - u * a.m;
+    } else if (a.by_rows) {
         blk = unit;
         jb = udiv(w0, a.m, a.m_inv);
         jlo = udiv(word, a.m, a.m_inv);
