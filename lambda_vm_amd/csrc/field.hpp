@@ -288,6 +288,26 @@ LVM_HD uint64_t dot3(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_
     return r;
 }
 
+// the same as a canonical value (any operands)
+LVM_HD uint64_t cdot3(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64_t a2, uint64_t b2) {
+    uint64_t l0, h0, l1, h1, l2, h2;
+    mul_wide(a0, b0, l0, h0);
+    mul_wide(a1, b1, l1, h1);
+    mul_wide(a2, b2, l2, h2);
+    const uint64_t lo = l0 + l1, lo2 = lo + l2;
+    const uint32_t c = (lo < l0) + (lo2 < lo);
+    const uint64_t hi = h0 + h1, hi2 = hi + h2, hi3 = hi2 + c;
+    const uint32_t over = (hi < h0) + (hi2 < hi) + (hi3 < hi2);
+    // over * 2^128 = -over * 2^32, over <= 2
+    return csub(cred(lo2, hi3), (uint64_t)over << 32);
+}
+
+LVM_HD fp3 cf3_mul(fp3 a, fp3 b) {
+    const uint64_t b1_2 = cadd(b.c1, b.c1), b2_2 = cadd(b.c2, b.c2);  // b canonical
+    return fp3{cdot3(a.c0, b.c0, a.c1, b2_2, a.c2, b1_2), cdot3(a.c0, b.c1, a.c1, b.c0, a.c2, b2_2),
+               cdot3(a.c0, b.c2, a.c1, b.c1, a.c2, b.c0)};
+}
+
 LVM_HD fp3 f3_mul(fp3 a, fp3 b) {
     uint64_t b1_2 = dbl(b.c1), b2_2 = dbl(b.c2);
     return fp3{dot3(a.c0, b.c0, a.c1, b2_2, a.c2, b1_2), dot3(a.c0, b.c1, a.c1, b.c0, a.c2, b2_2),
@@ -316,6 +336,11 @@ LVM_HD fp3 f3_pow(fp3 a, uint64_t e) {
     }
     return r;
 }
+
+// Canonical Fp3 operations: canonical operands, canonical results.
+LVM_HD fp3 cf3_add(fp3 a, fp3 b) { return fp3{cadd(a.c0, b.c0), cadd(a.c1, b.c1), cadd(a.c2, b.c2)}; }
+LVM_HD fp3 cf3_sub(fp3 a, fp3 b) { return fp3{csub(a.c0, b.c0), csub(a.c1, b.c1), csub(a.c2, b.c2)}; }
+LVM_HD fp3 cf3_mul_base(fp3 a, uint64_t b) { return fp3{cmul(b, a.c0), cmul(b, a.c1), cmul(b, a.c2)}; }
 
 // Delayed-reduction accumulator for dot products (the idea of the
 // reference's dot_product_3, goldilocks.rs:289-315, stretched over a whole
@@ -387,16 +412,19 @@ __device__ __forceinline__ void acc_mad_uniform(acc128 &a, uint64_t x, uint64_t 
 #endif
 }
 
-// value = s0 + c0*2^64 + s1*2^32 + c1*2^96 + s2*2^64 + c2*2^128 (mod p), with
-// 2^64 = EPS, 2^96 = -1, 2^128 = EPS^2
+// canonical value of s0 + c0*2^64 + s1*2^32 + c1*2^96 + s2*2^64 + c2*2^128 (fewer
+// than 2^31 products), with 2^64 = EPS, 2^96 = -1, 2^128 = -2^32: the words of
+// weight 2^64 are summed first and reduced as in cred, the counts of the higher
+// powers are subtracted as one word.
 LVM_HD uint64_t acc_reduce(const acc128 &a) {
-    uint64_t r = a.s0;
-    r = add(r, mul((uint64_t)a.c0, EPS));
-    r = add(r, reduce128(a.s1 << 32, a.s1 >> 32));
-    r = sub(r, (uint64_t)a.c1);
-    r = add(r, reduce128(0, a.s2));
-    r = add(r, mul((uint64_t)a.c2, EPS * EPS));
-    return r;
+    const uint64_t x = (a.s1 >> 32) + a.c0;
+    const uint64_t t = a.s2 + x;                       // weight 2^64
+    const uint32_t c2 = a.c2 + (t < x ? 1u : 0u);      // weight 2^128
+    const uint64_t l = a.s0 + (a.s1 << 32);
+    const uint64_t u = (uint64_t)(uint32_t)t * EPS + (uint32_t)~(uint32_t)(t >> 32);  // EPS too much
+    const uint64_t s = l + u;
+    const uint32_t k = (l < a.s0 ? 1u : 0u) + (s < u ? 1u : 0u);  // wraps of 2^64
+    return csub(cadd(ccanon(s), ((uint64_t)k << 32) - k), ((uint64_t)c2 << 32) + a.c1 + EPS);
 }
 
 LVM_HD uint64_t bswap64(uint64_t v) {

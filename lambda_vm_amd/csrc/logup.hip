@@ -13,13 +13,12 @@
 // Aux layout: row-major, C = committed + 1 Fp3 columns per row (committed
 // term columns, then the accumulated column).
 //
-// Kernel plan: each thread owns G consecutive rows. For every interaction it
-// builds the running products of its G fingerprints, inverts the last one
-// (one Fp3 inversion per G elements, Montgomery's trick within the thread),
-// and walks back recomputing each fingerprint instead of keeping it, so only
-// the running products and the term accumulators live in registers. Row sums
-// go to LDS, the block scans them, and a single-block pass scans the block
-// totals; a last pass writes the accumulated column.
+// Kernel plan: each thread owns G consecutive rows. For every output column it
+// puts the column's interactions over one denominator per row, inverts the
+// product of its G denominators (one Fp3 inversion per G rows, Montgomery's
+// trick within the thread) and walks back. Row sums go to LDS, the block scans
+// them, and a single-block pass scans the block totals; a last pass writes the
+// accumulated column.
 #include <algorithm>
 #include <cstring>
 #include <string>
@@ -57,77 +56,99 @@ struct MainView {
     __device__ __forceinline__ uint64_t at(uint64_t row, uint32_t col) const { return p[row * rs + col * cs]; }
 };
 
+// sum of coef_t * main[row][col_t] over terms [t0, t1) from `v` on, canonical;
+// most coefficients are one (a plain column)
+__device__ __forceinline__ uint64_t linear(const uint64_t *coef, const uint32_t *col, uint32_t t0, uint32_t t1,
+                                           uint64_t v, const MainView &mv, uint64_t row) {
+    for (uint32_t t = t0; t < t1; t++) {
+        const uint64_t c = coef[t], x = mv.at(row, col[t]);
+        v = cadd(v, c == 1 ? ccanon(x) : cmul(c, x));
+    }
+    return v;
+}
+
+// The alpha powers weigh base-field values and are the same for every row:
+// delayed-reduction dot products with scalar operands, one reduction each.
 __device__ __forceinline__ fp3 fingerprint(const LogupDev &d, uint32_t k, const MainView &mv, uint64_t row) {
-    fp3 lc = fp3{d.bus_ids[k], 0, 0};
+    acc128 s[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) acc_zero(s[j]);
     const uint32_t e1 = d.elem_offsets[k + 1];
     for (uint32_t e = d.elem_offsets[k]; e < e1; e++) {
-        uint64_t base = d.elem_const[e];
-        const uint32_t t1 = d.term_offsets[e + 1];
-        for (uint32_t t = d.term_offsets[e]; t < t1; t++) base = add(base, mul(d.term_coef[t], mv.at(row, d.term_col[t])));
+        const uint64_t base = linear(d.term_coef, d.term_col, d.term_offsets[e], d.term_offsets[e + 1],
+                                     ccanon(d.elem_const[e]), mv, row);
         const uint64_t *a = d.alpha + 3 * (uint64_t)d.elem_alpha_idx[e];
-        lc = f3_add(lc, f3_mul_base(fp3{a[0], a[1], a[2]}, base));
+#pragma unroll
+        for (int j = 0; j < 3; j++) acc_mad_uniform(s[j], a[j], base);
     }
-    return f3_sub(fp3{d.z0, d.z1, d.z2}, lc);
+    const uint64_t z0 = csub(ccanon(d.z0), ccanon(d.bus_ids[k]));
+    return fp3{csub(z0, acc_reduce(s[0])), csub(ccanon(d.z1), acc_reduce(s[1])), csub(ccanon(d.z2), acc_reduce(s[2]))};
 }
 
 __device__ __forceinline__ uint64_t multiplicity(const LogupDev &d, uint32_t k, const MainView &mv, uint64_t row) {
-    uint64_t m = d.mult_const[k];
-    const uint32_t t1 = d.mult_term_offsets[k + 1];
-    for (uint32_t t = d.mult_term_offsets[k]; t < t1; t++) m = add(m, mul(d.mult_term_coef[t], mv.at(row, d.mult_term_col[t])));
-    return m;
+    return linear(d.mult_term_coef, d.mult_term_col, d.mult_term_offsets[k], d.mult_term_offsets[k + 1],
+                  ccanon(d.mult_const[k]), mv, row);
 }
 
 // The terms of output columns [c0, c1) at the thread's rows r0 .. r0+cnt-1
-// (one batch inversion per interaction over those rows): committed columns
-// into aux, every column into terms_out, their sum added to rowsum.
+// (one batch inversion per column over those rows): committed columns into
+// aux, every column into terms_out, their sum added to rowsum. A column's
+// interactions are put over one denominator, m_a / f_a + m_b / f_b = (m_a f_b +
+// m_b f_a) / (f_a f_b), so that a pair costs one inversion's share and one set
+// of prefix products instead of two; numerators and denominators of the rows
+// stay in registers. VALU-bound: 2^18 rows of eight interactions 126 -> 93 us,
+// seven VM tables of 2^20 rows 677 -> 438 us each (in a whole proof) against an
+// inversion per interaction, fingerprints recomputed on the way back and every
+// element weighted by a full product.
 __device__ __forceinline__ void logup_terms(const LogupDev &d, const MainView &mv, uint64_t n, uint64_t r0, int cnt,
                                             uint32_t c0, uint32_t c1, uint64_t *__restrict__ aux,
                                             uint64_t *__restrict__ terms_out, fp3 rowsum[LOGUP_G]) {
+    if (cnt == 0) return;
     const uint32_t C = d.num_out_cols;
     for (uint32_t c = c0; c < c1; c++) {
-        fp3 term[LOGUP_G];
-#pragma unroll
-        for (int j = 0; j < LOGUP_G; j++) term[j] = fp3{0, 0, 0};
-        const uint32_t k1 = d.out_col_offsets[c + 1];
-        for (uint32_t ki = d.out_col_offsets[c]; ki < k1; ki++) {
-            const uint32_t k = d.out_col_interactions[ki];
-            fp3 pre[LOGUP_G];
-            fp3 run = fp3{1, 0, 0};
-#pragma unroll
-            for (int j = 0; j < LOGUP_G; j++) {
-                if (j < cnt) run = j == 0 ? fingerprint(d, k, mv, r0) : f3_mul(run, fingerprint(d, k, mv, r0 + j));
-                pre[j] = run;
-            }
-            if (cnt == 0) continue;
-            fp3 inv = f3_inv(run);  // (prod of the thread's fingerprints)^-1
-#pragma unroll
-            for (int j = LOGUP_G - 1; j >= 1; j--) {
-                if (j < cnt) {
-                    const fp3 f = fingerprint(d, k, mv, r0 + j);
-                    const fp3 r = f3_mul(inv, pre[j - 1]);
-                    inv = f3_mul(inv, f);
-                    term[j] = f3_add(term[j], f3_mul_base(r, multiplicity(d, k, mv, r0 + j)));
-                }
-            }
-            term[0] = f3_add(term[0], f3_mul_base(inv, multiplicity(d, k, mv, r0)));
-        }
+        const uint32_t k0 = d.out_col_offsets[c], k1 = d.out_col_offsets[c + 1];
+        fp3 num[LOGUP_G], den[LOGUP_G], pre[LOGUP_G];
 #pragma unroll
         for (int j = 0; j < LOGUP_G; j++) {
+            num[j] = fp3{0, 0, 0};
+            den[j] = fp3{1, 0, 0};
+            if (j < cnt) {
+                for (uint32_t ki = k0; ki < k1; ki++) {
+                    const uint32_t k = d.out_col_interactions[ki];
+                    const fp3 f = fingerprint(d, k, mv, r0 + j);
+                    const uint64_t m = multiplicity(d, k, mv, r0 + j);
+                    if (ki == k0) {
+                        num[j] = fp3{m, 0, 0};
+                        den[j] = f;
+                    } else {
+                        num[j] = cf3_add(cf3_mul(num[j], f), cf3_mul_base(den[j], m));
+                        den[j] = cf3_mul(den[j], f);
+                    }
+                }
+            }
+            pre[j] = j ? cf3_mul(pre[j - 1], den[j]) : den[j];
+        }
+        fp3 inv = f3_canon(f3_inv(pre[LOGUP_G - 1]));  // (prod of the thread's denominators)^-1
+#pragma unroll
+        for (int j = LOGUP_G - 1; j >= 0; j--) {
+            const fp3 r = j ? cf3_mul(inv, pre[j - 1]) : inv;
+            if (j) inv = cf3_mul(inv, den[j]);
+            const fp3 term = cf3_mul(num[j], r);
             if (j < cnt) {
                 const uint64_t row = r0 + j;
                 if (c + 1 < C) {
                     uint64_t *o = aux + 3 * (row * C + c);
-                    o[0] = term[j].c0;
-                    o[1] = term[j].c1;
-                    o[2] = term[j].c2;
+                    o[0] = term.c0;
+                    o[1] = term.c1;
+                    o[2] = term.c2;
                 }
                 if (terms_out) {
                     uint64_t *o = terms_out + 3 * ((uint64_t)c * n + row);
-                    o[0] = term[j].c0;
-                    o[1] = term[j].c1;
-                    o[2] = term[j].c2;
+                    o[0] = term.c0;
+                    o[1] = term.c1;
+                    o[2] = term.c2;
                 }
-                rowsum[j] = f3_add(rowsum[j], term[j]);
+                rowsum[j] = cf3_add(rowsum[j], term);
             }
         }
     }
