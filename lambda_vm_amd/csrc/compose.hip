@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void transpose_kernel(const uint64_t *__restri
     for (int i = threadIdx.x; i < T * T * E; i += 256) {
         const int rr = i / (T * E), ww = i % (T * E);
         const uint64_t r = r0 + rr, w = (uint64_t)c0 * E + ww;
-        if (r < N && w < wpr) tile[rr][ww] = in[(uint64_t)bitrev((uint32_t)r, logN) * wpr + w];
+        if (r < N && w < wpr) tile[rr][ww] = ccanon(in[(uint64_t)bitrev((uint32_t)r, logN) * wpr + w]);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < T * T * E; i += 256) {
@@ -420,7 +420,7 @@ __device__ __forceinline__ void transpose_bitrev_tile_body(const uint64_t *__res
     for (int q = 0; q < WC; q++) {
         const uint32_t i = threadIdx.x + 256 * q;
         const uint32_t ww = i % WC, j = (i / WC) % 8, l = i / (WC * 8);
-        tile[(__brev(j) >> 29) * 32 + l][ww] = v[q];
+        tile[(__brev(j) >> 29) * 32 + l][ww] = ccanon(v[q]);  // a handle may hold a caller's rows
     }
     __syncthreads();
 #pragma unroll
@@ -565,6 +565,13 @@ size_t put(std::vector<uint8_t> &blob, const T *v, size_t n) {
     return at;
 }
 
+// field elements, stored canonical (the compiled kernels' arithmetic expects it)
+size_t put_canon(std::vector<uint8_t> &blob, const uint64_t *v, size_t n) {
+    std::vector<uint64_t> c(n);
+    for (size_t i = 0; i < n; i++) c[i] = canon(v[i]);
+    return put(blob, c.data(), n);
+}
+
 bool is_pow2(size_t x) { return x && !(x & (x - 1)); }
 unsigned log2u(size_t x) { return (unsigned)__builtin_ctzll(x); }
 
@@ -585,7 +592,7 @@ struct ComposeJob {
     std::vector<uint32_t> root_node;
     const uint32_t *root_group = nullptr;
     size_t o_nodes = 0, o_bc = 0, o_ec = 0, o_rap = 0, o_al = 0, o_to = 0, o_roots = 0, o_eoff = 0, o_eidx = 0;
-    size_t o_beta = 0, o_rg = 0, o_z = 0, o_bcol = 0, o_baux = 0, o_bval = 0, o_bbeta = 0, o_bpcol = 0, o_bpflag = 0,
+    size_t o_beta = 0, o_betaw = 0, o_rg = 0, o_z = 0, o_bcol = 0, o_baux = 0, o_bval = 0, o_bbeta = 0, o_bpcol = 0, o_bpflag = 0,
            o_bpbeta = 0;
 };
 
@@ -692,9 +699,9 @@ int compose_prepare(const lvm_program *pg, const lvm_lde *main, const lvm_lde *a
     j.o_nodes = put(blob, pg->nodes, 2 * pg->num_nodes);
     j.o_bc = put(blob, pg->base_consts, pg->num_base_consts);
     j.o_ec = put(blob, pg->ext_consts, 3 * pg->num_ext_consts);
-    j.o_rap = put(blob, pg->rap_challenges, 3 * pg->num_rap);
-    j.o_al = put(blob, pg->alpha_powers, 3 * pg->num_alpha);
-    j.o_to = put(blob, pg->table_offset, pg->table_offset ? 3 : 0);
+    j.o_rap = put_canon(blob, pg->rap_challenges, 3 * pg->num_rap);
+    j.o_al = put_canon(blob, pg->alpha_powers, 3 * pg->num_alpha);
+    j.o_to = put_canon(blob, pg->table_offset, pg->table_offset ? 3 : 0);
     j.o_roots = put(blob, roots32.data(), roots32.size());
     j.o_eoff = put(blob, emit_off.data(), emit_off.size());
     j.o_eidx = put(blob, emit_idx.data(), emit_idx.size());
@@ -767,7 +774,19 @@ int compose_prepare(const lvm_program *pg, const lvm_lde *main, const lvm_lde *a
             a.step_const[3 * k + 1] = c.c1;
             a.step_const[3 * k + 2] = c.c2;
         }
-        j.o_beta = put(blob, cp->beta, 3 * pg->num_roots);
+        j.o_beta = put_canon(blob, cp->beta, 3 * pg->num_roots);
+        // an extension-valued constraint's words weigh beta, w beta, w^2 beta (w^3 = 2)
+        std::vector<uint64_t> bw(9 * pg->num_roots);
+        for (size_t c = 0; c < pg->num_roots; c++) {
+            fp3 b{canon(cp->beta[3 * c]), canon(cp->beta[3 * c + 1]), canon(cp->beta[3 * c + 2])};
+            for (int i = 0; i < 3; i++) {
+                bw[9 * c + 3 * i] = b.c0;
+                bw[9 * c + 3 * i + 1] = b.c1;
+                bw[9 * c + 3 * i + 2] = b.c2;
+                b = fp3{cadd(b.c2, b.c2), b.c0, b.c1};
+            }
+        }
+        j.o_betaw = put(blob, bw.data(), bw.size());
         j.o_rg = put(blob, cp->root_group, pg->num_roots);
         j.o_z = put(blob, zc.data(), B);
         j.o_bcol = put(blob, bcol.data(), bcol.size());
@@ -845,6 +864,7 @@ void compose_bind(ComposeJob &j, const uint8_t *db, const uint64_t *cm_main, con
     a.tw_hi = tb.fwd_hi;
     if (j.mode == 0) {
         a.beta = (const uint64_t *)(db + j.o_beta);
+        a.beta_w = (const uint64_t *)(db + j.o_betaw);
         a.root_group = (const uint32_t *)(db + j.o_rg);
         a.zcyc = (const uint64_t *)(db + j.o_z);
         a.b_col = (const uint32_t *)(db + j.o_bcol);

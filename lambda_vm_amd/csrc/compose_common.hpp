@@ -32,6 +32,7 @@ struct CompArgs {
     uint64_t next_step;
     // composition (mode 0) or per-constraint evals (mode 1)
     const uint64_t *beta;        // num_roots Fp3
+    const uint64_t *beta_w;      // num_roots x (beta, w beta, w^2 beta)
     const uint32_t *root_group;  // num_roots
     uint32_t num_groups;
     uint32_t group_ex[COMP_MAX_GROUPS];
@@ -62,10 +63,27 @@ struct CompArgs {
     uint64_t total_threads;
 };
 
+// Words that no kernel writes, in the constant address space: a uniform address
+// becomes a scalar load (the output pointer may alias a plain one). Table words
+// go through the global address space: as flat loads, which the compiler emits
+// for pointers read from memory, they count against the scalar loads' counter
+// and every wait for a challenge waits for the rows in flight.
+typedef const __attribute__((address_space(4))) uint64_t cmem_u64;
+#define LVM_CONST(p) ((lvm::cmem_u64 *)(p))
+
+typedef const __attribute__((address_space(4))) uint32_t cmem_u32;
+#define LVM_CONST32(p) ((lvm::cmem_u32 *)(p))
+
 __device__ __forceinline__ fp3 ld3(const uint64_t *p) { return fp3{p[0], p[1], p[2]}; }
+// the same from a table's copy, and from the argument block
+__device__ __forceinline__ fp3 ld3_row(const uint64_t *p) {
+    const gmem_u64 *g = LVM_GLOBAL_CONST(p);
+    return fp3{g[0], g[1], g[2]};
+}
+__device__ __forceinline__ fp3 ld3_arg(const uint64_t *p) { return fp3{LVM_CONST(p)[0], LVM_CONST(p)[1], LVM_CONST(p)[2]}; }
 // w_{2^32}^e from the two-level twiddle tables
 __device__ __forceinline__ uint64_t tw32_table(const uint64_t *lo, const uint64_t *hi, uint32_t e) {
-    return mul(lo[e & 0xFFFFu], hi[e >> 16]);
+    return mul(LVM_GLOBAL_CONST(lo)[e & 0xFFFFu], LVM_GLOBAL_CONST(hi)[e >> 16]);
 }
 __device__ __forceinline__ fp3 embed(uint64_t b) { return fp3{b, 0, 0}; }
 
@@ -84,7 +102,7 @@ __device__ __forceinline__ uint64_t frame_row(const CompArgs &a, uint32_t r, uin
 __device__ __forceinline__ fp3 composition_groups(const CompArgs &a, uint32_t r, const fp3 *gs) {
     // x = offset * w_N^r
     const uint64_t x = mul(a.offset, tw32_table(a.tw_lo, a.tw_hi, r << (32 - a.log_N)));
-    const uint64_t zc = a.zcyc[r & ((1u << a.log_B) - 1)];
+    const uint64_t zc = LVM_GLOBAL_CONST(a.zcyc)[r & ((1u << a.log_B) - 1)];
     fp3 h = fp3{0, 0, 0};
     for (uint32_t g = 0; g < a.num_groups; g++) {
         uint64_t z = zc;
@@ -114,18 +132,18 @@ __device__ __forceinline__ fp3 composition_tail(const CompArgs &a, uint32_t r, c
         // unrolled so that several columns' loads are in flight together
 #pragma unroll 8
         for (uint32_t e = a.bp_off[k]; e < a.bp_off[k + 1]; e++) {
-            const uint32_t fl = a.bp_flags[e];
-            const uint64_t v = a.main[((uint64_t)a.bp_col[e] << a.log_N) + r];
-            const uint64_t *bb = a.bp_beta + 6 * (uint64_t)e;
+            const uint32_t fl = LVM_CONST32(a.bp_flags)[e];
+            const uint64_t v = LVM_GLOBAL_CONST(a.main)[((uint64_t)LVM_CONST32(a.bp_col)[e] << a.log_N) + r];
+            cmem_u64 *bb = LVM_CONST(a.bp_beta) + 6 * (uint64_t)e;
             if (fl & 1) {
-                acc_mad(m00, bb[0], v);
-                acc_mad(m01, bb[1], v);
-                acc_mad(m02, bb[2], v);
+                acc_mad_uniform(m00, bb[0], v);
+                acc_mad_uniform(m01, bb[1], v);
+                acc_mad_uniform(m02, bb[2], v);
             }
             if (fl & 2) {
-                acc_mad(m10, bb[3], v);
-                acc_mad(m11, bb[4], v);
-                acc_mad(m12, bb[5], v);
+                acc_mad_uniform(m10, bb[3], v);
+                acc_mad_uniform(m11, bb[4], v);
+                acc_mad_uniform(m12, bb[5], v);
             }
         }
         for (uint32_t j = 0; j < 2 && s0 + j < a.num_steps; j++) {
@@ -137,10 +155,10 @@ __device__ __forceinline__ fp3 composition_tail(const CompArgs &a, uint32_t r, c
             else
                 acc = f3_add(acc, fp3{acc_reduce(m10), acc_reduce(m11), acc_reduce(m12)});
             for (uint32_t bi = a.step_off[s]; bi < a.step_off[s + 1]; bi++)
-                if (a.b_is_aux[bi])
-                    acc = f3_add(acc, f3_mul(ld3(a.b_beta + 3 * (uint64_t)bi),
-                                             ld3(a.aux + 3 * (((uint64_t)a.b_col[bi] << a.log_N) + r))));
-            h = f3_add(h, f3_mul_base(acc, a.binv[((uint64_t)s << a.log_N) + r]));
+                if (LVM_CONST32(a.b_is_aux)[bi])
+                    acc = f3_add(acc, f3_mul(ld3_arg(a.b_beta + 3 * (uint64_t)bi),
+                                             ld3_row(a.aux + 3 * (((uint64_t)LVM_CONST32(a.b_col)[bi] << a.log_N) + r))));
+            h = f3_add(h, f3_mul_base(acc, LVM_GLOBAL_CONST(a.binv)[((uint64_t)s << a.log_N) + r]));
         }
     }
     return h;

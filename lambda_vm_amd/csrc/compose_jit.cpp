@@ -8,9 +8,21 @@
 // value folded into its zerofier group's sum where its node is computed),
 // compiled for gfx950 with hipRTC and cached per program text for the life of
 // the process. The per-row walk then runs from registers, and the compiler
-// schedules the trace reads ahead of their uses. Arithmetic is the same
-// field.hpp code as the interpreter and performs the same operations per
-// node, so both produce the same values.
+// schedules the trace reads ahead of their uses. Every value is canonical from
+// its load on (the column copies and the argument block are stored so), which
+// halves the corrections of an add or sub against the interpreter's; both
+// produce the same residues.
+//
+// A sum of base values weighted by challenges, the fingerprints z - sum_j
+// alpha^j v_j of the bus interactions, is a chain of subtractions of products
+// whose extension factor is the same for every row. Such a chain is one set of
+// delayed-reduction dot products with scalar operands, 24 instructions per
+// element where a product and a subtraction take about 65, and one reduction.
+//
+// Challenges come through scalar loads and table words through global ones (see
+// LVM_CONST in compose_common.hpp). Together, per launch: three-table stage (2^21
+// x 80, 2^20 x 48, 2^18 x 24, blowup 4) 7.61 -> 5.11 ms, eight VM tables of 2^20
+// rows 7.24 -> 5.57 ms, Quadratic 2^20 x 48 alone 1.31 -> 0.97 ms.
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
@@ -39,11 +51,16 @@ std::string u64lit(uint64_t v) {
     return b;
 }
 
-std::string fp3lit(const uint64_t *v) { return "fp3{" + u64lit(v[0]) + ", " + u64lit(v[1]) + ", " + u64lit(v[2]) + "}"; }
+std::string fp3lit(const uint64_t *v) {
+    return "fp3{" + u64lit(canon(v[0])) + ", " + u64lit(canon(v[1])) + ", " + u64lit(canon(v[2])) + "}";
+}
 
 struct Operand {
     std::string expr;
     bool ext;
+    int node = -1;         // the node computing it, -1: a constant or challenge
+    bool uniform = false;  // an extension value that is the same for every row
+    uint64_t lit = 0;      // the value of a base constant
 };
 
 // Nodes per load window (trace reads of a window are issued together); the
@@ -76,145 +93,246 @@ std::string generate_row(const lvm_program *pg, const std::vector<uint32_t> &roo
         if (root_node[c] >= n || (mode == 0 && root_group[c] >= (uint32_t)COMP_MAX_GROUPS)) return "";
         emits[root_node[c]].push_back((uint32_t)c);
     }
-    uint32_t max_off = 0;
-    bool acc_group[COMP_MAX_GROUPS] = {false, false, false, false};
-    std::vector<std::string> base_slot(pg->num_base_slots), ext_slot(pg->num_ext_slots);
-    std::string body;
-    body.reserve(n * 96);
+    // pass 1: operands resolved through the slot assignment, classes checked
+    struct Node {
+        uint32_t op, x, y;
+        bool ext = false, uniform = false;
+        Operand p, q;
+        uint32_t uses = 0;
+    };
+    std::vector<Node> nodes(n);
+    std::vector<int> base_slot(pg->num_base_slots, -1), ext_slot(pg->num_ext_slots, -1);
     auto operand = [&](uint32_t enc, Operand &o) -> bool {
         const uint32_t kind = enc >> 29, x = enc & 0x1FFFFFFFu;
+        o = Operand();
         switch (kind) {
         case K_BASE_SLOT:
-            if (x >= base_slot.size() || base_slot[x].empty()) return false;
-            o = {base_slot[x], false};
+        case K_EXT_SLOT: {
+            const std::vector<int> &slots = kind == K_EXT_SLOT ? ext_slot : base_slot;
+            if (x >= slots.size() || slots[x] < 0) return false;
+            o.node = slots[x];
+            o.expr = "v" + std::to_string(o.node);
+            o.ext = kind == K_EXT_SLOT;
+            o.uniform = nodes[o.node].uniform;
+            nodes[o.node].uses++;
             return true;
-        case K_EXT_SLOT:
-            if (x >= ext_slot.size() || ext_slot[x].empty()) return false;
-            o = {ext_slot[x], true};
-            return true;
+        }
         case K_BASE_CONST:
             if (x >= pg->num_base_consts) return false;
-            o = {u64lit(pg->base_consts[x]), false};
+            o.lit = canon(pg->base_consts[x]);
+            o.expr = u64lit(o.lit);
+            o.ext = false;
             return true;
         case K_EXT_CONST:
             if (x >= pg->num_ext_consts) return false;
-            o = {fp3lit(pg->ext_consts + 3 * (size_t)x), true};
-            return true;
+            o.expr = fp3lit(pg->ext_consts + 3 * (size_t)x);
+            break;
         case K_RAP:
             if (x >= pg->num_rap) return false;
-            o = {"ld3(a.rap + " + std::to_string(3 * (size_t)x) + ")", true};
-            return true;
+            o.expr = "ld3_arg(a.rap + " + std::to_string(3 * (size_t)x) + ")";
+            break;
         case K_ALPHA:
             if (x >= pg->num_alpha) return false;
-            o = {"ld3(a.alpha + " + std::to_string(3 * (size_t)x) + ")", true};
-            return true;
+            o.expr = "ld3_arg(a.alpha + " + std::to_string(3 * (size_t)x) + ")";
+            break;
         case 6:
             if (!pg->table_offset) return false;
-            o = {"ld3(a.toff)", true};
-            return true;
+            o.expr = "ld3_arg(a.toff)";
+            break;
         default: return false;
         }
+        o.ext = o.uniform = true;
+        return true;
     };
+    for (size_t k = 0; k < n; k++) {
+        const uint64_t w0 = pg->nodes[2 * k], w1 = pg->nodes[2 * k + 1];
+        Node &v = nodes[k];
+        v.op = (uint32_t)w0;
+        v.x = (uint32_t)(w0 >> 32);
+        v.y = (uint32_t)w1;
+        const uint32_t res = (uint32_t)(w1 >> 32), slot = res & 0x7FFFFFFFu;
+        const bool rext = res >> 31;
+        if (slot >= (rext ? ext_slot.size() : base_slot.size())) return "";
+        switch (v.op) {
+        case OP_CONST_BASE:
+            if (!operand(K_BASE_CONST << 29 | v.x, v.p)) return "";
+            break;
+        case OP_VAR: v.ext = !((v.y >> 16) & 1); break;
+        case OP_CONST_EXT:
+        case OP_RAP:
+        case OP_ALPHA:
+        case OP_OFFSET:
+            if (v.x > 0x1FFFFFFFu) return "";
+            if (!operand((v.op == OP_CONST_EXT ? K_EXT_CONST
+                          : v.op == OP_RAP     ? K_RAP
+                          : v.op == OP_ALPHA   ? K_ALPHA
+                                               : 6u) << 29 | v.x, v.p))
+                return "";
+            v.ext = v.uniform = true;
+            break;
+        case OP_ADD:
+        case OP_SUB:
+        case OP_MUL:
+            if (!operand(v.x, v.p) || !operand(v.y, v.q)) return "";
+            v.ext = v.p.ext || v.q.ext;
+            break;
+        case OP_NEG:
+        case OP_EMBED:
+            if (!operand(v.x, v.p)) return "";
+            v.ext = v.op == OP_EMBED || v.p.ext;
+            break;
+        default: return "";
+        }
+        if (v.ext != rext) return "";  // result class differs from its slot class: leave it to the interpreter
+        (rext ? ext_slot : base_slot)[slot] = (int)k;
+    }
+    // pass 2: chains. A link adds or subtracts a term (a product of a base value
+    // and a uniform extension value that nothing else reads) to its rest; a rest
+    // that only the link reads and that is a link itself continues the chain.
+    struct Link {
+        int term = -1;      // the product node
+        bool minus = false;
+        int chain = -1;     // accumulator set
+        bool last = true;   // no further link continues it
+    };
+    std::vector<Link> link(n);
+    std::vector<bool> skip(n, false);  // computed as part of a chain
+    auto only = [&](int k) { return k >= 0 && nodes[k].uses == 1 && emits[k].empty(); };
+    auto is_term = [&](const Operand &o) {
+        if (!only(o.node) || nodes[o.node].op != OP_MUL) return false;
+        const Node &t = nodes[o.node];
+        return (!t.p.ext && t.q.uniform) || (!t.q.ext && t.p.uniform);
+    };
+    int chains = 0;
+    for (size_t k = 0; k < n; k++) {
+        const Node &v = nodes[k];
+        if (!v.ext || (v.op != OP_ADD && v.op != OP_SUB)) continue;
+        const bool q_term = is_term(v.q), p_term = !q_term && v.op == OP_ADD && is_term(v.p);
+        if (!q_term && !p_term) continue;
+        const Operand &rest = q_term ? v.p : v.q;
+        link[k].term = (q_term ? v.q : v.p).node;
+        link[k].minus = v.op == OP_SUB;
+        skip[link[k].term] = true;
+        if (only(rest.node) && link[rest.node].term >= 0) {
+            link[k].chain = link[rest.node].chain;
+            link[rest.node].last = false;
+        } else {
+            link[k].chain = chains++;
+        }
+    }
+    // the operand a chain starts from, kept until its last link
+    std::vector<Operand> chain_rest(chains);
+
+    // pass 3: the source of each node; trace reads are then moved to the front
+    // of their window of jit_load_window() nodes so that a window's loads are in
+    // flight together (they depend on nothing, so the order of values is unchanged)
+    uint32_t max_off = 0;
+    bool acc_group[COMP_MAX_GROUPS] = {false, false, false, false};
+    std::string body;
+    body.reserve(n * 96);
     auto as_ext = [](const Operand &o) { return o.ext ? o.expr : "embed(" + o.expr + ")"; };
-    // per-node source; trace reads are then moved to the front of their
-    // window of jit_load_window() nodes so that a window's loads are in flight
-    // together (they depend on nothing, so the order of values is unchanged)
+    // component q of a uniform extension operand
+    auto component = [&](const Operand &o, int q) -> std::string {
+        const Operand &e = o.node >= 0 ? nodes[o.node].p : o;  // a uniform node is its operand
+        if (e.expr.rfind("ld3_arg(", 0) == 0) return "LVM_CONST(" + e.expr.substr(8, e.expr.size() - 9) + ")[" + std::to_string(q) + "]";
+        return "(" + e.expr + ").c" + std::to_string(q);
+    };
+    auto pow2_log = [](uint64_t c) -> int {
+        return c > 1 && !(c & (c - 1)) && c <= (1ull << 32) ? __builtin_ctzll(c) : -1;
+    };
     std::vector<std::string> node_text(n);
     std::vector<bool> is_load(n, false);
     for (size_t k = 0; k < n; k++) {
-        const uint64_t w0 = pg->nodes[2 * k], w1 = pg->nodes[2 * k + 1];
-        const uint32_t op = (uint32_t)w0, x = (uint32_t)(w0 >> 32), y = (uint32_t)w1, res = (uint32_t)(w1 >> 32);
-        const bool rext = res >> 31;
-        const uint32_t slot = res & 0x7FFFFFFFu;
-        if (slot >= (rext ? ext_slot.size() : base_slot.size())) return "";
+        const Node &nd = nodes[k];
         const std::string v = "v" + std::to_string(k);
+        std::string &t = node_text[k];
         std::string expr;
-        bool ext = false;
-        switch (op) {
-        case OP_CONST_BASE:
-            if (x >= pg->num_base_consts) return "";
-            expr = u64lit(pg->base_consts[x]);
-            break;
-        case OP_CONST_EXT:
-            if (x >= pg->num_ext_consts) return "";
-            expr = fp3lit(pg->ext_consts + 3 * (size_t)x);
-            ext = true;
-            break;
-        case OP_VAR: {
-            const uint32_t col = x & 0xFFFF, is_main = (y >> 16) & 1, off = (y >> 8) & 0xFF;
-            max_off = off > max_off ? off : max_off;
-            const std::string idx = "(((uint64_t)" + std::to_string(col) + " << a.log_N) + f" + std::to_string(off) + ")";
-            if (is_main) {
-                expr = "a.main[" + idx + "]";
-            } else {
-                expr = "ld3(a.aux + 3 * " + idx + ")";
-                ext = true;
+        const bool ext = nd.ext;
+        const Operand &p = nd.p, &q = nd.q;
+        if (skip[k]) continue;
+        if (link[k].term >= 0) {
+            const Node &tm = nodes[link[k].term];
+            const Operand &base = tm.p.ext ? tm.q : tm.p, &uni = tm.p.ext ? tm.p : tm.q;
+            const Operand &rest = (q.node == link[k].term) ? p : q;
+            const std::string A = "c" + std::to_string(link[k].chain) + "_";
+            const bool starts = !(only(rest.node) && link[rest.node].term >= 0);
+            if (starts) {
+                chain_rest[link[k].chain] = rest;
+                for (int j = 0; j < 3; j++) t += "        acc128 " + A + std::to_string(j) + "; acc_zero(" + A + std::to_string(j) + ");\n";
             }
-            break;
-        }
+            // the sum is subtracted at the end: an added term enters negated
+            const std::string b = link[k].minus ? base.expr : "csub(0, " + base.expr + ")";
+            t += "        { const uint64_t e = " + b + ";\n";
+            for (int j = 0; j < 3; j++) t += "        acc_mad_uniform(" + A + std::to_string(j) + ", " + component(uni, j) + ", e);\n";
+            t += "        }\n";
+            if (!link[k].last) continue;
+            const Operand &r0 = chain_rest[link[k].chain];
+            const std::string sum = "fp3{acc_reduce(" + A + "0), acc_reduce(" + A + "1), acc_reduce(" + A + "2)}";
+            expr = r0.ext ? "cf3_sub(" + r0.expr + ", " + sum + ")" : "cf3_base_sub(" + r0.expr + ", " + sum + ")";
+        } else switch (nd.op) {
+        case OP_CONST_BASE:
+        case OP_CONST_EXT:
         case OP_RAP:
         case OP_ALPHA:
-        case OP_OFFSET: {
-            Operand o;
-            if (x > 0x1FFFFFFFu) return "";
-            if (!operand((op == OP_RAP ? K_RAP : op == OP_ALPHA ? K_ALPHA : 6u) << 29 | x, o)) return "";
-            expr = o.expr;
-            ext = true;
+        case OP_OFFSET: expr = p.expr; break;
+        case OP_VAR: {
+            const uint32_t col = nd.x & 0xFFFF, off = (nd.y >> 8) & 0xFF;
+            max_off = off > max_off ? off : max_off;
+            const std::string idx = "(((uint64_t)" + std::to_string(col) + " << a.log_N) + f" + std::to_string(off) + ")";
+            expr = ext ? "ld3_row(a.aux + 3 * " + idx + ")" : "LVM_GLOBAL_CONST(a.main)[" + idx + "]";
             break;
         }
         case OP_ADD:
+            if (!ext)
+                expr = "cadd(" + p.expr + ", " + q.expr + ")";
+            else if (!p.ext || !q.ext)
+                expr = "cf3_add_base(" + (p.ext ? p : q).expr + ", " + (p.ext ? q : p).expr + ")";
+            else
+                expr = "cf3_add(" + p.expr + ", " + q.expr + ")";
+            break;
         case OP_SUB:
-        case OP_MUL: {
-            Operand p, q;
-            if (!operand(x, p) || !operand(y, q)) return "";
-            if (!p.ext && !q.ext) {
-                expr = std::string(op == OP_ADD ? "add(" : op == OP_SUB ? "sub(" : "mul(") + p.expr + ", " + q.expr + ")";
-            } else {
-                ext = true;
-                if (op == OP_MUL && !p.ext)
-                    expr = "f3_mul_base(" + q.expr + ", " + p.expr + ")";
-                else if (op == OP_MUL && !q.ext)
-                    expr = "f3_mul_base(" + p.expr + ", " + q.expr + ")";
+            if (!ext)
+                expr = "csub(" + p.expr + ", " + q.expr + ")";
+            else if (!q.ext)
+                expr = "cf3_sub_base(" + p.expr + ", " + q.expr + ")";
+            else if (!p.ext)
+                expr = "cf3_base_sub(" + p.expr + ", " + q.expr + ")";
+            else
+                expr = "cf3_sub(" + p.expr + ", " + q.expr + ")";
+            break;
+        case OP_MUL:
+            if (!ext) {
+                const int lp = p.node < 0 ? pow2_log(p.lit) : -1, lq = q.node < 0 ? pow2_log(q.lit) : -1;
+                if (lq > 0)
+                    expr = "cmul_pow2<" + std::to_string(lq) + ">(" + p.expr + ")";
+                else if (lp > 0)
+                    expr = "cmul_pow2<" + std::to_string(lp) + ">(" + q.expr + ")";
                 else
-                    expr = std::string(op == OP_ADD ? "f3_add(" : op == OP_SUB ? "f3_sub(" : "f3_mul(") + as_ext(p) +
-                           ", " + as_ext(q) + ")";
+                    expr = "cmul(" + p.expr + ", " + q.expr + ")";
+            } else if (!p.ext || !q.ext) {
+                expr = "cf3_mul_base(" + (p.ext ? p : q).expr + ", " + (p.ext ? q : p).expr + ")";
+            } else {
+                expr = "cf3_mul(" + p.expr + ", " + q.expr + ")";
             }
             break;
+        case OP_NEG: expr = ext ? "cf3_base_sub(0, " + p.expr + ")" : "csub(0, " + p.expr + ")"; break;
+        default: expr = as_ext(p); break;  // OP_EMBED
         }
-        case OP_NEG: {
-            Operand p;
-            if (!operand(x, p)) return "";
-            ext = p.ext;
-            expr = (p.ext ? "f3_neg(" : "neg(") + p.expr + ")";
-            break;
-        }
-        case OP_EMBED: {
-            Operand p;
-            if (!operand(x, p)) return "";
-            ext = true;
-            expr = as_ext(p);
-            break;
-        }
-        default: return "";
-        }
-        if (ext != rext) return "";  // result class differs from its slot class: leave it to the interpreter
-        std::string &t = node_text[k];
-        is_load[k] = op == OP_VAR;
+        is_load[k] = nd.op == OP_VAR;
         t += std::string("        const ") + (ext ? "fp3 " : "uint64_t ") + v + " = " + expr + ";\n";
-        (ext ? ext_slot : base_slot)[slot] = v;
         for (uint32_t c : emits[k]) {
-            const std::string beta = "ld3(a.beta + " + std::to_string(3 * (size_t)c) + ")";
-            if (mode == 0 && ext) {
-                const std::string g = "g" + std::to_string(root_group[c]);
-                t += "        " + g + " = f3_add(" + g + ", f3_mul(" + v + ", " + beta + "));\n";
-            } else if (mode == 0) {
-                // a base-valued constraint enters its group's sum through three
-                // delayed-reduction dot products (one reduction per row)
+            if (mode == 0) {
+                // a constraint enters its group's sum through delayed-reduction dot
+                // products, one per component (one reduction per row): a base value
+                // weighs beta, an extension value's words beta, w beta, w^2 beta
                 const uint32_t g = root_group[c];
                 acc_group[g] = true;
-                for (int q = 0; q < 3; q++)
-                    t += "        acc_mad(A" + std::to_string(g) + "_" + std::to_string(q) + ", a.beta[" +
-                            std::to_string(3 * (size_t)c + q) + "], " + v + ");\n";
+                for (int i = 0; i < (ext ? 3 : 1); i++)
+                    for (int j = 0; j < 3; j++)
+                        t += "        acc_mad_uniform(A" + std::to_string(g) + "_" + std::to_string(j) + ", LVM_CONST(a.beta" +
+                             (ext ? "_w)[" + std::to_string(9 * (size_t)c + 3 * i + j)
+                                  : ")[" + std::to_string(3 * (size_t)c + j)) + "], " + v + (ext ? ".c" + std::to_string(i) : "") +
+                             ");\n";
             } else {
                 t += "        store3(a.out + 3 * ((uint64_t)" + std::to_string(c) + " * N + r), " +
                         (ext ? v : "embed(" + v + ")") + ");\n";
@@ -257,8 +375,8 @@ std::string generate_row(const lvm_program *pg, const std::vector<uint32_t> &roo
 std::string source_prelude() {
     std::string src = "typedef unsigned long long uint64_t;\ntypedef unsigned int uint32_t;\n";
     src += lvm_jit_field_src;
-    src += "\nnamespace lvm {\n__device__ __forceinline__ void store3(uint64_t *o, const fp3 &v) { o[0] = v.c0; o[1] = v.c1; "
-           "o[2] = v.c2; }\n}\n";
+    src += "\nnamespace lvm {\n__device__ __forceinline__ void store3(uint64_t *p, const fp3 &v) { gmem_u64 *o = LVM_GLOBAL(p); "
+           "o[0] = v.c0; o[1] = v.c1; o[2] = v.c2; }\n}\n";
     return src;
 }
 

@@ -302,6 +302,11 @@ LVM_HD uint64_t cdot3(uint64_t a0, uint64_t b0, uint64_t a1, uint64_t b1, uint64
     return csub(cred(lo2, hi3), (uint64_t)over << 32);
 }
 
+// with a base-field operand: a + b, a - b, b - a
+LVM_HD fp3 cf3_add_base(fp3 a, uint64_t b) { return fp3{cadd(a.c0, b), a.c1, a.c2}; }
+LVM_HD fp3 cf3_sub_base(fp3 a, uint64_t b) { return fp3{csub(a.c0, b), a.c1, a.c2}; }
+LVM_HD fp3 cf3_base_sub(uint64_t b, fp3 a) { return fp3{csub(b, a.c0), csub(0, a.c1), csub(0, a.c2)}; }
+
 LVM_HD fp3 cf3_mul(fp3 a, fp3 b) {
     const uint64_t b1_2 = cadd(b.c1, b.c1), b2_2 = cadd(b.c2, b.c2);  // b canonical
     return fp3{cdot3(a.c0, b.c0, a.c1, b2_2, a.c2, b1_2), cdot3(a.c0, b.c1, a.c1, b.c0, a.c2, b2_2),

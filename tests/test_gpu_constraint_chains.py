@@ -1,0 +1,91 @@
+"""Compiled constraint kernels on the forms they rewrite: chains of weighted base
+values with added, subtracted, shared and constant-weighted terms, chains that
+start from a base value, products with powers of two and negations, against the
+oracle's walk of the same program (canonical, exact)."""
+import numpy as np
+import pytest
+
+from lambda_vm_amd import constraint_ir as ir
+from lambda_vm_amd import workload
+
+pytestmark = pytest.mark.gpu
+P = np.uint64(workload.P)
+
+
+def canon(a):
+    a = np.asarray(a, dtype=np.uint64)
+    return np.where(a >= P, a - P, a)
+
+
+def _program():
+    b = ir.IrBuilder()
+    m = [b.main(0, c) for c in range(6)]
+    n0 = b.main(1, 0)
+    x = b.aux(0, 0)
+    al = [b.alpha_power(k) for k in range(5)]
+    z = b.challenge(0)
+    out = [
+        z - m[0] * al[1] - m[1] * al[2] - (m[2] + m[3] * (1 << 16)) * al[3],       # a fingerprint
+        x + m[0] * al[1] - m[1] * al[2] + m[4] * al[4],                           # both signs
+        m[5] - m[0] * z,                                                          # starts from a base value
+        (z - m[0] * al[1]) * (z - m[1] * al[1] - m[2] * al[2]),                   # chains as factors
+        x * (1 << 32) - x * n0,                                                   # extension times base
+    ]
+    shared = m[2] * al[2]                                                         # a term two sums read
+    out += [x - shared, x + shared - m[3] * al[3]]
+    run = z - m[4] * al[1]                                                        # a partial sum read twice
+    out += [run - m[5] * al[2], run * run, -(run), b.const_base(3) * m[0] - m[1] * m[1] * (1 << 8)]
+    for i, c in enumerate(out):
+        b.emit(i, c)
+    return b.finish(0), len(out)
+
+
+def _bitrev_perm(N):
+    bits = N.bit_length() - 1
+    return np.array([int(format(i, f"0{bits}b")[::-1], 2) for i in range(N)])
+
+
+@pytest.mark.parametrize("log_n", [2, 9])
+def test_chain_forms_match_oracle(gpu, ora, log_n):
+    prog, k = _program()
+    dev = ir.lower(prog, pin_roots=False)
+    n, B, g = 1 << log_n, 4, 3
+    w = ora.lde_weights(n, g)
+    hm, lm = gpu.coset_lde_row_major_with_merkle_tree_keep(workload.trace_table(61, 0, n, 6), n, 6, B, w)
+    ha, la = gpu.coset_lde_ext3_row_major_with_merkle_tree_keep(workload.trace_table(61, 1, n, 3), n, 1, B, w)
+    rap, alpha = workload.fp3_values(62, 2), workload.fp3_values(63, 5)
+    rap[0, 1] = alpha[2, 0] = 5
+    betas = workload.fp3_values(64, k)
+    groups, ex = [i % 2 for i in range(k)], [0, 1]
+    ev_ref = ora.eval_constraints(dev, lm, la, B, rap, alpha)
+    ref = ora.eval_composition(dev, lm, la, B, n, g, betas, groups, ex, rap=rap, alpha=alpha)
+    # the same residues as words above p too
+    lift = lambda a: np.where(a < np.uint64((1 << 32) - 1), a + P, a)  # noqa: E731
+    assert (lift(rap) != rap).any() and (lift(alpha) != alpha).any()
+    for r, al in ((rap, alpha), (lift(rap), lift(alpha))):
+        got = gpu.eval_constraints(dev, hm, ha, B, rap=r, alpha=al)
+        assert np.array_equal(canon(got), canon(ev_ref))
+        args = (dev, hm, ha, B, n, g, betas, groups, ex)
+        one = gpu.eval_composition(*args, rap=r, alpha=al).to_array(np.uint64, (n * B, 3))
+        assert np.array_equal(canon(one), canon(ref)[_bitrev_perm(n * B)])
+    many = gpu.eval_composition_batch([dict(dev=dev, main=hm, aux=ha, next_step=B, trace_rows=n, coset_offset=g,
+                                            betas=betas, root_group=groups, group_exemptions=ex, rap=rap,
+                                            alpha=alpha)] * 2)
+    for h in many:
+        assert np.array_equal(canon(h.to_array(np.uint64, (n * B, 3))), canon(ref)[_bitrev_perm(n * B)])
+
+
+def test_rows_above_p(gpu, ora):
+    """A handle over a caller's rows may hold words in [p, 2^64)."""
+    prog, _ = _program()
+    dev = ir.lower(prog, pin_roots=False)
+    n, B = 64, 4
+    rng = np.random.default_rng(7)
+    main = rng.integers(0, (1 << 32) - 1, size=(n * B, 6), dtype=np.uint64)
+    aux = rng.integers(0, (1 << 32) - 1, size=(n * B, 3), dtype=np.uint64)
+    rap, alpha = workload.fp3_values(65, 2), workload.fp3_values(66, 5)
+    res = []
+    for add in (np.uint64(0), P):
+        hs = [gpu.commit_rows_dev(gpu.DeviceBuffer.from_array(t + add), n * B, t.shape[1], n) for t in (main, aux)]
+        res.append((canon(gpu.eval_constraints(dev, *hs, B, rap=rap, alpha=alpha)), [h.root for h in hs]))
+    assert np.array_equal(res[0][0], res[1][0]) and res[0][1] == res[1][1]
