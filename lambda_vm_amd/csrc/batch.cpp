@@ -12,7 +12,7 @@
 //  - leaves: every table's row-pair leaves in one launch;
 //  - Merkle: step s of every table's tree (a wide level, or a subtree top of
 //    up to 6 levels through LDS) in one launch per step;
-//  - the roots gathered into one array and copied to pinned host memory.
+//  - each root goes to pinned host memory from the block that hashes it.
 // Blocks of a launch are assigned to tables by a prefix sum over their block
 // counts, largest table first so the small ones fill the tail. The kernels
 // read their arguments from the arena, so the launch sequence is captured
@@ -41,7 +41,7 @@ struct lvm_batch {
     std::vector<uint64_t *> coef, lde;
     std::vector<uint8_t *> nodes;
 
-    enum Kind { NTT, LEAVES, TREE, ROOTS };
+    enum Kind { NTT, LEAVES, TREE };
     struct Launch {
         Kind kind;
         int r;
@@ -53,7 +53,6 @@ struct lvm_batch {
         double bytes;      // compulsory HBM bytes (each input read once, each output written once)
     };
     std::vector<Launch> launches;
-    size_t roots_off = 0, trees_off = 0;
 
     uint8_t *h_arena = nullptr;  // pinned staging of the descriptors
     uint8_t *d_arena = nullptr;
@@ -95,18 +94,18 @@ struct Writer {
 
 // Tree steps above C nodes (a power of two): wide levels one per
 // step while more than TREE_TOP_CHILDREN children remain, then tree tops.
-std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t C) {
+std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t C, uint32_t root) {
     std::vector<std::pair<TreeStep, uint32_t>> out;  // (step, blocks)
     uint64_t *nodes = (uint64_t *)nodes_b;
     while (C > TREE_TOP_CHILDREN) {
-        TreeStep s{nodes, C - 1, C / 2 - 1, TREE_WIDE_SPAN, 1};
+        TreeStep s{nodes, C - 1, C / 2 - 1, TREE_WIDE_SPAN, 1, root, 0};
         out.push_back({s, (uint32_t)(C / (2 * TREE_WIDE_SPAN))});
         C /= 2;
     }
     while (C > 1) {
         const uint32_t span = (uint32_t)(C / 2 < TREE_TOP_SPAN ? C / 2 : TREE_TOP_SPAN);
         const uint64_t blocks = C / (2 * span);
-        TreeStep s{nodes, C - 1, C / 2 - 1, span, 32};
+        TreeStep s{nodes, C - 1, C / 2 - 1, span, 32, root, 0};
         out.push_back({s, (uint32_t)blocks});
         C = blocks;
     }
@@ -188,7 +187,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
             const lvm_table_desc &d = b->in[t];
             const uint64_t L = d.n * d.blowup / 2;
             const uint32_t span = L <= LEAF_TOP_LEAVES ? leaf_top_span(L) : 0;
-            jobs.push_back({b->lde[t], d.m, L, (uint64_t *)b->nodes[t], span, 0});
+            jobs.push_back({b->lde[t], d.m, L, (uint64_t *)b->nodes[t], span, (uint32_t)t});
             total += span ? L / span : (L + TREE_WIDE_SPAN - 1) / TREE_WIDE_SPAN;
             if (total >= (1ull << 31)) return fail(LVM_ERR_ARG, "batched launch exceeds 2^31 blocks");
             prefix.push_back((uint32_t)total);
@@ -209,7 +208,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         for (size_t t = 0; t < T; t++) {
             const lvm_table_desc &d = b->in[t];
             const uint64_t L = d.n * d.blowup / 2;
-            st[t] = tree_steps(b->nodes[t], L <= LEAF_TOP_LEAVES ? L / leaf_top_span(L) : L);
+            st[t] = tree_steps(b->nodes[t], L <= LEAF_TOP_LEAVES ? L / leaf_top_span(L) : L, (uint32_t)t);
             max_tree = std::max(max_tree, st[t].size());
         }
         for (size_t s = 0; s < max_tree; s++) {
@@ -235,18 +234,6 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
                                        "batch_merkle_s" + std::to_string(s), bytes});
         }
     }
-    // roots, in table index order
-    {
-        std::vector<uint64_t *> trees(T);
-        for (size_t t = 0; t < T; t++) trees[t] = (uint64_t *)b->nodes[t];
-        const size_t to = w.put(trees.data(), T);
-        const size_t ro = w.reserve(T * 32);
-        if (record) {
-            b->trees_off = to;
-            b->roots_off = ro;
-            b->launches.push_back({lvm_batch::ROOTS, 0, false, 0, to, ro, (uint32_t)T, 0, "batch_roots", 64.0 * T});
-        }
-    }
     return LVM_OK;
 }
 
@@ -263,22 +250,17 @@ void enqueue(lvm_batch *b, hipStream_t st, bool profile) {
         case lvm_batch::LEAVES: {
             ProfScope ps(profile ? l.name.c_str() : nullptr, st);
             launch_leaves_batched((const LeafJob *)(base + l.args_off), (const uint32_t *)(base + l.prefix_off),
-                                  l.count, l.blocks, st);
+                                  l.count, l.blocks, (uint64_t *)b->h_roots, st);
             break;
         }
         case lvm_batch::TREE: {
             ProfScope ps(profile ? l.name.c_str() : nullptr, st);
             launch_tree_steps_batched((const TreeStep *)(base + l.args_off), (const uint32_t *)(base + l.prefix_off),
-                                      l.count, l.blocks, st);
+                                      l.count, l.blocks, (uint64_t *)b->h_roots, st);
             break;
         }
-        case lvm_batch::ROOTS:
-            launch_gather_roots((uint64_t *const *)(base + l.args_off), l.count, (uint64_t *)(base + l.prefix_off),
-                                st);
-            break;
         }
     }
-    hipMemcpyAsync(b->h_roots, base + b->roots_off, b->in.size() * 32, hipMemcpyDeviceToHost, st);
 }
 
 int validate(const lvm_table_desc *tables, size_t count) {

@@ -111,24 +111,26 @@ int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blow
         TRY(ntt_coset_expand(coef.as<uint64_t>(), (uint32_t)w, lde.as<uint64_t>(), (uint32_t)w, (uint32_t)w,
                              log2u(n), log2u(blowup), d_weights, d->tb, st));
     }
-    uint64_t C;
-    {
-        ProfScope ps("keccak_leaves", st);
-        C = keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, true, nodes.as<uint8_t>(), st);
-        if (split) keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, true, pre.as<uint8_t>(), st);
-    }
-    {
-        ProfScope ps("merkle_inner", st);
-        merkle_build_inner(nodes.as<uint8_t>(), C, st);
-        if (split) merkle_build_inner(pre.as<uint8_t>(), C, st);
-    }
-    LVM_HIP(hipGetLastError());
-    uint8_t root[32];
+    uint8_t root[32], pre_root[32];
     {
         StageScope ss(st);
-        LVM_HIP(stage_download(root, nodes.as<uint8_t>(), 32, st));
-        if (split && pre_root_out) LVM_HIP(stage_download(pre_root_out, pre.as<uint8_t>(), 32, st));
+        void *r = nullptr, *pr = nullptr;
+        LVM_HIP(stage_result(root, 32, pre_root, split ? 32 : 0, st, &r, &pr));
+        uint64_t C;
+        {
+            ProfScope ps("keccak_leaves", st);
+            C = keccak_row_pair_leaves(lde.as<uint64_t>(), w, split, w, L, true, nodes.as<uint8_t>(), (uint64_t *)r, st);
+            if (split)
+                keccak_row_pair_leaves(lde.as<uint64_t>(), w, 0, split, L, true, pre.as<uint8_t>(), (uint64_t *)pr, st);
+        }
+        {
+            ProfScope ps("merkle_inner", st);
+            merkle_build_inner(nodes.as<uint8_t>(), C, (uint64_t *)r, st);
+            if (split) merkle_build_inner(pre.as<uint8_t>(), C, (uint64_t *)pr, st);
+        }
+        LVM_HIP(hipGetLastError());
         LVM_HIP(stage_sync(st));
+        if (split && pre_root_out) std::memcpy(pre_root_out, pre_root, 32);
         if (split && pre_nodes_host) {
             LVM_HIP(hipMemcpyAsync(pre_nodes_host, pre.p, (2 * L - 1) * 32, hipMemcpyDeviceToHost, st));
             LVM_HIP(hipStreamSynchronize(st));
@@ -350,20 +352,21 @@ int commit_owned_rows(Device *d, hipStream_t st, DevBuf &rows, size_t N, size_t 
     const size_t L = N / 2;
     DevBuf nodes;
     TRY(nodes.alloc((2 * L - 1) * 32, st));
-    uint64_t C;
-    {
-        ProfScope ps("keccak_leaves", st);
-        C = keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, false, nodes.as<uint8_t>(), st);
-    }
-    {
-        ProfScope ps("merkle_inner", st);
-        merkle_build_inner(nodes.as<uint8_t>(), C, st);
-    }
-    LVM_HIP(hipGetLastError());
     uint8_t root[32];
     {
         StageScope ss(st);
-        LVM_HIP(stage_download(root, nodes.as<uint8_t>(), 32, st));
+        void *r = nullptr;
+        LVM_HIP(stage_result(root, 32, nullptr, 0, st, &r, nullptr));
+        uint64_t C;
+        {
+            ProfScope ps("keccak_leaves", st);
+            C = keccak_row_pair_leaves(rows.as<uint64_t>(), w, 0, w, L, false, nodes.as<uint8_t>(), (uint64_t *)r, st);
+        }
+        {
+            ProfScope ps("merkle_inner", st);
+            merkle_build_inner(nodes.as<uint8_t>(), C, (uint64_t *)r, st);
+        }
+        LVM_HIP(hipGetLastError());
         LVM_HIP(stage_sync(st));
     }
     lvm_lde *h = new lvm_lde();
@@ -460,17 +463,24 @@ int lvm_lde_open(const lvm_lde *h, const uint64_t *positions, size_t count, uint
     if (!d) return LVM_ERR_DEVICE;
     hipStream_t st = thread_stream(d);
     const uint32_t depth = log2u(h->L);
+    // small answers go to mapped host memory from the kernel, larger ones by copy
+    const size_t pbytes = count * depth * 32, rbytes = rows_out ? count * 2 * h->w * 8 : 0;
+    const bool direct = pbytes + rbytes <= STAGE_RESULT;
     DevBuf dp, dpaths, drows;
     TRY(dp.alloc(count * 8, st));
-    TRY(dpaths.alloc(count * (depth ? depth : 1) * 32, st));
-    if (rows_out) TRY(drows.alloc(count * 2 * h->w * 8, st));
+    if (!direct) {
+        TRY(dpaths.alloc(pbytes, st));
+        if (rows_out) TRY(drows.alloc(rbytes, st));
+    }
     StageScope ss(st);
     LVM_HIP(stage_upload(dp.p, positions, count * 8, st));
-    launch_open((const uint64_t *)h->nodes, h->L, h->lde, h->w, dp.as<uint64_t>(), count, depth,
-                dpaths.as<uint64_t>(), rows_out ? drows.as<uint64_t>() : nullptr, st);
+    void *pp = dpaths.p, *rp = drows.p;
+    if (direct) LVM_HIP(stage_result(paths_out, pbytes, rows_out, rbytes, st, &pp, &rp));
+    launch_open((const uint64_t *)h->nodes, h->L, h->lde, h->w, dp.as<uint64_t>(), count, depth, (uint64_t *)pp,
+                rows_out ? (uint64_t *)rp : nullptr, st);
     LVM_HIP(hipGetLastError());
-    if (depth) LVM_HIP(stage_download(paths_out, dpaths.p, count * depth * 32, st));
-    if (rows_out) LVM_HIP(stage_download(rows_out, drows.p, count * 2 * h->w * 8, st));
+    if (!direct && depth) LVM_HIP(stage_download(paths_out, dpaths.p, pbytes, st));
+    if (!direct && rows_out) LVM_HIP(stage_download(rows_out, drows.p, rbytes, st));
     LVM_HIP(stage_sync(st));
     return LVM_OK;
 }
@@ -597,7 +607,7 @@ int lvm_build_merkle_tree(const uint8_t *leaves, size_t num_leaves, uint8_t *nod
     DevBuf nodes;
     TRY(nodes.alloc((2 * L - 1) * 32, st));
     LVM_HIP(hipMemcpyAsync(nodes.as<uint8_t>() + (L - 1) * 32, padded.data(), L * 32, hipMemcpyHostToDevice, st));
-    merkle_build_inner(nodes.as<uint8_t>(), L, st);
+    merkle_build_inner(nodes.as<uint8_t>(), L, nullptr, st);
     LVM_HIP(hipGetLastError());
     LVM_HIP(hipMemcpyAsync(nodes_out, nodes.p, (2 * L - 1) * 32, hipMemcpyDeviceToHost, st));
     LVM_HIP(hipStreamSynchronize(st));

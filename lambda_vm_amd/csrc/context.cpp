@@ -405,6 +405,19 @@ hipError_t stage_download(void *dst_host, const void *src_dev, size_t bytes, hip
     return e;
 }
 
+hipError_t stage_result(void *dst_a, size_t bytes_a, void *dst_b, size_t bytes_b, hipStream_t st, void **a, void **b) {
+    Stage &sg = t_stage;
+    const size_t first = (bytes_a + 255) & ~(size_t)255;
+    size_t off = 0;
+    hipError_t e = stage_region(sg, first + bytes_b, st, &off);
+    if (e != hipSuccess) return e;
+    if (bytes_a) sg.pend.push_back(PendingDownload{dst_a, off, bytes_a});
+    if (bytes_b) sg.pend.push_back(PendingDownload{dst_b, off + first, bytes_b});
+    *a = sg.buf + off;
+    if (b) *b = sg.buf + off + first;
+    return hipSuccess;
+}
+
 hipError_t stage_sync(hipStream_t st) {
     Stage &sg = t_stage;
     hipError_t e = hipStreamSynchronize(st);

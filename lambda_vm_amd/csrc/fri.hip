@@ -40,6 +40,8 @@ struct FoldJob {
     uint64_t ginv;  // inverse of the codeword's coset offset
     uint32_t log_half;
     uint32_t span;
+    uint32_t root;  // the layer tree's slot in the launch's root array
+    uint32_t pad;
 };
 
 __device__ __forceinline__ fp3 fold_one(const uint64_t *in, uint64_t j, fp3 zeta, uint64_t ginv, uint32_t log_half,
@@ -96,10 +98,11 @@ __device__ __forceinline__ void fri_fold_body(const FoldJob &j, uint64_t t, cons
 // thread, then leaves and the tree levels above them, one permutation per 16
 // lanes. A layer of up to LEAF_TOP_LEAVES leaves has too few to fill the chip
 // with one leaf per lane; what its tree costs is the chain of permutations.
-__device__ __forceinline__ void fri_fold_top(const FoldJob &j, uint64_t b, const uint64_t *ilo, const uint64_t *ihi) {
+__device__ __forceinline__ void fri_fold_top(const FoldJob &j, uint64_t b, const uint64_t *ilo, const uint64_t *ihi,
+                                             uint64_t *roots) {
     __shared__ TreeTopLds s;
     __shared__ uint64_t s_val[TREE_TOP_SPAN][6];  // a leaf's two elements, canonical
-    const TreeTop t(s);
+    const TreeTop t(s, roots + 4 * j.root);
     const uint64_t first = (uint64_t)j.span * b, L = j.half / 2;
     if (threadIdx.x < 2 * j.span) {
         const uint64_t e = 2 * first + threadIdx.x;
@@ -139,15 +142,16 @@ inline uint64_t fold_blocks(const FoldJob &j) {
 }
 
 __device__ __forceinline__ void fri_fold_block(const FoldJob &j, uint64_t b, const uint64_t *ilo,
-                                               const uint64_t *ihi) {
+                                               const uint64_t *ihi, uint64_t *roots) {
     if (j.span)
-        fri_fold_top(j, b, ilo, ihi);
+        fri_fold_top(j, b, ilo, ihi, roots);
     else
         fri_fold_body(j, b * FOLD_THREADS + threadIdx.x, ilo, ihi);
 }
 
-__global__ __launch_bounds__(FOLD_THREADS) void fri_fold_kernel(FoldJob j, const uint64_t *ilo, const uint64_t *ihi) {
-    fri_fold_block(j, blockIdx.x, ilo, ihi);
+__global__ __launch_bounds__(FOLD_THREADS) void fri_fold_kernel(FoldJob j, const uint64_t *ilo, const uint64_t *ihi,
+                                                                uint64_t *roots) {
+    fri_fold_block(j, blockIdx.x, ilo, ihi, roots);
 }
 
 // The same fold for several codewords in one launch: blocks [prefix[t],
@@ -155,31 +159,36 @@ __global__ __launch_bounds__(FOLD_THREADS) void fri_fold_kernel(FoldJob j, const
 __global__ __launch_bounds__(FOLD_THREADS) void fri_fold_batched_kernel(const FoldJob *__restrict__ jobs,
                                                                         const uint32_t *__restrict__ prefix,
                                                                         uint32_t count, const uint64_t *ilo,
-                                                                        const uint64_t *ihi) {
+                                                                        const uint64_t *ihi, uint64_t *roots) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const FoldJob j = jobs[t];
-    fri_fold_block(j, b - prefix[t], ilo, ihi);
+    fri_fold_block(j, b - prefix[t], ilo, ihi, roots);
 }
 
-// Symmetric evaluations and authentication paths of one layer for every
-// query (crypto/stark/src/fri/mod.rs:153-205): index_l = iota >> l,
-// eval_sym = e_l[index_l ^ 1], path of leaf index_l >> 1.
-__global__ void fri_query_layer_kernel(const uint64_t *evals, const uint64_t *nodes, uint64_t L, uint32_t depth,
-                                       const uint64_t *iotas, uint64_t count, uint32_t layer, uint64_t *sym_out,
-                                       uint64_t *paths_out) {
-    uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= count) return;
-    uint64_t idx = iotas[q] >> layer;
-    const uint64_t *e = evals + 3 * (idx ^ 1);
-    sym_out[3 * q] = e[0];
-    sym_out[3 * q + 1] = e[1];
-    sym_out[3 * q + 2] = e[2];
-    uint64_t node = (idx >> 1) + L - 1;
-    for (uint32_t k = 0; k < depth; k++) {
-        uint64_t sib = (node % 2 == 0) ? node - 1 : node + 1;
-        for (int w = 0; w < 4; w++) paths_out[(q * depth + k) * 4 + w] = nodes[sib * 4 + w];
-        node = (node % 2 == 0) ? (node - 1) / 2 : node / 2;
+// Symmetric evaluations and authentication paths of every layer for every
+// query (crypto/stark/src/fri/mod.rs:153-205): index_l = iota >> l, eval_sym =
+// e_l[index_l ^ 1], path of leaf index_l >> 1. Block (query, layer), all words
+// read at once (level k's L >> k nodes start at (L >> k) - 1); 13 launches of 30
+// threads walking a path each took 12 us apiece.
+struct QueryLayer {
+    const uint64_t *evals, *nodes;
+    uint64_t L;
+    uint64_t paths_off;  // words before the layer's paths
+    uint32_t depth;
+    uint32_t pad;
+};
+__global__ __launch_bounds__(128) void fri_query_kernel(const QueryLayer *__restrict__ layers,
+                                                        const uint64_t *__restrict__ iotas, uint64_t count,
+                                                        uint64_t *sym_out, uint64_t *paths_out) {
+    const uint64_t q = blockIdx.x;
+    const uint32_t li = blockIdx.y;
+    const QueryLayer l = layers[li];
+    const uint64_t idx = iotas[q] >> li, p = idx >> 1;
+    if (threadIdx.x < 3) sym_out[(li * count + q) * 3 + threadIdx.x] = l.evals[3 * (idx ^ 1) + threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < 4 * l.depth; i += 128) {
+        const uint32_t k = i / 4;
+        paths_out[l.paths_off + q * l.depth * 4 + i] = l.nodes[4 * ((l.L >> k) - 1 + ((p >> k) ^ 1)) + i % 4];
     }
 }
 
@@ -277,19 +286,21 @@ static int fri_fold_impl(lvm_fri *f, const uint64_t zeta[3], bool commit, uint8_
     const uint64_t ginv = inv(f->offset);
     const uint32_t log_half = log2u(half);
     const uint32_t span = commit ? fold_span(layer.L) : 0;
-    {
-        ProfScope ps(commit ? "fri_fold_leaves" : "fri_fold", st);
-        const FoldJob j{f->cur, out, (uint64_t *)layer.nodes, half, zeta[0], zeta[1], zeta[2], ginv, log_half, span};
-        hipLaunchKernelGGL(fri_fold_kernel, dim3((unsigned)fold_blocks(j)), dim3(FOLD_THREADS), 0, st, j,
-                           d->tb.inv_lo, d->tb.inv_hi);
-    }
-    if (commit) {
-        ProfScope ps("fri_merkle", st);
-        merkle_build_inner(layer.nodes, span ? layer.L / span : layer.L, st);
-    }
     StageScope ss(st);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && commit) e = stage_download(layer.root, layer.nodes, 32, st);
+    void *root = nullptr;
+    hipError_t e = commit ? stage_result(layer.root, 32, nullptr, 0, st, &root, nullptr) : hipSuccess;
+    if (e == hipSuccess) {
+        ProfScope ps(commit ? "fri_fold_leaves" : "fri_fold", st);
+        const FoldJob j{f->cur, out, (uint64_t *)layer.nodes, half, zeta[0], zeta[1], zeta[2], ginv, log_half, span,
+                        0, 0};
+        hipLaunchKernelGGL(fri_fold_kernel, dim3((unsigned)fold_blocks(j)), dim3(FOLD_THREADS), 0, st, j,
+                           d->tb.inv_lo, d->tb.inv_hi, (uint64_t *)root);
+    }
+    if (e == hipSuccess && commit) {
+        ProfScope ps("fri_merkle", st);
+        merkle_build_inner(layer.nodes, span ? layer.L / span : layer.L, (uint64_t *)root, st);
+    }
+    if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = stage_sync(st);
     if (e != hipSuccess) {
         lvm_free(out);
@@ -318,8 +329,8 @@ namespace lvm {
 
 // One fold of every codeword fs[0..count) (zeta t at zetas[3t]) on the
 // calling thread's stream: one work-list launch for the folds (and their
-// leaves), one launch per tree step over all layer trees, one copy of all
-// roots. Each state then holds what fri_fold_impl would leave. On a device
+// leaves), one launch per tree step over all layer trees, roots written to
+// mapped host memory. Each state then holds what fri_fold_impl would leave. On a device
 // error no state changes.
 int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool commit, uint8_t *roots_out) {
     if (!fs || !zetas || (commit && !roots_out)) return fail(LVM_ERR_ARG, "null argument");
@@ -343,7 +354,7 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
         }
         lvm_free(arena);
     };
-    // descriptors: fold jobs + block prefix, then per tree step the steps + prefix, then the tree pointers
+    // descriptors: fold jobs + block prefix, then per tree step the steps + prefix
     std::vector<FoldJob> jobs(count);
     std::vector<uint32_t> prefix(1, 0);
     uint64_t total = 0;
@@ -363,11 +374,12 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
                 return fail(LVM_ERR_NOMEM, "FRI tree allocation failed");
             }
             const uint32_t span = fold_span(layers[t].L);
-            tsteps[t] = tree_steps(layers[t].nodes, span ? layers[t].L / span : layers[t].L);
+            tsteps[t] = tree_steps(layers[t].nodes, span ? layers[t].L / span : layers[t].L, (uint32_t)t);
             max_steps = std::max(max_steps, tsteps[t].size());
         }
         jobs[t] = FoldJob{f->cur, outs[t], (uint64_t *)layers[t].nodes, half, zetas[3 * t], zetas[3 * t + 1],
-                          zetas[3 * t + 2], inv(f->offset), log2u(half), commit ? fold_span(layers[t].L) : 0};
+                          zetas[3 * t + 2], inv(f->offset), log2u(half), commit ? fold_span(layers[t].L) : 0,
+                          (uint32_t)t, 0};
         total += fold_blocks(jobs[t]);
         if (total >= (1ull << 31)) {
             release();
@@ -402,32 +414,27 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
         steps_l.push_back({put(steps.data(), steps.size() * sizeof(TreeStep)), put(sp.data(), sp.size() * 4),
                            (uint32_t)steps.size(), (uint32_t)sb});
     }
-    std::vector<uint64_t *> trees(count);
-    for (size_t t = 0; t < count; t++) trees[t] = (uint64_t *)layers[t].nodes;
-    const size_t o_trees = put(trees.data(), count * sizeof(uint64_t *));
-    const size_t o_roots = (blob.size() + 15) & ~(size_t)15;  // the gathered roots
-    blob.resize(o_roots + count * 32);
     if (lvm_malloc(&arena, blob.size()) != hipSuccess) {
         release();
         return fail(LVM_ERR_NOMEM, "FRI descriptor allocation failed");
     }
     StageScope ss(st);
     hipError_t e = stage_upload(arena, blob.data(), blob.size(), st);
+    void *roots = nullptr;
+    if (e == hipSuccess && commit) e = stage_result(roots_out, count * 32, nullptr, 0, st, &roots, nullptr);
     if (e == hipSuccess) {
         ProfScope ps(commit ? "fri_fold_leaves" : "fri_fold", st);
         hipLaunchKernelGGL(fri_fold_batched_kernel, dim3((unsigned)total), dim3(FOLD_THREADS), 0, st,
                            (const FoldJob *)(arena + o_jobs), (const uint32_t *)(arena + o_prefix), (uint32_t)count,
-                           d->tb.inv_lo, d->tb.inv_hi);
+                           d->tb.inv_lo, d->tb.inv_hi, (uint64_t *)roots);
     }
     if (e == hipSuccess && commit) {
         ProfScope ps("fri_merkle", st);
         for (const StepLaunch &l : steps_l)
             launch_tree_steps_batched((const TreeStep *)(arena + l.steps_off), (const uint32_t *)(arena + l.prefix_off),
-                                      l.count, l.blocks, st);
-        launch_gather_roots((uint64_t *const *)(arena + o_trees), (uint32_t)count, (uint64_t *)(arena + o_roots), st);
+                                      l.count, l.blocks, (uint64_t *)roots, st);
     }
     if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess && commit) e = stage_download(roots_out, arena + o_roots, count * 32, st);
     if (e == hipSuccess) e = stage_sync(st);
     if (e != hipSuccess) {
         release();
@@ -504,9 +511,22 @@ int lvm_fri_query(const lvm_fri *f, const uint64_t *iotas, size_t count, uint64_
     Device *d = device_state();
     if (!d) return LVM_ERR_DEVICE;
     hipStream_t st = thread_stream(d);
-    // per layer: count sym evals (3 u64) and count paths (depth_l x 32 bytes)
+    if (count >= (1u << 31)) return fail(LVM_ERR_ARG, "too many queries");
+    // per layer: count sym evals (3 u64) and count paths (depth_l x 32 bytes);
+    // the layers' descriptors and the indexes go up in one blob
+    const size_t layers = f->layers.size();
+    std::vector<uint64_t> blob((layers * sizeof(QueryLayer)) / 8 + count);
+    QueryLayer *ql = (QueryLayer *)blob.data();
     size_t path_words = 0;
-    for (auto &l : f->layers) path_words += count * log2u(l.L) * 4;
+    for (size_t li = 0; li < layers; li++) {
+        const FriLayer &l = f->layers[li];
+        ql[li] = QueryLayer{l.evals, (const uint64_t *)l.nodes, l.L, path_words, log2u(l.L), 0};
+        path_words += count * log2u(l.L) * 4;
+    }
+    std::memcpy(blob.data() + layers * sizeof(QueryLayer) / 8, iotas, count * 8);
+    const size_t sbytes = layers * count * 24, pbytes = path_words * 8;
+    // small answers go to mapped host memory from the kernel, larger ones by copy
+    const bool direct = sbytes + pbytes <= STAGE_RESULT;
     // released on every exit (stream-ordered: a block is reused on this stream
     // only after the work queued before its release)
     struct Owned {
@@ -514,24 +534,24 @@ int lvm_fri_query(const lvm_fri *f, const uint64_t *iotas, size_t count, uint64_
         ~Owned() {
             if (p) lvm_free(p);
         }
-    } dio, dsym, dpaths;
-    LVM_HIP(lvm_malloc(&dio.p, count * 8));
-    LVM_HIP(lvm_malloc(&dsym.p, f->layers.size() * count * 24));
-    LVM_HIP(lvm_malloc(&dpaths.p, (path_words ? path_words : 1) * 8));
-    StageScope ss(st);
-    LVM_HIP(stage_upload(dio.p, iotas, count * 8, st));
-    size_t poff = 0;
-    for (size_t li = 0; li < f->layers.size(); li++) {
-        const FriLayer &l = f->layers[li];
-        uint32_t depth = log2u(l.L);
-        hipLaunchKernelGGL(fri_query_layer_kernel, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, st, l.evals,
-                           (const uint64_t *)l.nodes, l.L, depth, dio.p, count, (uint32_t)li,
-                           dsym.p + li * count * 3, dpaths.p + poff);
-        poff += count * depth * 4;
+    } dblob, dsym, dpaths;
+    LVM_HIP(lvm_malloc(&dblob.p, blob.size() * 8));
+    if (!direct) {
+        LVM_HIP(lvm_malloc(&dsym.p, sbytes));
+        LVM_HIP(lvm_malloc(&dpaths.p, pbytes ? pbytes : 8));
     }
+    StageScope ss(st);
+    LVM_HIP(stage_upload(dblob.p, blob.data(), blob.size() * 8, st));
+    void *sym = dsym.p, *paths = dpaths.p;
+    if (direct) LVM_HIP(stage_result(evals_sym_out, sbytes, paths_out, pbytes, st, &sym, &paths));
+    hipLaunchKernelGGL(fri_query_kernel, dim3((unsigned)count, (unsigned)layers), dim3(128), 0, st,
+                       (const QueryLayer *)dblob.p, dblob.p + layers * sizeof(QueryLayer) / 8, (uint64_t)count,
+                       (uint64_t *)sym, (uint64_t *)paths);
     LVM_HIP(hipGetLastError());
-    LVM_HIP(stage_download(evals_sym_out, dsym.p, f->layers.size() * count * 24, st));
-    if (path_words) LVM_HIP(stage_download(paths_out, dpaths.p, path_words * 8, st));
+    if (!direct) {
+        LVM_HIP(stage_download(evals_sym_out, dsym.p, sbytes, st));
+        if (pbytes) LVM_HIP(stage_download(paths_out, dpaths.p, pbytes, st));
+    }
     LVM_HIP(stage_sync(st));
     return LVM_OK;
 }

@@ -86,6 +86,13 @@ inline hipError_t lvm_malloc(T **p, size_t bytes) {
 hipError_t stage_upload(void *dst_dev, const void *src_host, size_t bytes, hipStream_t st);
 hipError_t stage_download(void *dst_host, const void *src_dev, size_t bytes, hipStream_t st);
 hipError_t stage_sync(hipStream_t st);
+// Room in the area for one or two results that kernels queued next on `st`
+// write themselves (page-locked memory is mapped): the bytes reach the
+// destinations at stage_sync, without a copy's launch. For results of up to
+// STAGE_RESULT bytes, written once. No other stage_* call may come between this
+// one and the last of those kernels' launches (it could drain the area).
+constexpr size_t STAGE_RESULT = 64 << 10;
+hipError_t stage_result(void *dst_a, size_t bytes_a, void *dst_b, size_t bytes_b, hipStream_t st, void **a, void **b);
 struct StageScope {
     explicit StageScope(hipStream_t st);
     ~StageScope();
@@ -149,11 +156,12 @@ int ntt_coset_expand(const uint64_t *coef, uint32_t coef_pitch, uint64_t *lde, u
 // into node L-1+i of the tree. Small tables' blocks go on to the levels above
 // their leaves; returns the nodes C of the topmost level written, which lie at
 // [C-1, 2C-1): what merkle_build_inner goes on from. canonical: every word is
-// known to be below p (the NTT's output).
+// known to be below p (the NTT's output). root_out (nullable, here and below):
+// where the block that hashes the root writes it too.
 uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
-                                bool canonical, uint8_t *nodes, hipStream_t st);
+                                bool canonical, uint8_t *nodes, uint64_t *root_out, hipStream_t st);
 // the levels above the C nodes (a power of two) at [C-1, 2C-1) of a tree
-void merkle_build_inner(uint8_t *nodes, uint64_t C, hipStream_t st);
+void merkle_build_inner(uint8_t *nodes, uint64_t C, uint64_t *root_out, hipStream_t st);
 
 size_t padded_leaves(size_t n);
 
@@ -207,13 +215,15 @@ struct LeafJob {
     uint64_t num_leaves;
     uint64_t *nodes;       // the table's tree
     uint32_t span;         // leaves per block of a small table (leaf_top_span), 0: TREE_THREADS of them, no levels
-    uint32_t pad;
+    uint32_t root;         // the table's slot in the launch's root array
 };
 struct TreeStep {
     uint64_t *nodes;
     uint64_t cstart, pstart;  // first child / first parent index of the level
     uint32_t span;            // parents per block at the first level
     uint32_t levels;          // levels this step builds
+    uint32_t root;            // the tree's slot in the launch's root array
+    uint32_t pad;
 };
 // Trees of more children than this have their level hashed one node per lane;
 // below, the step is a tree top: blocks of TREE_TOP_SPAN parents, all their
@@ -225,16 +235,16 @@ constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
 // too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch.
 constexpr uint64_t LEAF_TOP_LEAVES = 1u << 13;
 inline uint32_t leaf_top_span(uint64_t L) { return (uint32_t)(L < TREE_TOP_SPAN ? L : TREE_TOP_SPAN); }
+// roots: 32-byte slots, written by the blocks that hash a root
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
-                           hipStream_t st);
+                           uint64_t *roots, hipStream_t st);
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
-                               hipStream_t st);
-void launch_gather_roots(uint64_t *const *d_trees, uint32_t count, uint64_t *d_roots, hipStream_t st);
+                               uint64_t *roots, hipStream_t st);
 // One FRI fold of each of count codewords in shared launches (fri.hip);
 // zetas: count x 3; roots_out (count x 32) when committing.
 int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool commit, uint8_t *roots_out);
 // the launches above the C nodes (a power of two) at [C-1, 2C-1) of a tree: (step, blocks)
-std::vector<std::pair<TreeStep, uint32_t>> tree_steps(uint8_t *nodes, uint64_t C);
+std::vector<std::pair<TreeStep, uint32_t>> tree_steps(uint8_t *nodes, uint64_t C, uint32_t root);
 
 // Constraint programs (compose.hip interpreter, compose_jit.cpp compiled form).
 struct CompArgs;

@@ -73,9 +73,10 @@ __device__ __forceinline__ void row_pair_leaf(const uint64_t *__restrict__ rows,
 // LEAF_TOP_LEAVES leaves would fill at most an eighth of the chip's lanes with
 // one leaf each, at 7.2 us per absorbed block; nodes is the whole tree.
 __device__ __forceinline__ void row_pair_leaf_top(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1,
-                                                  uint64_t L, uint32_t span, uint64_t b, uint64_t *nodes) {
+                                                  uint64_t L, uint32_t span, uint64_t b, uint64_t *nodes,
+                                                  uint64_t *root) {
     __shared__ TreeTopLds s;
-    const TreeTop t(s);
+    const TreeTop t(s, root);
     const uint64_t first = (uint64_t)span * b;
     if (t.wave_on(span)) {
         const bool on = t.g < span;
@@ -116,8 +117,8 @@ __device__ __forceinline__ void row_pair_leaf_top(const uint64_t *rows, uint64_t
 
 __global__ __launch_bounds__(TREE_THREADS) void leaf_top_kernel(const uint64_t *rows, uint64_t pitch, uint64_t w0,
                                                                 uint64_t w1, uint64_t L, uint32_t span,
-                                                                uint64_t *nodes) {
-    row_pair_leaf_top(rows, pitch, w0, w1, L, span, blockIdx.x, nodes);
+                                                                uint64_t *nodes, uint64_t *root) {
+    row_pair_leaf_top(rows, pitch, w0, w1, L, span, blockIdx.x, nodes, root);
 }
 
 template <bool CONTIG, bool CANON>
@@ -135,12 +136,13 @@ __global__ __launch_bounds__(256) void keccak_row_pair_leaves_kernel(const uint6
 // levels above for a small table.
 __global__ __launch_bounds__(TREE_THREADS) void keccak_leaves_batched_kernel(const LeafJob *__restrict__ jobs,
                                                                             const uint32_t *__restrict__ prefix,
-                                                                            uint32_t count) {
+                                                                            uint32_t count, uint64_t *roots) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const LeafJob j = jobs[t];
     if (j.span) {
-        row_pair_leaf_top(j.rows, j.pitch, 0, j.pitch, j.num_leaves, j.span, b - prefix[t], j.nodes);
+        row_pair_leaf_top(j.rows, j.pitch, 0, j.pitch, j.num_leaves, j.span, b - prefix[t], j.nodes,
+                          roots + 4 * j.root);
         return;
     }
     const uint64_t i = (uint64_t)(b - prefix[t]) * TREE_THREADS + threadIdx.x;
@@ -177,9 +179,9 @@ __global__ __launch_bounds__(256) void merkle_level_kernel(uint64_t *nodes, uint
 // A tree of 2^11 leaves: 98 -> 48 us against one lane per node with its rounds
 // unrolled; 2^17 leaves (top of 2^14): 130 -> 62 us.
 __device__ __forceinline__ void merkle_top_body(uint64_t *nodes, uint64_t cstart, uint64_t pstart, uint32_t span,
-                                                uint64_t b) {
+                                                uint64_t b, uint64_t *root) {
     __shared__ TreeTopLds s;
-    const TreeTop t(s);
+    const TreeTop t(s, root);
     const uint64_t pbase = pstart + (uint64_t)span * b;  // first parent of this block
     if (t.wave_on(span)) {
         const bool on = t.g < span;
@@ -192,31 +194,22 @@ __device__ __forceinline__ void merkle_top_body(uint64_t *nodes, uint64_t cstart
 }
 
 __global__ __launch_bounds__(TREE_THREADS) void merkle_top_kernel(uint64_t *nodes, uint64_t cstart, uint64_t pstart,
-                                                                  uint32_t span) {
-    merkle_top_body(nodes, cstart, pstart, span, blockIdx.x);
+                                                                  uint32_t span, uint64_t *root) {
+    merkle_top_body(nodes, cstart, pstart, span, blockIdx.x, root);
 }
 
 // One tree step for each of several trees: blocks [prefix[t], prefix[t+1])
 // run step t (one wide level, TREE_THREADS parents per block, or a tree top).
 __global__ __launch_bounds__(TREE_THREADS) void merkle_steps_batched_kernel(const TreeStep *__restrict__ steps,
                                                                             const uint32_t *__restrict__ prefix,
-                                                                            uint32_t count) {
+                                                                            uint32_t count, uint64_t *roots) {
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const TreeStep s = steps[t];
     if (s.span > TREE_TOP_SPAN)
         merkle_parent(s.nodes, s.pstart + (uint64_t)s.span * (b - prefix[t]) + threadIdx.x);
     else
-        merkle_top_body(s.nodes, s.cstart, s.pstart, s.span, b - prefix[t]);
-}
-
-// Copy each tree's root (node 0) into roots[t].
-__global__ void gather_roots_kernel(uint64_t *const *__restrict__ trees, uint32_t count, uint64_t *__restrict__ roots) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    const uint64_t *r = trees[t];
-#pragma unroll
-    for (int k = 0; k < 4; k++) roots[4 * t + k] = r[k];
+        merkle_top_body(s.nodes, s.cstart, s.pstart, s.span, b - prefix[t], roots + 4 * s.root);
 }
 
 size_t padded_leaves(size_t n) {
@@ -226,11 +219,11 @@ size_t padded_leaves(size_t n) {
 }
 
 uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w0, uint64_t w1, uint64_t L,
-                                bool canonical, uint8_t *nodes, hipStream_t st) {
+                                bool canonical, uint8_t *nodes, uint64_t *root_out, hipStream_t st) {
     if (L <= LEAF_TOP_LEAVES) {
         const uint32_t span = leaf_top_span(L);
         hipLaunchKernelGGL(leaf_top_kernel, dim3((unsigned)(L / span)), dim3(TREE_THREADS), 0, st, rows, pitch, w0, w1,
-                           L, span, (uint64_t *)nodes);
+                           L, span, (uint64_t *)nodes, root_out);
         return L / span;
     }
     uint64_t *leaves = (uint64_t *)(nodes + (L - 1) * 32);
@@ -248,7 +241,7 @@ uint64_t keccak_row_pair_leaves(const uint64_t *rows, uint64_t pitch, uint64_t w
     return L;
 }
 
-void merkle_build_inner(uint8_t *nodes_b, uint64_t C, hipStream_t st) {
+void merkle_build_inner(uint8_t *nodes_b, uint64_t C, uint64_t *root_out, hipStream_t st) {
     uint64_t *nodes = (uint64_t *)nodes_b;
     // wide levels: one fully parallel launch per level
     while (C > TREE_TOP_CHILDREN) {
@@ -262,26 +255,23 @@ void merkle_build_inner(uint8_t *nodes_b, uint64_t C, hipStream_t st) {
         const uint32_t span = (uint32_t)(C / 2 < TREE_TOP_SPAN ? C / 2 : TREE_TOP_SPAN);
         const uint64_t blocks = C / (2 * span);
         hipLaunchKernelGGL(merkle_top_kernel, dim3((unsigned)blocks), dim3(TREE_THREADS), 0, st, nodes, C - 1,
-                           C / 2 - 1, span);
+                           C / 2 - 1, span, root_out);
         C = blocks;
     }
 }
 
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
-                           hipStream_t st) {
+                           uint64_t *roots, hipStream_t st) {
     if (blocks)
         hipLaunchKernelGGL(keccak_leaves_batched_kernel, dim3(blocks), dim3(TREE_THREADS), 0, st, d_jobs, d_prefix,
-                           count);
+                           count, roots);
 }
 
 void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
-                               hipStream_t st) {
+                               uint64_t *roots, hipStream_t st) {
     if (blocks)
-        hipLaunchKernelGGL(merkle_steps_batched_kernel, dim3(blocks), dim3(TREE_THREADS), 0, st, d_steps, d_prefix, count);
-}
-
-void launch_gather_roots(uint64_t *const *d_trees, uint32_t count, uint64_t *d_roots, hipStream_t st) {
-    if (count) hipLaunchKernelGGL(gather_roots_kernel, dim3((count + 63) / 64), dim3(64), 0, st, d_trees, count, d_roots);
+        hipLaunchKernelGGL(merkle_steps_batched_kernel, dim3(blocks), dim3(TREE_THREADS), 0, st, d_steps, d_prefix, count,
+                           roots);
 }
 
 }  // namespace lvm

@@ -69,28 +69,31 @@ void launch_gather_bitrev_rows(const uint64_t *src, uint64_t *dst, uint64_t rows
 // Merkle authentication paths (sibling of each node from the leaf up,
 // crypto/crypto/src/merkle_tree/merkle.rs:291-308) and the two opened rows
 // per position (physical rows 2*pos and 2*pos+1 of the bit-reversed table).
-__global__ void open_kernel(const uint64_t *nodes, uint64_t L, const uint64_t *lde, uint64_t w,
-                            const uint64_t *pos, uint64_t count, uint32_t depth, uint64_t *paths,
-                            uint64_t *rows) {
-    uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= count) return;
-    uint64_t p = pos[q];
-    uint64_t idx = p + L - 1;
-    for (uint32_t k = 0; k < depth; k++) {
-        uint64_t sib = (idx % 2 == 0) ? idx - 1 : idx + 1;
-        for (int j = 0; j < 4; j++) paths[(q * depth + k) * 4 + j] = nodes[sib * 4 + j];
-        idx = (idx % 2 == 0) ? (idx - 1) / 2 : idx / 2;
+// One block per position, every path node and row word read at once: level k's
+// L >> k nodes start at (L >> k) - 1, so the sibling of leaf p's ancestor there
+// is node (L >> k) - 1 + ((p >> k) ^ 1). 30 positions of a 2^21-leaf tree: a
+// thread walking its path and rows took 43 us.
+__global__ __launch_bounds__(256) void open_kernel(const uint64_t *__restrict__ nodes, uint64_t L,
+                                                   const uint64_t *__restrict__ lde, uint64_t w,
+                                                   const uint64_t *__restrict__ pos, uint32_t depth, uint64_t *paths,
+                                                   uint64_t *rows) {
+    const uint64_t q = blockIdx.x, p = pos[q];
+    for (uint32_t i = threadIdx.x; i < 4 * depth; i += 256) {
+        const uint32_t k = i / 4;
+        paths[q * depth * 4 + i] = nodes[4 * ((L >> k) - 1 + ((p >> k) ^ 1)) + i % 4];
     }
-    if (rows) {
-        for (uint64_t j = 0; j < 2 * w; j++) rows[q * 2 * w + j] = lde[2 * p * w + j];
-    }
+    if (rows)
+        for (uint64_t j = threadIdx.x; j < 2 * w; j += 256) rows[q * 2 * w + j] = lde[2 * p * w + j];
 }
 
 void launch_open(const uint64_t *nodes, uint64_t L, const uint64_t *lde, uint64_t w, const uint64_t *pos,
                  uint64_t count, uint32_t depth, uint64_t *paths, uint64_t *rows, hipStream_t st) {
-    if (!count) return;
-    hipLaunchKernelGGL(open_kernel, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, st, nodes, L, lde, w, pos,
-                       count, depth, paths, rows);
+    // launches of at most 2^30 positions
+    for (uint64_t q = 0; q < count; q += 1u << 30) {
+        const uint64_t n = count - q < (1u << 30) ? count - q : 1u << 30;
+        hipLaunchKernelGGL(open_kernel, dim3((unsigned)n), dim3(256), 0, st, nodes, L, lde, w, pos + q, depth,
+                           paths + q * depth * 4, rows ? rows + q * 2 * w : nullptr);
+    }
 }
 
 // Plain 16-byte-vector device copy (grid-stride), the calibration kernel for

@@ -524,19 +524,23 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
     const uint64_t n = h->n, w = h->w;
     const unsigned logN = log2u(h->N);
     Scratch s;
-    uint64_t *dz, *scale, *partial, *vfd, *dout;
+    uint64_t *dz, *scale, *partial, *vfd, *dout = nullptr;
     // 64 rows per thread, fewer (down to 4) when the grid would have under 1024 blocks
     const uint64_t cgroups = (w + 255) / 256, RB = 256 / bary_cols(w);
     uint64_t rpb = 64 * RB;
     while (rpb > 4 * RB && ((n + rpb - 1) / rpb) * cgroups < 1024) rpb /= 2;
     const uint64_t chunks = (n + rpb - 1) / rpb;
-    TRYS(s.get(&dz, K * 24));
+    TRYS(s.get(&dz, 2 * K * 24));  // the points, then their vanishing factors
+    vfd = dz + 3 * K;
     TRYS(s.get(&scale, K * n * 24));
     TRYS(s.get(&partial, chunks * K * w * 24));
-    TRYS(s.get(&vfd, K * 24));
-    TRYS(s.get(&dout, K * w * 24));
+    const size_t obytes = K * w * 24;
+    const bool direct = obytes <= STAGE_RESULT;  // the combine kernel writes to mapped host memory
+    if (!direct) TRYS(s.get(&dout, obytes));
     // vanishing factors n^-1 * g^-n * (z_k^n - g^n) (trace.rs:900-905)
-    std::vector<uint64_t> vf(3 * K);
+    std::vector<uint64_t> zv(6 * K);
+    std::memcpy(zv.data(), z, K * 24);
+    uint64_t *vf = zv.data() + 3 * K;
     const uint64_t gn = pow(coset_offset, n), nig = mul(inv((uint64_t)n), inv(gn));
     for (size_t k = 0; k < K; k++) {
         fp3 zn = f3_pow(fp3{z[3 * k], z[3 * k + 1], z[3 * k + 2]}, n);
@@ -546,8 +550,8 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
         vf[3 * k + 2] = v.c2;
     }
     StageScope ss(st);
-    LVM_HIP(stage_upload(dz, z, K * 24, st));
-    LVM_HIP(stage_upload(vfd, vf.data(), K * 24, st));
+    LVM_HIP(stage_upload(dz, zv.data(), 2 * K * 24, st));
+    if (direct) LVM_HIP(stage_result(out, obytes, nullptr, 0, st, (void **)&dout, nullptr));
     {
         ProfScope ps("bary_denoms", st);
         // scale[k][p] = x_p / (z_k - x_p)
@@ -570,7 +574,7 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
                            (uint32_t)K, w, vfd, dout);
     }
     LVM_HIP(hipGetLastError());
-    LVM_HIP(stage_download(out, dout, K * w * 24, st));
+    if (!direct) LVM_HIP(stage_download(out, dout, obytes, st));
     LVM_HIP(stage_sync(st));
     return LVM_OK;
 }
@@ -662,10 +666,9 @@ int lvm_deep_composition(const lvm_lde *main, const lvm_lde *aux, const lvm_lde 
         times_w(&wh[9 * j + 3], &wh[9 * j + 6]);
     }
     Scratch s;
-    uint64_t *dpoles, *inv_den, *dargs;
-    TRYS(s.get(&dpoles, npoles * 24));
+    uint64_t *inv_den, *dargs;
     TRYS(s.get(&inv_den, (uint64_t)npoles * N * 24));
-    // consts, powers and weights in one upload
+    // poles, consts, powers and weights in one upload
     std::vector<uint64_t> blob;
     auto put = [&](const void *p, size_t bytes) {
         const size_t at = blob.size();
@@ -673,16 +676,15 @@ int lvm_deep_composition(const lvm_lde *main, const lvm_lde *aux, const lvm_lde 
         if (bytes) std::memcpy(&blob[at], p, bytes);
         return at;
     };
-    const size_t o_consts = put(consts.data(), (K + 1) * 24), o_rp = put(rp.data(), K * 24);
+    const size_t o_poles = put(poles.data(), npoles * 24), o_consts = put(consts.data(), (K + 1) * 24), o_rp = put(rp.data(), K * 24);
     const size_t o_wt = put(wt.data(), wt.size() * 8), o_wh = put(wh.data(), wh.size() * 8);
     TRYS(s.get(&dargs, blob.size() * 8));
     StageScope ss(st);
-    LVM_HIP(stage_upload(dpoles, poles.data(), npoles * 24, st));
     LVM_HIP(stage_upload(dargs, blob.data(), blob.size() * 8, st));
     {
         ProfScope ps("deep_denoms", st);
         // 1 / (x - z) (XMinusZ, crypto/math-cuda/src/inverse.rs:241-300)
-        launch_pole_inverse(inv_den, N, log2u(N), coset_offset, dpoles, npoles, 0, d->tb.fwd_lo, d->tb.fwd_hi, st);
+        launch_pole_inverse(inv_den, N, log2u(N), coset_offset, dargs + o_poles, npoles, 0, d->tb.fwd_lo, d->tb.fwd_hi, st);
     }
     {
         ProfScope ps("deep_rows", st);

@@ -19,7 +19,8 @@ struct TreeTop {
     CoopKeccak k;
     uint32_t *ws;
     uint32_t g, y, half;
-    __device__ __forceinline__ explicit TreeTop(TreeTopLds &s) {
+    uint64_t *root;  // nullable: where node 0 goes too
+    __device__ __forceinline__ TreeTop(TreeTopLds &s, uint64_t *root_out) : root(root_out) {
         ws = s.pi[threadIdx.x >> 6];
         coop_setup(k, ws);
         g = threadIdx.x >> 4;
@@ -38,6 +39,11 @@ struct TreeTop {
         for (int x = 0; x < 4; x++) {
             d[2 * x + half] = a[x];
             s.dig[buf][g][2 * x + half] = a[x];
+        }
+        if (node == 0 && root) {
+            gmem_u32 *r = (gmem_u32 *)root;
+#pragma unroll
+            for (int x = 0; x < 4; x++) r[2 * x + half] = a[x];
         }
     }
 };
