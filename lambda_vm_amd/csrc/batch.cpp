@@ -92,6 +92,22 @@ struct Writer {
 
 }  // namespace
 
+// leaf_top_span of the tables whose leaves are hashed one permutation per 16
+// lanes, 0 for the others: the tables of up to LEAF_TOP_LEAVES leaves, when those
+// have at most LEAF_TOP_BATCH together. Sixteen lanes do a permutation in under
+// half the time, at a third of the chip's rate, so the form is for leaves that
+// leave the chip mostly idle. Batches, this form against one leaf per lane: four
+// tables of 2^13 leaves 256 against 311 us, twenty of 2^10 rows 314 against 357;
+// sixteen of 2^11 to 2^13 rows 810 against 659.
+std::vector<uint32_t> lvm::leaf_top_spans(const std::vector<uint64_t> &leaves) {
+    uint64_t sum = 0;
+    for (uint64_t L : leaves) sum += L <= LEAF_TOP_LEAVES ? L : 0;
+    std::vector<uint32_t> span;
+    for (uint64_t L : leaves)
+        span.push_back(L <= LEAF_TOP_LEAVES && sum <= LEAF_TOP_BATCH ? leaf_top_span(L) : 0);
+    return span;
+}
+
 // Tree steps above C nodes (a power of two): wide levels one per
 // step while more than TREE_TOP_CHILDREN children remain, then tree tops.
 std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t C, uint32_t root) {
@@ -179,14 +195,17 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         }
     }
     // leaves
+    std::vector<uint64_t> leaves(T);
+    for (size_t t = 0; t < T; t++) leaves[t] = b->in[t].n * b->in[t].blowup / 2;
+    const std::vector<uint32_t> spans = leaf_top_spans(leaves);
     {
         std::vector<LeafJob> jobs;
         std::vector<uint32_t> prefix(1, 0);
         uint64_t total = 0;
         for (size_t t : b->order) {
             const lvm_table_desc &d = b->in[t];
-            const uint64_t L = d.n * d.blowup / 2;
-            const uint32_t span = L <= LEAF_TOP_LEAVES ? leaf_top_span(L) : 0;
+            const uint64_t L = leaves[t];
+            const uint32_t span = spans[t];
             jobs.push_back({b->lde[t], d.m, L, (uint64_t *)b->nodes[t], span, (uint32_t)t});
             total += span ? L / span : (L + TREE_WIDE_SPAN - 1) / TREE_WIDE_SPAN;
             if (total >= (1ull << 31)) return fail(LVM_ERR_ARG, "batched launch exceeds 2^31 blocks");
@@ -206,9 +225,7 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
         std::vector<std::vector<std::pair<TreeStep, uint32_t>>> st(T);
         size_t max_tree = 0;
         for (size_t t = 0; t < T; t++) {
-            const lvm_table_desc &d = b->in[t];
-            const uint64_t L = d.n * d.blowup / 2;
-            st[t] = tree_steps(b->nodes[t], L <= LEAF_TOP_LEAVES ? L / leaf_top_span(L) : L, (uint32_t)t);
+            st[t] = tree_steps(b->nodes[t], spans[t] ? leaves[t] / spans[t] : leaves[t], (uint32_t)t);
             max_tree = std::max(max_tree, st[t].size());
         }
         for (size_t s = 0; s < max_tree; s++) {

@@ -234,7 +234,9 @@ constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
 // Trees of at most this many leaves hash them one permutation per 16 lanes
 // too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch.
 constexpr uint64_t LEAF_TOP_LEAVES = 1u << 13;
+constexpr uint64_t LEAF_TOP_BATCH = 1u << 15;  // together, in one batched launch
 inline uint32_t leaf_top_span(uint64_t L) { return (uint32_t)(L < TREE_TOP_SPAN ? L : TREE_TOP_SPAN); }
+std::vector<uint32_t> leaf_top_spans(const std::vector<uint64_t> &leaves);  // per table of one launch (batch.cpp)
 // roots: 32-byte slots, written by the blocks that hash a root
 void launch_leaves_batched(const LeafJob *d_jobs, const uint32_t *d_prefix, uint32_t count, uint32_t blocks,
                            uint64_t *roots, hipStream_t st);
