@@ -12,6 +12,8 @@
 namespace lvm {
 void launch_gl_op(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, uint64_t n, bool ext3,
                   hipStream_t st);
+void launch_gather_bitrev_words(const uint64_t *src, uint64_t *dst, uint32_t log_rows, uint64_t w, uint64_t first,
+                                uint64_t count, hipStream_t st);
 void launch_gather_bitrev_rows(const uint64_t *src, uint64_t *dst, uint64_t rows, uint32_t log_rows, uint64_t w,
                                hipStream_t st);
 void launch_coset_weights(uint64_t n, uint64_t offset, uint64_t scale, uint64_t *out, hipStream_t st);
@@ -86,15 +88,25 @@ int check_lde_shape(size_t n, size_t w, size_t blowup) {
     return LVM_OK;
 }
 
+// The natural-order rows of a bit-reversed N x w table through the ring's slots;
+// the caller ends with ring.finish().
+hipError_t ring_download_natural(HostRing &ring, const uint64_t *lde, size_t N, size_t w, uint64_t *host_out,
+                                 hipStream_t st) {
+    return ring.download(host_out, N * w * 8, [=](void *slot, size_t off, size_t bytes) {
+        launch_gather_bitrev_words(lde, (uint64_t *)slot, log2u(N), w, off / 8, bytes / 8, st);
+    });
+}
+
 // LDE + commit from device-resident trace rows (n x w words) and weights.
 // Coset LDE of a device trace and its Merkle tree over the row-pair leaves of
 // columns [split, w) (all columns when split = 0). With split > 0 a second
 // tree over columns [0, split) is built too (a preprocessed table's fixed
 // columns): its root goes to pre_root_out and, when pre_nodes_host is set,
-// its node buffer to the host.
+// its node buffer to the host. With host_lde_out the natural-order rows leave
+// through `ring` ahead of the tree's kernels.
 int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blowup, const uint64_t *d_weights,
              lvm_lde **out, uint8_t root_out[32], size_t split = 0, uint8_t *pre_nodes_host = nullptr,
-             uint8_t *pre_root_out = nullptr) {
+             uint8_t *pre_root_out = nullptr, HostRing *ring = nullptr, uint64_t *host_lde_out = nullptr) {
     TRY(check_lde_shape(n, w, blowup));
     const size_t N = n * blowup;
     TRY(check_fault());
@@ -111,6 +123,7 @@ int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blow
         TRY(ntt_coset_expand(coef.as<uint64_t>(), (uint32_t)w, lde.as<uint64_t>(), (uint32_t)w, (uint32_t)w,
                              log2u(n), log2u(blowup), d_weights, d->tb, st));
     }
+    if (host_lde_out) LVM_HIP(ring_download_natural(*ring, lde.as<uint64_t>(), N, w, host_lde_out, st));
     uint8_t root[32], pre_root[32];
     {
         StageScope ss(st);
@@ -129,6 +142,7 @@ int lde_core(Device *d, const uint64_t *d_trace, size_t n, size_t w, size_t blow
             if (split) merkle_build_inner(pre.as<uint8_t>(), C, (uint64_t *)pr, st);
         }
         LVM_HIP(hipGetLastError());
+        if (host_lde_out) LVM_HIP(ring->finish());  // the last slots' host copies run beside the tree
         LVM_HIP(stage_sync(st));
         if (split && pre_root_out) std::memcpy(pre_root_out, pre_root, 32);
         if (split && pre_nodes_host) {
@@ -161,11 +175,18 @@ int lde_from_host(const uint64_t *trace, size_t n, size_t w, size_t blowup, cons
     DevBuf dt, dw;
     TRY(dt.alloc(n * w * 8, st));
     TRY(dw.alloc(n * 8, st));
-    LVM_HIP(hipMemcpyAsync(dt.p, trace, n * w * 8, hipMemcpyHostToDevice, st));
-    LVM_HIP(hipMemcpyAsync(dw.p, weights, n * 8, hipMemcpyHostToDevice, st));
+    HostRing ring(st);
+    if (ring.ready()) {
+        LVM_HIP(ring.upload(dt.as<uint64_t>(), trace, n * w));
+        LVM_HIP(ring.upload(dw.as<uint64_t>(), weights, n));
+    } else {
+        LVM_HIP(hipMemcpyAsync(dt.p, trace, n * w * 8, hipMemcpyHostToDevice, st));
+        LVM_HIP(hipMemcpyAsync(dw.p, weights, n * 8, hipMemcpyHostToDevice, st));
+    }
     lvm_lde *h = nullptr;
-    TRY(lde_core(d, dt.as<uint64_t>(), n, w, blowup, dw.as<uint64_t>(), &h, root_out));
-    if (host_lde_out) {
+    TRY(lde_core(d, dt.as<uint64_t>(), n, w, blowup, dw.as<uint64_t>(), &h, root_out, 0, nullptr, nullptr, &ring,
+                 ring.ready() ? host_lde_out : nullptr));
+    if (host_lde_out && !ring.ready()) {
         int rc = lvm_lde_download(h, host_lde_out);
         if (rc != LVM_OK) {
             lvm_lde_release(h);
@@ -428,6 +449,12 @@ int lvm_lde_download(const lvm_lde *h, uint64_t *host_out) {
     Device *d = dev_or_fail();
     if (!d) return LVM_ERR_DEVICE;
     hipStream_t st = thread_stream(d);
+    HostRing ring(st);
+    if (ring.ready()) {
+        LVM_HIP(ring_download_natural(ring, h->lde, h->N, h->w, host_out, st));
+        LVM_HIP(ring.finish());
+        return LVM_OK;
+    }
     DevBuf tmp;
     TRY(tmp.alloc(h->N * h->w * 8, st));
     launch_gather_bitrev_rows(h->lde, tmp.as<uint64_t>(), h->N, log2u(h->N), h->w, st);

@@ -4,6 +4,7 @@
 #include <atomic>
 #include <stdint.h>
 #include <stddef.h>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -93,6 +94,38 @@ hipError_t stage_sync(hipStream_t st);
 // one and the last of those kernels' launches (it could drain the area).
 constexpr size_t STAGE_RESULT = 64 << 10;
 hipError_t stage_result(void *dst_a, size_t bytes_a, void *dst_b, size_t bytes_b, hipStream_t st, void **a, void **b);
+// Transfers of whole tables between pageable host memory and the device, in
+// slots of a page-locked ring that the calling thread keeps: the host copies
+// one slot while the device moves another. The device side is a kernel that reads
+// or writes the slot itself (the memory is mapped): queuing a DMA copy costs the
+// host some 25 us a slot against 4 for a launch, and a download's rows are
+// reordered on their way out. download() queues every slot
+// and delivers all but the last ones; finish() delivers those, so what is
+// queued on the stream in between runs beside the host's copies. One ring
+// object per call and thread at a time. ready() is false when the ring cannot be
+// allocated: the caller then copies directly.
+constexpr size_t RING_SLOT = 512u << 10, RING_SLOTS = 8;
+class HostRing {
+  public:
+    explicit HostRing(hipStream_t st);
+    ~HostRing();
+    bool ready() const { return buf_ != nullptr; }
+    hipError_t upload(uint64_t *dst_dev, const uint64_t *src_host, size_t words);
+    // produce(slot, off, n): queue on the stream the kernel that writes bytes
+    // [off, off + n) of the result to `slot`
+    using Produce = std::function<void(void *slot, size_t off, size_t n)>;
+    hipError_t download(void *dst_host, size_t bytes, const Produce &produce);
+    hipError_t finish();
+
+  private:
+    hipError_t deliver_oldest();
+    hipStream_t st_;
+    uint8_t *buf_ = nullptr;
+    hipEvent_t ev_[RING_SLOTS] = {};
+    uint64_t head_ = 0, tail_ = 0;  // slots queued and slots whose event was waited for
+    uint8_t *dst_[RING_SLOTS] = {};  // where a slot's bytes go (nullptr: an upload)
+    size_t len_[RING_SLOTS] = {};
+};
 struct StageScope {
     explicit StageScope(hipStream_t st);
     ~StageScope();

@@ -48,22 +48,37 @@ void launch_gl_op(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, u
         hipLaunchKernelGGL(gl_op_kernel, grid, dim3(256), 0, st, op, a, b, out, n);
 }
 
-// dst natural row r <- src physical row bitrev(r) (rows of `w` words)
-__global__ void gather_bitrev_rows_kernel(const uint64_t *src, uint64_t *dst, uint64_t rows, uint32_t log_rows,
-                                          uint64_t w) {
-    uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= rows * w) return;
-    uint64_t r = idx / w, c = idx - r * w;
-    uint64_t pr = bitrev((uint32_t)r, log_rows);
+__global__ void copy_words_kernel(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, uint64_t count) {
+    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < count) dst[idx] = src[idx];
+}
+
+void launch_copy_words(const uint64_t *src, uint64_t *dst, uint64_t count, hipStream_t st) {
+    if (!count) return;
+    hipLaunchKernelGGL(copy_words_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, src, dst, count);
+}
+
+// Words [first, first + count) of the natural-order table (row r = physical row
+// bitrev(r), rows of `w` words) to dst[0, count).
+__global__ void gather_bitrev_rows_kernel(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
+                                          uint32_t log_rows, uint64_t w, uint64_t first, uint64_t count) {
+    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= count) return;
+    const uint64_t r = (first + idx) / w, c = first + idx - r * w;
+    const uint64_t pr = log_rows ? bitrev((uint32_t)r, log_rows) : 0;
     dst[idx] = src[pr * w + c];
+}
+
+void launch_gather_bitrev_words(const uint64_t *src, uint64_t *dst, uint32_t log_rows, uint64_t w, uint64_t first,
+                                uint64_t count, hipStream_t st) {
+    if (!count) return;
+    hipLaunchKernelGGL(gather_bitrev_rows_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, src, dst,
+                       log_rows, w, first, count);
 }
 
 void launch_gather_bitrev_rows(const uint64_t *src, uint64_t *dst, uint64_t rows, uint32_t log_rows, uint64_t w,
                                hipStream_t st) {
-    uint64_t total = rows * w;
-    if (!total) return;
-    hipLaunchKernelGGL(gather_bitrev_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, src,
-                       dst, rows, log_rows, w);
+    launch_gather_bitrev_words(src, dst, log_rows, w, 0, rows * w, st);
 }
 
 // Merkle authentication paths (sibling of each node from the leaf up,
