@@ -98,13 +98,14 @@ struct Writer {
 // half the time, at a third of the chip's rate, so the form is for leaves that
 // leave the chip mostly idle. Batches, this form against one leaf per lane: four
 // tables of 2^13 leaves 256 against 311 us, twenty of 2^10 rows 314 against 357;
-// sixteen of 2^11 to 2^13 rows 810 against 659.
+// sixteen of 2^11 to 2^13 rows 810 against 659. A table of one leaf always takes
+// the form: its leaf is its root, which no tree step would write out.
 std::vector<uint32_t> lvm::leaf_top_spans(const std::vector<uint64_t> &leaves) {
     uint64_t sum = 0;
     for (uint64_t L : leaves) sum += L <= LEAF_TOP_LEAVES ? L : 0;
     std::vector<uint32_t> span;
     for (uint64_t L : leaves)
-        span.push_back(L <= LEAF_TOP_LEAVES && sum <= LEAF_TOP_BATCH ? leaf_top_span(L) : 0);
+        span.push_back(L == 1 || (L <= LEAF_TOP_LEAVES && sum <= LEAF_TOP_BATCH) ? leaf_top_span(L) : 0);
     return span;
 }
 
