@@ -103,9 +103,10 @@ __global__ __launch_bounds__(256) void open_kernel(const uint64_t *__restrict__ 
 
 void launch_open(const uint64_t *nodes, uint64_t L, const uint64_t *lde, uint64_t w, const uint64_t *pos,
                  uint64_t count, uint32_t depth, uint64_t *paths, uint64_t *rows, hipStream_t st) {
-    // launches of at most 2^30 positions
-    for (uint64_t q = 0; q < count; q += 1u << 30) {
-        const uint64_t n = count - q < (1u << 30) ? count - q : 1u << 30;
+    // a grid holds fewer than 2^32 threads: launches of at most 2^23 positions
+    constexpr uint64_t MOST = 1u << 23;
+    for (uint64_t q = 0; q < count; q += MOST) {
+        const uint64_t n = count - q < MOST ? count - q : MOST;
         hipLaunchKernelGGL(open_kernel, dim3((unsigned)n), dim3(256), 0, st, nodes, L, lde, w, pos + q, depth,
                            paths + q * depth * 4, rows ? rows + q * 2 * w : nullptr);
     }

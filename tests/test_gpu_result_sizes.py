@@ -41,3 +41,15 @@ def test_fri_answers(gpu, count):
         ev, nodes = h.layer(i)
         assert np.array_equal(sym[i], ev[(iotas >> np.uint64(i)) ^ np.uint64(1)])
     h.close()
+
+
+def test_more_openings_than_a_grid_has_blocks(gpu):
+    """2^24 positions of a block of 256 threads are 2^32 threads, more than one
+    launch takes; a table of four leaves, every answer from its own rows and nodes."""
+    m, L, count = 1, 4, (1 << 24) + 5
+    h = gpu.coset_lde_dev(gpu.DeviceBuffer.from_array(workload.trace_table(53, m, L, m)), L, m, 2,
+                          gpu.coset_weights_dev(L, 7))
+    pos = np.random.default_rng(1).integers(0, L, count).astype(np.uint64)
+    want_paths, want_rows = h.open(np.arange(L, dtype=np.uint64))
+    paths, rows = h.open(pos)
+    assert np.array_equal(rows, want_rows[pos]) and np.array_equal(paths, want_paths[pos])
