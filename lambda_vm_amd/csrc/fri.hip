@@ -179,9 +179,9 @@ struct QueryLayer {
     uint32_t pad;
 };
 __global__ __launch_bounds__(128) void fri_query_kernel(const QueryLayer *__restrict__ layers,
-                                                        const uint64_t *__restrict__ iotas, uint64_t count,
-                                                        uint64_t *sym_out, uint64_t *paths_out) {
-    const uint64_t q = blockIdx.x;
+                                                        const uint64_t *__restrict__ iotas, uint64_t first,
+                                                        uint64_t count, uint64_t *sym_out, uint64_t *paths_out) {
+    const uint64_t q = first + blockIdx.x;
     const uint32_t li = blockIdx.y;
     const QueryLayer l = layers[li];
     const uint64_t idx = iotas[q] >> li, p = idx >> 1;
@@ -511,7 +511,6 @@ int lvm_fri_query(const lvm_fri *f, const uint64_t *iotas, size_t count, uint64_
     Device *d = device_state();
     if (!d) return LVM_ERR_DEVICE;
     hipStream_t st = thread_stream(d);
-    if (count >= (1u << 31)) return fail(LVM_ERR_ARG, "too many queries");
     // per layer: count sym evals (3 u64) and count paths (depth_l x 32 bytes);
     // the layers' descriptors and the indexes go up in one blob
     const size_t layers = f->layers.size();
@@ -544,9 +543,13 @@ int lvm_fri_query(const lvm_fri *f, const uint64_t *iotas, size_t count, uint64_
     LVM_HIP(stage_upload(dblob.p, blob.data(), blob.size() * 8, st));
     void *sym = dsym.p, *paths = dpaths.p;
     if (direct) LVM_HIP(stage_result(evals_sym_out, sbytes, paths_out, pbytes, st, &sym, &paths));
-    hipLaunchKernelGGL(fri_query_kernel, dim3((unsigned)count, (unsigned)layers), dim3(128), 0, st,
-                       (const QueryLayer *)dblob.p, dblob.p + layers * sizeof(QueryLayer) / 8, (uint64_t)count,
-                       (uint64_t *)sym, (uint64_t *)paths);
+    // a grid row holds fewer than 2^32 threads: launches of at most 2^24 queries
+    constexpr uint64_t MOST = 1u << 24;
+    for (uint64_t q = 0; q < count; q += MOST)
+        hipLaunchKernelGGL(fri_query_kernel, dim3((unsigned)(count - q < MOST ? count - q : MOST), (unsigned)layers),
+                           dim3(128), 0, st, (const QueryLayer *)dblob.p,
+                           dblob.p + layers * sizeof(QueryLayer) / 8, q, (uint64_t)count, (uint64_t *)sym,
+                           (uint64_t *)paths);
     LVM_HIP(hipGetLastError());
     if (!direct) {
         LVM_HIP(stage_download(evals_sym_out, dsym.p, sbytes, st));

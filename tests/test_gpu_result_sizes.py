@@ -53,3 +53,15 @@ def test_more_openings_than_a_grid_has_blocks(gpu):
     want_paths, want_rows = h.open(np.arange(L, dtype=np.uint64))
     paths, rows = h.open(pos)
     assert np.array_equal(rows, want_rows[pos]) and np.array_equal(paths, want_paths[pos])
+
+
+def test_more_queries_than_a_grid_has_blocks(gpu):
+    """2^25 queries of a block of 128 threads, on one committed layer of four values."""
+    h = gpu.GpuFri(np.random.default_rng(6).integers(0, workload.P, size=(8, 3), dtype=np.uint64), 7)
+    h.fold_and_commit_layer([3, 5, 7])
+    iotas = np.random.default_rng(2).integers(0, 4, (1 << 25) + 5).astype(np.uint64)
+    want_sym, want_paths = h.query(np.arange(4, dtype=np.uint64))
+    sym, paths = h.query(iotas)
+    assert len(paths) == 1 and np.array_equal(sym[0], want_sym[0][iotas])
+    assert np.array_equal(paths[0], want_paths[0][iotas])
+    h.close()
