@@ -175,18 +175,20 @@ int lde_from_host(const uint64_t *trace, size_t n, size_t w, size_t blowup, cons
     DevBuf dt, dw;
     TRY(dt.alloc(n * w * 8, st));
     TRY(dw.alloc(n * 8, st));
-    HostRing ring(st);
-    if (ring.ready()) {
-        LVM_HIP(ring.upload(dt.as<uint64_t>(), trace, n * w));
-        LVM_HIP(ring.upload(dw.as<uint64_t>(), weights, n));
-    } else {
-        LVM_HIP(hipMemcpyAsync(dt.p, trace, n * w * 8, hipMemcpyHostToDevice, st));
-        LVM_HIP(hipMemcpyAsync(dw.p, weights, n * 8, hipMemcpyHostToDevice, st));
-    }
+    const bool ring_out = host_lde_out && ring_takes_download(host_lde_out, n * blowup * w * 8);
+    const bool ring_trace = ring_takes_upload(trace), ring_weights = ring_takes_upload(weights);
+    HostRing ring(st, ring_out || ring_trace || ring_weights);
+    auto upload = [&](DevBuf &to, const uint64_t *from, size_t words, bool by_ring) {
+        return by_ring && ring.ready() ? ring.upload(to.as<uint64_t>(), from, words)
+                                       : hipMemcpyAsync(to.p, from, words * 8, hipMemcpyHostToDevice, st);
+    };
+    LVM_HIP(upload(dt, trace, n * w, ring_trace));
+    LVM_HIP(upload(dw, weights, n, ring_weights));
+    const bool beside_tree = ring_out && ring.ready();
     lvm_lde *h = nullptr;
     TRY(lde_core(d, dt.as<uint64_t>(), n, w, blowup, dw.as<uint64_t>(), &h, root_out, 0, nullptr, nullptr, &ring,
-                 ring.ready() ? host_lde_out : nullptr));
-    if (host_lde_out && !ring.ready()) {
+                 beside_tree ? host_lde_out : nullptr));
+    if (host_lde_out && !beside_tree) {
         int rc = lvm_lde_download(h, host_lde_out);
         if (rc != LVM_OK) {
             lvm_lde_release(h);
@@ -449,7 +451,7 @@ int lvm_lde_download(const lvm_lde *h, uint64_t *host_out) {
     Device *d = dev_or_fail();
     if (!d) return LVM_ERR_DEVICE;
     hipStream_t st = thread_stream(d);
-    HostRing ring(st);
+    HostRing ring(st, ring_takes_download(host_out, h->N * h->w * 8));
     if (ring.ready()) {
         LVM_HIP(ring_download_natural(ring, h->lde, h->N, h->w, host_out, st));
         LVM_HIP(ring.finish());

@@ -434,7 +434,24 @@ hipError_t stage_sync(hipStream_t st) {
 
 void launch_copy_words(const uint64_t *src, uint64_t *dst, uint64_t count, hipStream_t st);  // misc.hip
 
-HostRing::HostRing(hipStream_t st) : st_(st) {
+static hipMemoryType memory_type(const void *p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipMemoryTypeUnregistered;
+    }
+    return a.type;
+}
+
+bool ring_takes_upload(const void *src) { return memory_type(src) == hipMemoryTypeUnregistered; }
+
+bool ring_takes_download(const void *dst, size_t bytes) {
+    const hipMemoryType t = memory_type(dst);
+    return t == hipMemoryTypeUnregistered || (t == hipMemoryTypeHost && bytes <= RING_LOCKED_OUT);
+}
+
+HostRing::HostRing(hipStream_t st, bool wanted) : st_(st) {
+    if (!wanted) return;
     for (hipEvent_t &ev : ev_)
         if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
             ev = nullptr;
@@ -489,7 +506,10 @@ hipError_t HostRing::upload(uint64_t *dst_dev, const uint64_t *src_host, size_t 
         if (e != hipSuccess) return e;
         const size_t i = head_ % RING_SLOTS, n = std::min(W, words - off);
         std::memcpy(buf_ + i * RING_SLOT, src_host + off, n * 8);
-        launch_copy_words((const uint64_t *)(buf_ + i * RING_SLOT), dst_dev + off, n, st_);
+        {
+            ProfScope ps("host_ring_in", st_);
+            launch_copy_words((const uint64_t *)(buf_ + i * RING_SLOT), dst_dev + off, n, st_);
+        }
         dst_[i] = nullptr;
         head_++;  // counted before the event: the destructor waits for the kernel also when it fails
         e = hipGetLastError();
@@ -504,7 +524,10 @@ hipError_t HostRing::download(void *dst_host, size_t bytes, const Produce &produ
         hipError_t e = head_ - tail_ == RING_SLOTS ? deliver_oldest() : hipSuccess;
         if (e != hipSuccess) return e;
         const size_t i = head_ % RING_SLOTS, n = std::min(RING_SLOT, bytes - off);
-        produce(buf_ + i * RING_SLOT, off, n);
+        {
+            ProfScope ps("host_ring_out", st_);
+            produce(buf_ + i * RING_SLOT, off, n);
+        }
         dst_[i] = (uint8_t *)dst_host + off;
         len_[i] = n;
         head_++;
