@@ -176,7 +176,7 @@ int lde_from_host(const uint64_t *trace, size_t n, size_t w, size_t blowup, cons
     TRY(dt.alloc(n * w * 8, st));
     TRY(dw.alloc(n * 8, st));
     const bool ring_out = host_lde_out && ring_takes_download(host_lde_out, n * blowup * w * 8);
-    const bool ring_trace = ring_takes_upload(trace), ring_weights = ring_takes_upload(weights);
+    const bool ring_trace = ring_takes_upload(trace, n * w * 8), ring_weights = ring_takes_upload(weights, n * 8);
     HostRing ring(st, ring_out || ring_trace || ring_weights);
     auto upload = [&](DevBuf &to, const uint64_t *from, size_t words, bool by_ring) {
         return by_ring && ring.ready() ? ring.upload(to.as<uint64_t>(), from, words)

@@ -443,7 +443,9 @@ static hipMemoryType memory_type(const void *p) {
     return a.type;
 }
 
-bool ring_takes_upload(const void *src) { return memory_type(src) == hipMemoryTypeUnregistered; }
+bool ring_takes_upload(const void *src, size_t bytes) {
+    return bytes <= RING_MOST_IN && memory_type(src) == hipMemoryTypeUnregistered;
+}
 
 bool ring_takes_download(const void *dst, size_t bytes) {
     const hipMemoryType t = memory_type(dst);

@@ -112,9 +112,14 @@ hipError_t stage_result(void *dst_a, size_t bytes_a, void *dst_b, size_t bytes_b
 // directly; the 2 GiB LDE down 100 ms against 38.4. Only page-locked results of up
 // to RING_LOCKED_OUT come through it, as a copy's launch costs more than they
 // (16 KiB 16 us against 26, 512 KiB 35 against 40, 1 MiB 51 against 50, 2 MiB 111
-// against 69).
-bool ring_takes_upload(const void *src);
+// against 69). Pageable tables of more than RING_MOST_IN go up directly too: the
+// runtime pins large pageable memory in place, which beats one thread's copies
+// (commitments from 16 MiB 812 us against 780 through the ring, 32 MiB 1573 against
+// 1602, 128 MiB 5.4 ms against 6.3, 512 MiB 21.6 against 25.0). On the way down
+// the ring stays ahead at every size (1 GiB 56.7 ms against 60.5).
+bool ring_takes_upload(const void *src, size_t bytes);
 bool ring_takes_download(const void *dst, size_t bytes);
+constexpr size_t RING_MOST_IN = 32u << 20;
 constexpr size_t RING_LOCKED_OUT = 1u << 20;
 constexpr size_t RING_SLOT = 512u << 10, RING_SLOTS = 8;
 class HostRing {

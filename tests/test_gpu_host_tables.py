@@ -125,3 +125,16 @@ def test_small_page_locked_results(gpu):
         assert _ring_use(gpu, lambda: _native.call("lvm_lde_download", h.h, p)) == (0, slots)
         assert np.array_equal(x.a.reshape(n, m), h.download())
         x.free()
+
+
+@pytest.mark.parametrize("m,slots", [(32, 64), (33, 0)])  # 2^17 rows: 32 MiB, and past it
+def test_large_pageable_tables_go_up_directly(gpu, m, slots):
+    n = 1 << 17
+    tr = workload.trace_table_modp(37, m, n, m)
+    w = gpu.coset_weights_dev(n, 7)
+    want = gpu.coset_lde_dev(gpu.DeviceBuffer.from_array(tr), n, m, 1, w).root
+    hw = w.to_array(np.uint64, (n,))
+    p = [a.ctypes.data_as(_native.u64p) for a in (tr, hw)]
+    hs = []
+    used = _ring_use(gpu, lambda: hs.append(gpu.GpuLde(_commit(p[0], n, m, 1, p[1], None).value)))
+    assert used == (slots + 2, 0) and hs[0].root == want  # the weights are two slots
