@@ -7,7 +7,9 @@
 // x_p = g * w_N^bitrev_N(p). Its first n physical rows are the sub-coset
 // g*<w_n> the barycentric formula of crypto/stark/src/trace.rs:831-1110
 // reads (natural rows i*B), so those reads are contiguous here.
+#include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "lvm_internal.hpp"
@@ -176,34 +178,43 @@ static void launch_pole_inverse(uint64_t *out, uint64_t rows, uint32_t log_N, ui
 
 constexpr int BARY_MAX_K = 8;
 // partial[chunk][k][c] = sum over the chunk's rows p of lde[p][c] * scale[k][p]
-// block: 256 threads over min(w, 256) adjacent columns and as many rows RB at
-// once as fit (thread = row * columns + column, so a block's loads are runs of
-// whole rows and no lane idles on a narrow table: with 64 lanes a row, 17
-// columns used 17 of them); grid (chunks of rpb rows, groups of 256 columns).
-// The three components of each point's sum are delayed-reduction dot products
-// (one 128-bit accumulate per product, one reduction per thread), loads of U
-// rows issued together; the RB partial sums of a column meet in LDS.
-__host__ __device__ inline uint32_t bary_cols(uint64_t w) { return w < 256 ? (uint32_t)w : 256u; }
+// block: 256 threads over a group of gc adjacent columns and as many rows RB at
+// once as fit; grid (chunks of rpb rows, column groups). The three components
+// of each point's sum are delayed-reduction dot products (one 128-bit accumulate
+// per product, one reduction per thread), loads of U rows issued together; the
+// RB partial sums of a column meet in LDS. Two forms:
+//  - packed: thread = row * columns + column, so a block's loads are runs of whole
+//    rows and no lane idles on a narrow table (with 64 lanes a row, 17 columns
+//    used 17 of them); every lane loads its row's scales;
+//  - WAVE: a row per wave, 64 columns a group, the scales by scalar loads and as
+//    scalar operands: half the registers, one vector load a row instead of 1 + 3 K.
+// bary_shape says which, with both measured.
+constexpr int BARY_WAVE_MAX_K = 2;
 
-template <int K>
+template <int K, bool WAVE>
 __global__ __launch_bounds__(256) void bary_partial_kernel(const uint64_t *__restrict__ lde, uint64_t w, uint64_t n,
-                                                           uint64_t rpb, const uint64_t *__restrict__ scale,
+                                                           uint32_t gc, uint64_t rpb,
+                                                           const uint64_t *__restrict__ scale,
                                                            uint64_t *__restrict__ partial) {
     constexpr int U = K <= 2 ? 4 : 2;
     __shared__ uint64_t red[256][3];
     const uint32_t t = threadIdx.x;
-    const uint64_t c0 = (uint64_t)blockIdx.y * 256;
-    const uint32_t wc = bary_cols(w - c0), RB = 256 / wc;
-    const uint32_t r = t / wc, c = t - r * wc;
+    const uint64_t c0 = (uint64_t)blockIdx.y * gc;
+    const uint32_t have = w - c0 < gc ? (uint32_t)(w - c0) : gc;
+    const uint32_t wc = WAVE ? 64 : have, RB = 256 / wc;
+    const uint32_t r = WAVE ? __builtin_amdgcn_readfirstlane(t / 64) : t / wc, c = t - r * wc;
     const uint64_t p0 = (uint64_t)blockIdx.x * rpb, pend = p0 + rpb < n ? p0 + rpb : n;
     acc128 acc[K][3];
 #pragma unroll
     for (int k = 0; k < K; k++)
 #pragma unroll
         for (int j = 0; j < 3; j++) acc_zero(acc[k][j]);
-    if (r < RB) {
+    if (WAVE ? c < have : r < RB) {
         const gmem_u64 *f = LVM_GLOBAL_CONST(lde) + c0 + c;
-        const gmem_u64 *sc = LVM_GLOBAL_CONST(scale);
+        // scales of a wave's row in the constant address space (no kernel in flight
+        // writes them): a uniform address becomes a scalar load
+        using scale_u64 = std::conditional_t<WAVE, const __attribute__((address_space(4))) uint64_t, const gmem_u64>;
+        scale_u64 *sc = (scale_u64 *)scale;
         uint64_t p = p0 + r;
         for (; p + (U - 1) * RB < pend; p += U * RB) {
             uint64_t v[U], s[U][K][3];
@@ -222,7 +233,12 @@ __global__ __launch_bounds__(256) void bary_partial_kernel(const uint64_t *__res
 #pragma unroll
                 for (int k = 0; k < K; k++)
 #pragma unroll
-                    for (int j = 0; j < 3; j++) acc_mad(acc[k][j], s[u][k][j], v[u]);
+                    for (int j = 0; j < 3; j++) {
+                        if constexpr (WAVE)
+                            acc_mad_uniform(acc[k][j], s[u][k][j], v[u]);
+                        else
+                            acc_mad(acc[k][j], s[u][k][j], v[u]);
+                    }
         }
         for (; p < pend; p += RB) {
             const uint64_t v = f[p * w];
@@ -245,15 +261,54 @@ __global__ __launch_bounds__(256) void bary_partial_kernel(const uint64_t *__res
             }
             left = half;
         }
-        if (r == 0) st3(partial + 3 * (((uint64_t)blockIdx.x * K + k) * w + c0 + c), v);
+        if (r == 0 && c < have) st3(partial + 3 * (((uint64_t)blockIdx.x * K + k) * w + c0 + c), v);
         __syncthreads();  // the sums are rewritten for the next point
     }
 }
 
+struct BaryShape {
+    bool wave;
+    uint32_t gc;               // columns of a group
+    uint64_t cgroups, rpb, chunks;
+};
+
+// A table of 64 columns or more takes a row per wave for one point, and for two
+// where that leaves at most a quarter of the lanes idle (bary_sum of 2^20 rows,
+// packed form against this one, K = 1 and 2: 64 columns 174 against 127 us and 231
+// against 207; 65 columns 206 against 185 and 288 against 428; 100 columns 295
+// against 209 and 430 against 370; 129 columns 419 against 325 and 577 against
+// 616; 256 columns 604 against 400 and 858 against 673; 48 columns K = 2 188 against
+// 183). Three points run out of scalar registers (256 columns 1165 against 1293).
+// Packed groups are all of a row up to 128 columns, then equal groups of at most
+// 64, which leave few lanes over (one group of 200 used 200 of 256: K = 4 1827
+// against 1240). A chunk is 1024 rows (64 a thread when more than 16 fit side by
+// side), less when the grid would have under 1024 blocks: chunks of 64 rows of wide
+// tables made the partial sums 16 times as large (2^22 x 300 at eight points 3.8
+// GB) and were no faster.
+BaryShape bary_shape(uint64_t n, uint64_t w, size_t K) {
+    BaryShape b;
+    b.wave = w >= 64 && (K == 1 || (K == BARY_WAVE_MAX_K && 4 * w >= 3 * 64 * ((w + 63) / 64)));
+    b.cgroups = b.wave || w > 128 ? (w + 63) / 64 : 1;
+    b.gc = b.wave ? 64 : (uint32_t)((w + b.cgroups - 1) / b.cgroups);
+    const uint64_t RB = 256 / b.gc;
+    b.rpb = std::max<uint64_t>(1024, 64 * RB);
+    while (b.rpb > 4 * RB && ((n + b.rpb - 1) / b.rpb) * b.cgroups < 1024) b.rpb /= 2;
+    b.chunks = (n + b.rpb - 1) / b.rpb;
+    return b;
+}
+
 template <int K>
-static void launch_bary_partial(dim3 grid, hipStream_t st, const uint64_t *lde, uint64_t w, uint64_t n,
-                                uint64_t rpb, const uint64_t *scale, uint64_t *partial) {
-    hipLaunchKernelGGL(bary_partial_kernel<K>, grid, dim3(256), 0, st, lde, w, n, rpb, scale, partial);
+static void launch_bary_partial(const BaryShape &b, hipStream_t st, const uint64_t *lde, uint64_t w, uint64_t n,
+                                const uint64_t *scale, uint64_t *partial) {
+    const dim3 grid((unsigned)b.chunks, (unsigned)b.cgroups);
+    if constexpr (K <= BARY_WAVE_MAX_K) {
+        if (b.wave) {
+            hipLaunchKernelGGL((bary_partial_kernel<K, true>), grid, dim3(256), 0, st, lde, w, n, b.gc, b.rpb, scale,
+                               partial);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((bary_partial_kernel<K, false>), grid, dim3(256), 0, st, lde, w, n, b.gc, b.rpb, scale, partial);
 }
 
 // out[k][c] = vf[k] * sum over chunks of partial[chunk][k][c]; one block per
@@ -525,11 +580,8 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
     const unsigned logN = log2u(h->N);
     Scratch s;
     uint64_t *dz, *scale, *partial, *vfd, *dout = nullptr;
-    // 64 rows per thread, fewer (down to 4) when the grid would have under 1024 blocks
-    const uint64_t cgroups = (w + 255) / 256, RB = 256 / bary_cols(w);
-    uint64_t rpb = 64 * RB;
-    while (rpb > 4 * RB && ((n + rpb - 1) / rpb) * cgroups < 1024) rpb /= 2;
-    const uint64_t chunks = (n + rpb - 1) / rpb;
+    const BaryShape shape = bary_shape(n, w, K);
+    const uint64_t chunks = shape.chunks;
     TRYS(s.get(&dz, 2 * K * 24));  // the points, then their vanishing factors
     vfd = dz + 3 * K;
     TRYS(s.get(&scale, K * n * 24));
@@ -559,16 +611,15 @@ int lvm_barycentric_base_multi(const lvm_lde *h, uint64_t coset_offset, const ui
     }
     {
         ProfScope ps("bary_sum", st);
-        dim3 grid((unsigned)chunks, (unsigned)cgroups);
         switch (K) {
-        case 1: launch_bary_partial<1>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 2: launch_bary_partial<2>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 3: launch_bary_partial<3>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 4: launch_bary_partial<4>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 5: launch_bary_partial<5>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 6: launch_bary_partial<6>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        case 7: launch_bary_partial<7>(grid, st, h->lde, w, n, rpb, scale, partial); break;
-        default: launch_bary_partial<8>(grid, st, h->lde, w, n, rpb, scale, partial); break;
+        case 1: launch_bary_partial<1>(shape, st, h->lde, w, n, scale, partial); break;
+        case 2: launch_bary_partial<2>(shape, st, h->lde, w, n, scale, partial); break;
+        case 3: launch_bary_partial<3>(shape, st, h->lde, w, n, scale, partial); break;
+        case 4: launch_bary_partial<4>(shape, st, h->lde, w, n, scale, partial); break;
+        case 5: launch_bary_partial<5>(shape, st, h->lde, w, n, scale, partial); break;
+        case 6: launch_bary_partial<6>(shape, st, h->lde, w, n, scale, partial); break;
+        case 7: launch_bary_partial<7>(shape, st, h->lde, w, n, scale, partial); break;
+        default: launch_bary_partial<8>(shape, st, h->lde, w, n, scale, partial); break;
         }
         hipLaunchKernelGGL(bary_combine_kernel, dim3((unsigned)(K * w)), dim3(256), 0, st, partial, chunks,
                            (uint32_t)K, w, vfd, dout);

@@ -1,10 +1,12 @@
 """Barycentric sums and DEEP at the widths and row counts where the kernels
-split their work: column groups of 256 and 16, rows below a block, and trace
+split their work: column groups of 64 and 16, rows below a block, and trace
 terms with zero weights (pruned openings). Canonical values, exact."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from lambda_vm_amd import workload
+from lambda_vm_amd import _native, workload
 
 pytestmark = pytest.mark.gpu
 P = np.uint64(workload.P)
@@ -59,3 +61,31 @@ def test_deep_widths_and_zero_weights(gpu, ora, log_n, m, ma, np_, K, pruned):
     got = gpu.deep_composition(hm, g, zp, tood, gtr, aux=ha, parts=hp, **kw).to_array(np.uint64, (N, 3))
     ref = ora.deep_composition(lm, g, zp, tood, gtr, aux=la, parts=lp, **kw)
     assert np.array_equal(canon(got), canon(ref[bitrev_perm(N.bit_length() - 1)]))
+
+
+# one point of 64 columns, or two where few lanes idle, take one row per wave, the
+# others rows side by side: the edges of both and of their column groups, few rows
+# and several chunks
+@pytest.mark.parametrize("log_n,m,K", [(1, 64, 1), (12, 63, 1), (12, 64, 2), (12, 65, 1), (11, 64, 3), (10, 129, 2),
+                                       (9, 65, 2), (10, 96, 2), (10, 95, 2), (6, 129, 1),
+                                       (10, 129, 3), (10, 192, 8), (9, 193, 4), (11, 200, 1), (3, 1480, 2),
+                                       (16, 64, 2), (17, 17, 3)])
+def test_barycentric_groups(gpu, ora, log_n, m, K):
+    test_barycentric_widths(gpu, ora, log_n, m, K)
+
+
+def test_barycentric_scratch_is_small_beside_the_weights(gpu):
+    """Device memory of a call on a wide table: the row weights (24 K n bytes) and
+    partial sums that stay below them, by the pool's high-water mark."""
+    lib, n, m, K = _native.lib(), 1 << 18, 300, 8
+    h = gpu.coset_lde_dev(gpu.splitmix_table_dev(n, m, 7, 1), n, m, 1, gpu.coset_weights_dev(n, 7))
+    pool, v = C.c_void_p(), C.c_uint64(0)
+    assert lib.hipDeviceGetDefaultMemPool(C.byref(pool), 0) == 0
+    gpu.trim()
+    assert lib.hipMemPoolGetAttribute(pool, 7, C.byref(v)) == 0  # hipMemPoolAttrUsedMemCurrent
+    before = v.value
+    v = C.c_uint64(0)
+    assert lib.hipMemPoolSetAttribute(pool, 8, C.byref(v)) == 0  # hipMemPoolAttrUsedMemHigh
+    gpu.barycentric_base_multi(h, 7, workload.fp3_values(9, K))
+    assert lib.hipMemPoolGetAttribute(pool, 8, C.byref(v)) == 0
+    assert 24 * K * n <= v.value - before <= 2 * 24 * K * n
