@@ -92,14 +92,16 @@ struct Writer {
 
 }  // namespace
 
-// leaf_top_span of the tables whose leaves are hashed one permutation per 16
-// lanes, 0 for the others: the tables of up to LEAF_TOP_LEAVES leaves, when those
-// have at most LEAF_TOP_BATCH together. Sixteen lanes do a permutation in under
-// half the time, at a third of the chip's rate, so the form is for leaves that
-// leave the chip mostly idle. Batches, this form against one leaf per lane: four
-// tables of 2^13 leaves 256 against 311 us, twenty of 2^10 rows 314 against 357;
-// sixteen of 2^11 to 2^13 rows 810 against 659. A table of one leaf always takes
-// the form: its leaf is its root, which no tree step would write out.
+// leaf_top_span of the tables (or FRI layers) of one launch whose leaves are hashed
+// one permutation per 16 lanes, 0 for the others: those of up to LEAF_TOP_LEAVES
+// leaves, when they have at most LEAF_TOP_BATCH together. Sixteen lanes do a
+// permutation in under half the time, at a third of the chip's rate, so the form is
+// for leaves that leave the chip mostly idle. Batches, this form against one leaf
+// per lane: four tables of 2^13 leaves 256 against 311 us, twenty of 2^10 rows 314
+// against 357; sixteen of 2^11 to 2^13 rows 810 against 659. FRI folds with their
+// tree steps, sixteen codewords of 2^15 points 853 against 659 us, 64 of them 2086
+// against 923. A table of one leaf always takes the form: its leaf is its root,
+// which no tree step would write out.
 std::vector<uint32_t> lvm::leaf_top_spans(const std::vector<uint64_t> &leaves) {
     uint64_t sum = 0;
     for (uint64_t L : leaves) sum += L <= LEAF_TOP_LEAVES ? L : 0;
@@ -109,24 +111,34 @@ std::vector<uint32_t> lvm::leaf_top_spans(const std::vector<uint64_t> &leaves) {
     return span;
 }
 
-// Tree steps above C nodes (a power of two): wide levels one per
-// step while more than TREE_TOP_CHILDREN children remain, then tree tops.
-std::vector<std::pair<TreeStep, uint32_t>> lvm::tree_steps(uint8_t *nodes_b, uint64_t C, uint32_t root) {
-    std::vector<std::pair<TreeStep, uint32_t>> out;  // (step, blocks)
-    uint64_t *nodes = (uint64_t *)nodes_b;
-    while (C > TREE_TOP_CHILDREN) {
-        TreeStep s{nodes, C - 1, C / 2 - 1, TREE_WIDE_SPAN, 1, root, 0};
-        out.push_back({s, (uint32_t)(C / (2 * TREE_WIDE_SPAN))});
-        C /= 2;
+// A launch takes one level of every tree of more than TREE_TOP_CHILDREN nodes, and
+// the top of the smaller ones when those have at most TREE_TOP_BATCH nodes
+// together: sixteen lanes a permutation pays while the chip is mostly idle (see
+// leaf_top_spans), however the nodes are spread over trees. Above that every tree
+// of more than one block's worth has one level hashed, a node per lane. Tree steps
+// of a batch at budgets of 2^14, 2^15, 2^16 and 2^17: sixteen tables of 2^14 leaves
+// 171, 165, 177 and 211 us (tops of every tree in one launch whatever their number:
+// 292), 64 of 2^14 352, 351, 355 and 389 (907), 512 of 2^10 210, 210, 232 and 268
+// (512), four of 2^14 120, 115, 127 and 125 (127).
+std::vector<std::vector<std::pair<TreeStep, uint32_t>>> lvm::tree_steps(std::vector<TreeAt> trees) {
+    std::vector<std::vector<std::pair<TreeStep, uint32_t>>> out;
+    while (true) {
+        uint64_t sum = 0;
+        for (const TreeAt &t : trees) sum += t.C > 1 && t.C <= TREE_TOP_CHILDREN ? t.C : 0;
+        std::vector<std::pair<TreeStep, uint32_t>> launch;
+        for (TreeAt &t : trees) {
+            if (t.C <= 1) continue;
+            const uint64_t parents = t.C / 2;
+            const bool wide = t.C > TREE_TOP_CHILDREN || (sum > TREE_TOP_BATCH && parents > TREE_TOP_SPAN);
+            const uint32_t span = wide ? TREE_WIDE_SPAN : (uint32_t)std::min<uint64_t>(parents, TREE_TOP_SPAN);
+            const uint64_t blocks = (parents + span - 1) / span;
+            launch.push_back({TreeStep{(uint64_t *)t.nodes, t.C - 1, parents - 1, span, (uint32_t)parents, t.root, 0},
+                              (uint32_t)blocks});
+            t.C = wide ? parents : blocks;
+        }
+        if (launch.empty()) return out;
+        out.push_back(launch);
     }
-    while (C > 1) {
-        const uint32_t span = (uint32_t)(C / 2 < TREE_TOP_SPAN ? C / 2 : TREE_TOP_SPAN);
-        const uint64_t blocks = C / (2 * span);
-        TreeStep s{nodes, C - 1, C / 2 - 1, span, 32, root, 0};
-        out.push_back({s, (uint32_t)blocks});
-        C = blocks;
-    }
-    return out;
 }
 
 namespace {
@@ -223,27 +235,23 @@ int layout(lvm_batch *b, Writer &w, bool record, const Tables &tb) {
     }
     // tree steps
     {
-        std::vector<std::vector<std::pair<TreeStep, uint32_t>>> st(T);
-        size_t max_tree = 0;
-        for (size_t t = 0; t < T; t++) {
-            st[t] = tree_steps(b->nodes[t], spans[t] ? leaves[t] / spans[t] : leaves[t], (uint32_t)t);
-            max_tree = std::max(max_tree, st[t].size());
-        }
-        for (size_t s = 0; s < max_tree; s++) {
+        std::vector<TreeAt> trees;
+        for (size_t t : b->order)
+            trees.push_back({b->nodes[t], spans[t] ? leaves[t] / spans[t] : leaves[t], (uint32_t)t});
+        const auto st = tree_steps(trees);
+        for (size_t s = 0; s < st.size(); s++) {
             std::vector<TreeStep> steps;
             std::vector<uint32_t> prefix(1, 0);
             uint64_t total = 0;
             double bytes = 0;
-            for (size_t t : b->order) {
-                if (s >= st[t].size()) continue;
-                const TreeStep &ts = st[t][s].first;
+            for (const auto &step : st[s]) {
+                const TreeStep &ts = step.first;
                 steps.push_back(ts);
-                total += st[t][s].second;
+                total += step.second;
                 prefix.push_back((uint32_t)total);
-                // parents built: span per block at the first level, halving per further level
-                uint64_t parents = ts.span, cnt = ts.span;
-                for (uint32_t lv = 1; lv < ts.levels && cnt > 1; lv++) parents += (cnt /= 2);
-                bytes += 96.0 * parents * st[t][s].second;
+                // parents built: the first level's, and a top's levels up to one node per block
+                const double parents = ts.span > TREE_TOP_SPAN ? ts.parents : 2.0 * ts.parents - step.second;
+                bytes += 96.0 * parents;
             }
             const size_t so = w.put(steps.data(), steps.size());
             const size_t po = w.put(prefix.data(), prefix.size());

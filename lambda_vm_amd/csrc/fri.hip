@@ -217,9 +217,6 @@ namespace {
 bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
 unsigned log2u(uint64_t x) { return (unsigned)__builtin_ctzll(x); }
 
-// leaves per block of a committed layer's fold (FoldJob::span)
-uint32_t fold_span(uint64_t L) { return L <= LEAF_TOP_LEAVES ? leaf_top_span(L) : 0; }
-
 void free_fri(lvm_fri *f) {
     if (f->cur && f->cur_owned) lvm_free(f->cur);
     for (auto &l : f->layers) {
@@ -285,7 +282,7 @@ static int fri_fold_impl(lvm_fri *f, const uint64_t zeta[3], bool commit, uint8_
     }
     const uint64_t ginv = inv(f->offset);
     const uint32_t log_half = log2u(half);
-    const uint32_t span = commit ? fold_span(layer.L) : 0;
+    const uint32_t span = commit ? leaf_top_spans({layer.L})[0] : 0;
     StageScope ss(st);
     void *root = nullptr;
     hipError_t e = commit ? stage_result(layer.root, 32, nullptr, 0, st, &root, nullptr) : hipSuccess;
@@ -358,8 +355,10 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
     std::vector<FoldJob> jobs(count);
     std::vector<uint32_t> prefix(1, 0);
     uint64_t total = 0;
-    std::vector<std::vector<std::pair<TreeStep, uint32_t>>> tsteps(count);
-    size_t max_steps = 0;
+    std::vector<uint64_t> leaves(count, 0);
+    for (size_t t = 0; commit && t < count; t++) leaves[t] = padded_leaves(fs[t]->len / 4);
+    const std::vector<uint32_t> spans = leaf_top_spans(leaves);
+    std::vector<TreeAt> trees;
     for (size_t t = 0; t < count; t++) {
         lvm_fri *f = fs[t];
         const uint64_t half = f->len / 2;
@@ -368,18 +367,15 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
             return fail(LVM_ERR_NOMEM, "FRI layer allocation failed");
         }
         if (commit) {
-            layers[t].L = padded_leaves(half / 2);
+            layers[t].L = leaves[t];
             if (lvm_malloc(&layers[t].nodes, (2 * layers[t].L - 1) * 32) != hipSuccess) {
                 release();
                 return fail(LVM_ERR_NOMEM, "FRI tree allocation failed");
             }
-            const uint32_t span = fold_span(layers[t].L);
-            tsteps[t] = tree_steps(layers[t].nodes, span ? layers[t].L / span : layers[t].L, (uint32_t)t);
-            max_steps = std::max(max_steps, tsteps[t].size());
+            trees.push_back({layers[t].nodes, spans[t] ? leaves[t] / spans[t] : leaves[t], (uint32_t)t});
         }
         jobs[t] = FoldJob{f->cur, outs[t], (uint64_t *)layers[t].nodes, half, zetas[3 * t], zetas[3 * t + 1],
-                          zetas[3 * t + 2], inv(f->offset), log2u(half), commit ? fold_span(layers[t].L) : 0,
-                          (uint32_t)t, 0};
+                          zetas[3 * t + 2], inv(f->offset), log2u(half), commit ? spans[t] : 0, (uint32_t)t, 0};
         total += fold_blocks(jobs[t]);
         if (total >= (1ull << 31)) {
             release();
@@ -401,14 +397,13 @@ int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool
         uint32_t count, blocks;
     };
     std::vector<StepLaunch> steps_l;
-    for (size_t s = 0; s < max_steps; s++) {
+    for (const auto &launch : tree_steps(trees)) {
         std::vector<TreeStep> steps;
         std::vector<uint32_t> sp(1, 0);
         uint64_t sb = 0;
-        for (size_t t = 0; t < count; t++) {
-            if (s >= tsteps[t].size()) continue;
-            steps.push_back(tsteps[t][s].first);
-            sb += tsteps[t][s].second;
+        for (const auto &step : launch) {
+            steps.push_back(step.first);
+            sb += step.second;
             sp.push_back((uint32_t)sb);
         }
         steps_l.push_back({put(steps.data(), steps.size() * sizeof(TreeStep)), put(sp.data(), sp.size() * 4),

@@ -271,7 +271,7 @@ struct TreeStep {
     uint64_t *nodes;
     uint64_t cstart, pstart;  // first child / first parent index of the level
     uint32_t span;            // parents per block at the first level
-    uint32_t levels;          // levels this step builds
+    uint32_t parents;         // parents of the first level
     uint32_t root;            // the tree's slot in the launch's root array
     uint32_t pad;
 };
@@ -280,6 +280,7 @@ struct TreeStep {
 // levels, one permutation per 16 lanes (merkle.hip).
 constexpr uint64_t TREE_TOP_CHILDREN = 1u << 14;
 constexpr uint32_t TREE_TOP_SPAN = 32;
+constexpr uint64_t TREE_TOP_BATCH = 1u << 15;  // children of the tops of one batched launch, together
 constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
 // Trees of at most this many leaves hash them one permutation per 16 lanes
 // too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch.
@@ -295,8 +296,14 @@ void launch_tree_steps_batched(const TreeStep *d_steps, const uint32_t *d_prefix
 // One FRI fold of each of count codewords in shared launches (fri.hip);
 // zetas: count x 3; roots_out (count x 32) when committing.
 int fri_fold_batch(lvm_fri *const *fs, size_t count, const uint64_t *zetas, bool commit, uint8_t *roots_out);
-// the launches above the C nodes (a power of two) at [C-1, 2C-1) of a tree: (step, blocks)
-std::vector<std::pair<TreeStep, uint32_t>> tree_steps(uint8_t *nodes, uint64_t C, uint32_t root);
+// What is left of a tree: the levels above its C nodes (a power of two) at [C-1, 2C-1).
+struct TreeAt {
+    uint8_t *nodes;
+    uint64_t C;
+    uint32_t root;  // the tree's slot in the launch's root array
+};
+// The launches that build several trees: for each, its steps (in the trees' order) and their blocks.
+std::vector<std::vector<std::pair<TreeStep, uint32_t>>> tree_steps(std::vector<TreeAt> trees);
 
 // Constraint programs (compose.hip interpreter, compose_jit.cpp compiled form).
 struct CompArgs;

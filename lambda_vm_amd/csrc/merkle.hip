@@ -206,9 +206,10 @@ __global__ __launch_bounds__(TREE_THREADS) void merkle_steps_batched_kernel(cons
     const uint32_t b = blockIdx.x;
     const uint32_t t = find_slot(prefix, count, b);
     const TreeStep s = steps[t];
-    if (s.span > TREE_TOP_SPAN)
-        merkle_parent(s.nodes, s.pstart + (uint64_t)s.span * (b - prefix[t]) + threadIdx.x);
-    else
+    if (s.span > TREE_TOP_SPAN) {
+        const uint32_t i = s.span * (b - prefix[t]) + threadIdx.x;
+        if (i < s.parents) merkle_parent(s.nodes, s.pstart + i);
+    } else
         merkle_top_body(s.nodes, s.cstart, s.pstart, s.span, b - prefix[t], roots + 4 * s.root);
 }
 

@@ -46,3 +46,42 @@ def test_one_leaf_tables(gpu, shapes):
     assert roots == want
     for h, root in zip(handles, roots):
         assert h.nodes()[0].tobytes() == root and h.root == root
+
+
+# blocks of each tree launch: 512 parents of a level each while the small trees
+# have more than 2^15 nodes together, then tops of 32 parents and their levels
+@pytest.mark.parametrize("count,rows,blocks", [(64, 8192, [512, 256, 128, 64, 512, 64]),
+                                               (16, 16384, [256, 128, 64, 512, 16]),
+                                               (5, 8192, [40, 320, 5]), (512, 1024, [512, 512, 512, 512, 512]),
+                                               (4, 8192, [16, 4]), (2, 16384, [512, 8, 2])])
+def test_tree_launches_of_many_trees(gpu, count, rows, blocks):
+    w = gpu.coset_weights_dev(rows, 7)
+    tables = [(gpu.splitmix_table_dev(rows, 1, 7, t), w, rows, 1, 2) for t in range(count)]
+    plan = gpu.BatchPlan(tables, use_graph=True)
+    got = [b for name, _, b in plan.launches() if name.startswith("batch_merkle")]
+    assert got == blocks, got
+    roots = plan.run()
+    for t in sorted({0, 1, count - 1}):
+        h = gpu.coset_lde_dev(tables[t][0], rows, 1, 2, w)
+        assert roots[t] == h.root and np.array_equal(plan.take(t).nodes(), h.nodes())
+    plan.close()
+
+
+# log2 points of the codewords: first layers of 2^13 leaves past the sum, with small
+# ones beside them; layers of one leaf; one below and at the sum
+@pytest.mark.parametrize("logs", [[15] * 5 + [4, 3], [15] * 4, [13] * 17 + [16], [10] * 40 + [14, 5], [4] * 3])
+def test_fri_layers_of_many_codewords(gpu, logs):
+    evs = [np.random.default_rng(100 * t + L).integers(0, workload.P, size=(1 << L, 3), dtype=np.uint64)
+           for t, L in enumerate(logs)]
+    fris = [gpu.GpuFri(e, 7) for e in evs]
+    ts = [gpu.Transcript(b"%d" % t) for t in range(len(logs))]
+    got = gpu.fri_commit_phase_batch(fris, ts, [1] * len(logs), 1)
+    for t, e in enumerate(evs):
+        f, tr = gpu.GpuFri(e, 7), gpu.Transcript(b"%d" % t)
+        roots, coeffs = f.commit_phase(tr, 1, 1)
+        assert np.array_equal(got[t][0], roots) and np.array_equal(got[t][1], coeffs) and ts[t].state() == tr.state()
+        for i in range(f.num_layers()):
+            a, b = fris[t].layer(i), f.layer(i)
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+        f.close()
+        fris[t].close()
