@@ -367,25 +367,27 @@ struct DeepArgs {
 // through LDS with coalesced row-segment loads (the next chunk's loads are
 // issued before the current chunk is accumulated); each thread accumulates
 // its row's sum_j gt_{j,k} * t_j[p] as 3*KA delayed-reduction dot products.
-// The weights are the same for every row: scalar loads and scalar operands.
-// A zero weight is skipped (a bus table opens one column at its next row, so
-// all its other weights of k = 1 are zero). KA < K when the trace-term weights
-// are geometric in k past the first KA - 1 points (gt_{j,k} = gt_{j,KA-1} *
-// r^(k-KA+1) for every column j, which the reference's weights are: gamma^(W +
-// j(K-1) + k - 1) for k >= 1, crypto/stark/src/prover.rs:2400-2460): then
-// sum_j gt_{j,k} t_j = r^(k-KA+1) * sum_j gt_{j,KA-1} t_j, and rpow[k] holds
-// r^(k-KA+1).
-template <int K, int KA>
+// The weights are the same for every row: scalar loads and scalar operands, a
+// zero weight skipped (a bus table opens one column at its next row, so all its
+// other weights of k = 1 are zero), or, LW, beside the columns in LDS
+// (launch_deep). KA < K when the trace-term weights are geometric in k past the
+// first KA - 1 points (gt_{j,k} = gt_{j,KA-1} * r^(k-KA+1) for every column j,
+// which the reference's weights are: gamma^(W + j(K-1) + k - 1) for k >= 1,
+// crypto/stark/src/prover.rs:2400-2460): then sum_j gt_{j,k} t_j = r^(k-KA+1) *
+// sum_j gt_{j,KA-1} t_j, and rpow[k] holds r^(k-KA+1).
+template <int K, int KA, bool LW>
 __global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
     __shared__ uint64_t tile[256][DEEP_CHUNK + 1];
-    const int t = threadIdx.x;
+    __shared__ uint64_t sw[LW ? DEEP_CHUNK * 3 * KA : 1];
+    const uint32_t t = threadIdx.x;
     const uint64_t N = a.N, r0 = (uint64_t)blockIdx.x * 256, p = r0 + t;
-    uint64_t nv[DEEP_CHUNK];
+    uint64_t nv[DEEP_CHUNK], nw = 0;
     // columns [j0, j0 + cw) of the block's rows: thread t loads column t % 16 of
     // rows t / 16, t / 16 + 16, ... (16 lanes per row segment)
     const uint32_t lc = t & 15, lr = t >> 4;
     const uint32_t rows = N - r0 < 256 ? (uint32_t)(N - r0) : 256u;  // a power of two
-    auto fetch = [&](const DeepSegment &s, uint32_t j0, uint32_t cw) {
+    auto fetch = [&](const DeepSegment &s, uint32_t j0, uint32_t cw, const uint64_t *w, uint32_t words) {
+        if (LW) nw = t < cw * words ? LVM_GLOBAL_CONST(w)[t] : 0;  // columns past the chunk weigh nothing
         if (lc >= cw || lr >= rows) return;
         const gmem_u64 *src = LVM_GLOBAL_CONST(s.rows) + (r0 + lr) * s.cols + j0 + lc;
         const uint64_t step = 16 * s.cols;
@@ -402,12 +404,28 @@ __global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < 16; q++) tile[lr + 16 * q][lc] = nv[q];
+        if (LW && t < DEEP_CHUNK * 3 * KA) sw[t] = nw;
         __syncthreads();
     };
     // acc[k] += w_k * (the thread's value) over the chunk's columns; a column's
-    // weights are loaded while the previous one is accumulated
+    // scalar weights are loaded while the previous one is accumulated
     auto accumulate = [&](auto &acc, const uint64_t *w, uint32_t cw) {
         constexpr int NK = sizeof(acc) / sizeof(acc[0]);
+        if constexpr (LW) {
+            // eight columns' LDS reads together (2^12 x 600, one sum: 78 us, four 93)
+            for (uint32_t c0 = 0; c0 < cw; c0 += 8) {
+#pragma unroll
+                for (uint32_t cc = c0; cc < c0 + 8; cc++) {
+                    const uint64_t v = tile[t][cc];
+                    const uint64_t *g = sw + 3 * NK * cc;
+#pragma unroll
+                    for (int k = 0; k < NK; k++)
+#pragma unroll
+                        for (int j = 0; j < 3; j++) acc_mad(acc[k][j], g[3 * k + j], v);
+                }
+            }
+            return;
+        }
         uint64_t g[3 * NK];
 #pragma unroll
         for (int i = 0; i < 3 * NK; i++) g[i] = w[i];
@@ -443,12 +461,12 @@ __global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
         const DeepSegment s = a.trace[sgi];
         const uint32_t cols = (uint32_t)s.cols, cm = width(cols);
         if (!cols) continue;
-        fetch(s, 0, cm);
+        fetch(s, 0, cm, w, 3 * KA);
         for (uint32_t j0 = 0; j0 < cols; j0 += cm) {
             const uint32_t cw = cols - j0 < cm ? cols - j0 : cm;
             stage();
             const uint32_t next = j0 + cm;
-            if (next < cols) fetch(s, next, cols - next < cm ? cols - next : cm);
+            if (next < cols) fetch(s, next, cols - next < cm ? cols - next : cm, w + (uint64_t)cw * 3 * KA, 3 * KA);
             accumulate(acc, w, cw);
             w += (uint64_t)cw * 3 * KA;
         }
@@ -471,7 +489,7 @@ __global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
         for (int j = 0; j < 3; j++) acc_zero(ha[0][j]);
         for (uint32_t j0 = 0; j0 < cols; j0 += cm) {
             const uint32_t cw = cols - j0 < cm ? cols - j0 : cm;
-            fetch(a.parts, j0, cw);
+            fetch(a.parts, j0, cw, a.gh + 3 * j0, 3);
             stage();
             accumulate(ha, a.gh + 3 * j0, cw);
         }
@@ -483,9 +501,27 @@ __global__ __launch_bounds__(256) void deep_kernel(DeepArgs a) {
     if (p < N) st3(a.out + 3 * p, r);
 }
 
+// Where the weights come from. Scalar loads with scalar operands win where several
+// blocks a CU hide their latency, one trip to the L2 per column, and above all
+// where weights are zero; with fewer blocks, and where the weights outgrow the scalar
+// cache, the chunk's weights through LDS do. deep_rows, scalar against LDS: two
+// sums of 2^20 x 200 471 against 488 us (one weight in two zero 394 against 479), of
+// 2^18 x 600 366 against 358 (304 against 349), but of 2^17 x 600 279 against 200,
+// 2^14 x 64 44 against 24, 2^12 x 1480 731 against 295. One sum and four are never
+// better off scalar (2^20 x 64 172 against 162 and 401 against 364); three (weights
+// that are not geometric) are from 2^20 rows on with weights that fit the 16 KiB
+// cache (64 columns 284 against 304, 200 columns 644 against 651, 400 columns 1446
+// against 1166; 2^18 x 200 216 against 177).
 template <int K, int KA>
 static void launch_deep(hipStream_t st, const DeepArgs &a) {
-    hipLaunchKernelGGL((deep_kernel<K, KA>), dim3((unsigned)((a.N + 255) / 256)), dim3(256), 0, st, a);
+    const uint64_t blocks = (a.N + 255) / 256, weights = 24 * KA * (a.trace[0].cols + a.trace[1].cols);
+    if constexpr (KA == 2 || KA == 3) {
+        if (KA == 2 ? blocks >= 1024 : blocks >= 4096 && weights <= (16u << 10)) {
+            hipLaunchKernelGGL((deep_kernel<K, KA, false>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((deep_kernel<K, KA, true>), dim3((unsigned)blocks), dim3(256), 0, st, a);
 }
 }  // namespace lvm
 

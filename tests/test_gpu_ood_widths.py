@@ -38,6 +38,20 @@ def test_barycentric_widths(gpu, ora, log_n, m, K):
                                                      (7, 48, 5, 2, 3, False), (8, 4, 22, 1, 2, True),
                                                      (4, 15, 0, 6, 4, False), (9, 120, 2, 2, 2, True)])
 def test_deep_widths_and_zero_weights(gpu, ora, log_n, m, ma, np_, K, pruned):
+    _deep_matches(gpu, ora, log_n, m, ma, np_, K, "pruned" if pruned else "")
+
+
+# weights by scalar loads: two sums from 2^18 rows on, three from 2^20 with up to 227
+# columns; a geometric case has two
+@pytest.mark.parametrize("log_n,m,ma,np_,K,kind", [(17, 17, 2, 1, 2, "pruned"), (17, 3, 0, 0, 2, ""),
+                                                   (17, 5, 1, 2, 3, "geometric"), (16, 5, 1, 2, 4, "geometric"),
+                                                   (17, 6, 1, 0, 4, "geometric"), (19, 3, 1, 1, 3, ""),
+                                                   (18, 3, 1, 1, 3, ""), (17, 2, 0, 1, 1, ""), (17, 2, 0, 1, 4, "")])
+def test_deep_weights_scalar_and_in_lds(gpu, ora, log_n, m, ma, np_, K, kind):
+    _deep_matches(gpu, ora, log_n, m, ma, np_, K, kind)
+
+
+def _deep_matches(gpu, ora, log_n, m, ma, np_, K, kind):
     n, blowup, g = 1 << log_n, 2, 3
     N = n * blowup
     w = ora.lde_weights(n, g)
@@ -52,8 +66,12 @@ def test_deep_widths_and_zero_weights(gpu, ora, log_n, m, ma, np_, K, pruned):
     cols = m + ma
     zp, tood = workload.fp3_values(55, K), workload.fp3_values(56, cols * K)
     gtr = workload.fp3_values(57, cols * K).reshape(cols, K, 3)
-    if pruned:  # only the last column opens at the next rows, as a bus table's
+    if kind == "pruned":  # only the last column opens at the next rows, as a bus table's
         gtr[:-1, 1:] = 0
+    if kind == "geometric":  # gamma^(cols + j(K-1) + k-1), as the transcript's
+        powers = gpu.fp3_powers(workload.fp3_values(61, 1)[0], cols * K)
+        gtr[:, 0] = powers[:cols]
+        gtr[:, 1:] = powers[cols:].reshape(cols, K - 1, 3)
     gtr = gtr.reshape(-1, 3)
     kw = dict(z_parts=workload.fp3_values(58, 1)[0] if np_ else None,
               parts_ood=workload.fp3_values(59, np_) if np_ else None,
