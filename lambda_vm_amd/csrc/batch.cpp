@@ -552,7 +552,7 @@ int lvm_set_ntt_plan(unsigned log_n, const int *radices, int count) {
 int lvm_get_ntt_plan(unsigned log_n, int *radices_out, int *count_out) {
     if (!radices_out || !count_out) return fail(LVM_ERR_ARG, "null output");
     if (log_n < 1 || log_n > 32) return fail(LVM_ERR_ARG, "log_n out of range");
-    *count_out = plan_passes(log_n, radices_out);
+    *count_out = plan_passes(log_n, 0, radices_out);
     return LVM_OK;
 }
 

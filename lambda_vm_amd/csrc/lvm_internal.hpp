@@ -181,7 +181,6 @@ struct PassArgs {
     uint32_t inverse;              // 1: inverse transform (tw_* hold inverse powers)
     uint32_t in_canonical;         // 1: input values are below p (an earlier pass wrote them)
     // tiling (pass_tiling): runs of `run` words in `wins` windows of 16
-    uint32_t by_rows;              // 1: a run is the S*m words of a block's rows, 0: one row's m words
     uint32_t run, wins, tiles;
     uint32_t win_inv, m_inv;       // udiv multipliers of wins and m
     uint32_t blocks;               // blocks that cover the tiles once
@@ -250,7 +249,7 @@ __device__ __forceinline__ uint32_t find_slot(const uint32_t *__restrict__ prefi
     }
     return lo;
 }
-int plan_passes(unsigned log_n, int *r);              // radices of a size-2^log_n transform
+int plan_passes(unsigned log_n, uint32_t m, int *r);  // radices of a size-2^log_n transform of m columns
 bool set_ntt_plan(unsigned log_n, const int *r, int np);  // np = 0 restores the default
 void launch_pass_batched(int r, bool coset, uint32_t rows, const PassArgs *d_args, const uint32_t *d_prefix,
                          uint32_t count, uint32_t blocks, hipStream_t st);

@@ -65,20 +65,19 @@ static uint32_t udiv_inv(uint32_t d) { return d == 1 ? ~0u : (uint32_t)((1ull <<
 // leave most of the chip idle (2^10 x 8 commitment: 141 -> 111 us).
 uint32_t pass_tiling(int r, uint32_t cosets, PassArgs &a) {
     const uint64_t S = 1ull << a.log_s, words = S * a.m;
-    a.by_rows = words < (1ull << 31) ? 1u : 0u;
     a.units = a.log_s == 0 && a.m <= PASS_C / 2 ? PASS_C / a.m : 1;
-    a.run = a.by_rows ? (uint32_t)words * a.units : a.m;
+    a.run = (uint32_t)words * a.units;  // words < 2^31 (plan_passes)
     a.wins = (uint32_t)(((uint64_t)a.run + PASS_C - 1) / PASS_C);
     a.win_inv = udiv_inv(a.wins);
     a.m_inv = udiv_inv(a.m);
-    const uint64_t runs = a.by_rows ? ((a.total_groups >> a.log_s) + a.units - 1) / a.units : a.total_groups;
+    const uint64_t runs = ((a.total_groups >> a.log_s) + a.units - 1) / a.units;
     a.tiles = (uint32_t)(runs * a.wins);
     const uint32_t per = pass_tiles_per_block(r);
     a.blocks = (a.tiles + per - 1) / per;
     // rows a window spans: its first word lies at most m - gcd(16, m) into a row
     uint32_t g = PASS_C;
     while (a.m % g) g /= 2;
-    a.rows = a.by_rows && a.log_s ? 1 + (a.m - g + PASS_C - 1) / a.m : 1;
+    a.rows = a.log_s ? 1 + (a.m - g + PASS_C - 1) / a.m : 1;
     if (a.rows > S) a.rows = (uint32_t)S;
     const uint32_t copies = a.blocks < COSET_SPLIT_BLOCKS ? cosets : 1;
     a.cosets_per_block = cosets / copies;
@@ -104,8 +103,12 @@ static void launch_pass(int r, const PassArgs &a0, uint32_t cosets, hipStream_t 
 static int g_plan[33][8];
 static int g_plan_len[33];
 
-int plan_passes(unsigned log_n, int *r) {
-    if (log_n <= 32 && g_plan_len[log_n] > 0) {
+// A pass indexes a run, the S*m words of a block's rows, with 31 bits; the first
+// pass has the longest. An installed split whose first radix is too small for
+// that (tables of tens of GB) gives way to the default, whose runs are n*m/256 words,
+// below 2^31 for every table that fits the device's memory.
+int plan_passes(unsigned log_n, uint32_t m, int *r) {
+    if (log_n <= 32 && g_plan_len[log_n] > 0 && ((uint64_t)m << (log_n - g_plan[log_n][0])) < (1ull << 31)) {
         for (int i = 0; i < g_plan_len[log_n]; i++) r[i] = g_plan[log_n][i];
         return g_plan_len[log_n];
     }
@@ -138,7 +141,7 @@ bool set_ntt_plan(unsigned log_n, const int *r, int np) {
 int lde_pass_list(const uint64_t *trace, uint32_t m, unsigned log_n, unsigned log_blowup, const uint64_t *weights,
                   uint64_t *coef, uint64_t *lde, const Tables &tb, int *r_out, PassArgs *a_out, uint32_t *blocks_out) {
     int r[8];
-    const int np = plan_passes(log_n, r);
+    const int np = plan_passes(log_n, m, r);
     if (np == 0) return -1;
     int k = 0;
     unsigned done = 0;
@@ -228,7 +231,7 @@ static void run_passes(uint64_t *buf, uint32_t pitch, uint32_t m, size_t rows, u
 void ntt_inverse_rows(const uint64_t *in, uint32_t in_pitch, uint64_t *out, uint32_t out_pitch, uint32_t m,
                       unsigned log_n, const Tables &tb, hipStream_t st) {
     int r[8];
-    int np = plan_passes(log_n, r);
+    int np = plan_passes(log_n, m, r);
     if (np == 0) {
         (void)hipMemcpy2DAsync(out, out_pitch * 8, in, in_pitch * 8, m * 8, 1, hipMemcpyDeviceToDevice, st);
         return;
@@ -254,7 +257,7 @@ void ntt_inverse_rows(const uint64_t *in, uint32_t in_pitch, uint64_t *out, uint
 void ntt_forward_rows(const uint64_t *in, uint32_t in_pitch, uint64_t *out, uint32_t out_pitch, uint32_t m,
                       unsigned log_n, const Tables &tb, hipStream_t st) {
     int r[8];
-    int np = plan_passes(log_n, r);
+    int np = plan_passes(log_n, m, r);
     if (np == 0) {
         (void)hipMemcpy2DAsync(out, out_pitch * 8, in, in_pitch * 8, m * 8, 1, hipMemcpyDeviceToDevice, st);
         return;
@@ -284,7 +287,7 @@ int ntt_coset_expand(const uint64_t *coef, uint32_t coef_pitch, uint64_t *lde, u
                       unsigned log_n, unsigned log_blowup, const uint64_t *weights, const Tables &tb,
                       hipStream_t st) {
     int r[8];
-    int np = plan_passes(log_n, r);
+    int np = plan_passes(log_n, m, r);
     if (np == 0) return LVM_ERR_ARG;
     const uint32_t B = 1u << log_blowup;
     PassArgs a{};

@@ -86,13 +86,13 @@ __device__ __forceinline__ uint32_t udiv(uint32_t n, uint32_t d, uint32_t inv) {
 
 // Body of one pass for block `block` of the table's tiles.
 //
-// Tiles: run-major windows of PASS_C words. by_rows: a run is the S rows of one
-// block (run = S*m), lane c of window w takes word w*16 + c, i.e. row jlo = word
-// / m and column word % m; else (tables whose runs exceed 32 bits) a run is one
-// row's m words. In the last pass (S = 1) of a table of at most 8 columns a tile
-// packs `units` = 16 / m whole runs side by side. NJ: rows a window can span, each with factors of its own in LDS
-// (1 for m a multiple of 16, 2 for most m, 4 for m >= 4); 0: more than 4 (m <
-// 4), every lane forms its factors itself.
+// Tiles: run-major windows of PASS_C words. A run is the S rows of one block (run =
+// S*m words, below 2^31), lane c of window w takes word w*16 + c, i.e. row jlo =
+// word / m and column word % m. In the last pass (S = 1) of a table of at most 8
+// columns a tile packs `units` = 16 / m whole runs side by side. NJ: rows a window
+// can span, each with factors of its own in LDS (1 for m a multiple of 16, 2 for
+// most m, 4 for m >= 4); 0: more than 4 (m < 4), every lane forms its factors
+// itself.
 // COSET: the first pass of a coset expansion (bit-reversed input rows,
 // pre-multiplied, several cosets from one read).
 template <int LOG_R1, int LOG_R2, bool COSET, int NJ>
@@ -123,7 +123,6 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs &a, uint32_t block)
     const bool t_ok = tile < a.tiles;
 
     const uint32_t log_s = a.log_s;
-    const uint32_t S1 = (uint32_t)((1ull << log_s) - 1);
     // unit: the tile's run; jb: its window's first row, jl: the lane's row past it
     const uint32_t unit = t_ok ? udiv(tile, a.wins, a.win_inv) : 0;
     const uint32_t w0 = t_ok ? (tile - unit * a.wins) * C : 0;
@@ -138,16 +137,12 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs &a, uint32_t block)
         if (!c_ok) blk = 0;
         jb = jlo = 0;
         col = word - u * a.m;
-    } else if (a.by_rows) {
+    } else {
         blk = unit;
         jb = udiv(w0, a.m, a.m_inv);
         jlo = udiv(word, a.m, a.m_inv);
         col = word - jlo * a.m;
         if (NJ > 1) nj = udiv(w0 + C - 1 < a.run ? w0 + C - 1 : a.run - 1, a.m, a.m_inv) - jb + 1;
-    } else {
-        blk = unit >> log_s;
-        jb = jlo = unit & S1;
-        col = word;
     }
     const uint32_t jl = NJ > 1 ? jlo - jb : 0;
     const uint64_t rowb = blk << a.log_msub;  // logical row of t = 0, j = 0

@@ -70,3 +70,30 @@ def test_batched_fri_arguments_refused_before_device_work():
     f = lib.lvm_fri_commit_phase_batch
     assert f(None, None, ctypes.c_size_t(0), None, ctypes.c_uint(2), None, None, None, None) == 0
     assert f(None, None, ctypes.c_size_t(1), None, ctypes.c_uint(2), None, None, None, None) == 1
+
+
+@pytest.mark.parametrize("log_n,m,split,want", [
+    (22, 64, [6, 8, 8], [6, 8, 8]),                       # runs of 2^22 words
+    (26, 63, [1, 8, 8, 8, 1], [1, 8, 8, 8, 1]),           # just below 2^31
+    (26, 64, [1, 8, 8, 8, 1], [8, 8, 8, 2]),              # 2^31
+    (31, 2, [1, 6, 8, 8, 8], [8, 8, 8, 7]),
+    (31, 1, [1, 6, 8, 8, 8], [1, 6, 8, 8, 8]),
+    (4, 1 << 30, [2, 2], [4]),                            # a wide row: the default is one pass, runs of one row
+    (9, (1 << 23) - 1, [1, 8], [1, 8]), (9, 1 << 23, [1, 8], [8, 1]),
+])
+def test_ntt_splits_of_long_runs_give_way_to_the_default(log_n, m, split, want):
+    """The library's own choice of passes for a table of m columns (host code): an
+    installed split stays only while a run of its first pass is below 2^31 words;
+    the one read back is the installed one either way."""
+    lib = _native.lib()
+    plan = getattr(lib, "_ZN3lvm11plan_passesEjjPi")  # lvm::plan_passes(unsigned, uint32_t, int *)
+    out, n = (ctypes.c_int * 8)(), ctypes.c_int()
+    assert lib.lvm_get_ntt_plan(log_n, out, ctypes.byref(n)) == 0
+    keep = list(out[:n.value])
+    try:
+        assert lib.lvm_set_ntt_plan(log_n, (ctypes.c_int * len(split))(*split), len(split)) == 0
+        k = plan(ctypes.c_uint(log_n), ctypes.c_uint32(m), out)
+        assert list(out[:k]) == want
+        assert lib.lvm_get_ntt_plan(log_n, out, ctypes.byref(n)) == 0 and list(out[:n.value]) == split
+    finally:
+        lib.lvm_set_ntt_plan(log_n, (ctypes.c_int * len(keep))(*keep), len(keep))
