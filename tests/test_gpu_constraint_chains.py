@@ -12,6 +12,19 @@ pytestmark = pytest.mark.gpu
 P = np.uint64(workload.P)
 
 
+@pytest.fixture(autouse=True)
+def compiled(gpu):
+    """Compiled kernels ran, and the interpreter never."""
+    gpu.set_constraint_jit(True)
+    gpu.prof_reset()
+    gpu.prof_enable(True)
+    yield
+    gpu.prof_enable(False)
+    ran = {nm: gpu.prof_query(nm)[0] for nm in ("constraint_evals_compiled", "composition_compiled",
+                                                "constraint_evals", "composition")}
+    assert ran["constraint_evals_compiled"] > 0 and ran["constraint_evals"] == ran["composition"] == 0, ran
+
+
 def canon(a):
     a = np.asarray(a, dtype=np.uint64)
     return np.where(a >= P, a - P, a)
@@ -66,11 +79,14 @@ def test_chain_forms_match_oracle(gpu, ora, log_n):
         got = gpu.eval_constraints(dev, hm, ha, B, rap=r, alpha=al)
         assert np.array_equal(canon(got), canon(ev_ref))
         args = (dev, hm, ha, B, n, g, betas, groups, ex)
+        before = gpu.prof_query("composition_compiled")[0]
         one = gpu.eval_composition(*args, rap=r, alpha=al).to_array(np.uint64, (n * B, 3))
         assert np.array_equal(canon(one), canon(ref)[_bitrev_perm(n * B)])
+        assert gpu.prof_query("composition_compiled")[0] == before + 1
     many = gpu.eval_composition_batch([dict(dev=dev, main=hm, aux=ha, next_step=B, trace_rows=n, coset_offset=g,
                                             betas=betas, root_group=groups, group_exemptions=ex, rap=rap,
                                             alpha=alpha)] * 2)
+    assert gpu.prof_query("composition_compiled")[0] == before + 2  # both tables in one launch
     for h in many:
         assert np.array_equal(canon(h.to_array(np.uint64, (n * B, 3))), canon(ref)[_bitrev_perm(n * B)])
 
