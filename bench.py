@@ -356,10 +356,9 @@ def run_ragged(args) -> dict:
     dom = max(per_launch, key=lambda k: per_launch[k][0])
     avg_ms, nbytes, _ = per_launch[dom]
     achieved = nbytes / (avg_ms / 1e3) / 1e9
-    stage = {"ntt": 0.0, "leaves": 0.0, "merkle": 0.0, "roots": 0.0}
+    stage = {"ntt": 0.0, "leaves": 0.0, "merkle": 0.0}
     for name, (ms, _, _) in per_launch.items():
-        key = name.split("_")[1]
-        stage["ntt" if key == "ntt" else "leaves" if key == "leaves" else "merkle" if key == "merkle" else "roots"] += ms
+        stage[name.split("_")[1]] += ms
     roofline = {
         "bound": "hbm",
         "kernel": dom,

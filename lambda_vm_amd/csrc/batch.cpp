@@ -82,12 +82,6 @@ struct Writer {
         off += n * sizeof(T);
         return at;
     }
-    size_t reserve(size_t bytes) {
-        off = (off + 15) & ~(size_t)15;
-        const size_t at = off;
-        off += bytes;
-        return at;
-    }
 };
 
 }  // namespace

@@ -263,7 +263,7 @@ struct LeafJob {
     uint64_t pitch;
     uint64_t num_leaves;
     uint64_t *nodes;       // the table's tree
-    uint32_t span;         // leaves per block of a small table (leaf_top_span), 0: TREE_THREADS of them, no levels
+    uint32_t span;         // leaves per block of a small table (leaf_top_span), 0: TREE_WIDE_SPAN of them, no levels
     uint32_t root;         // the table's slot in the launch's root array
 };
 struct TreeStep {
@@ -276,15 +276,17 @@ struct TreeStep {
 };
 // Trees of more children than this have their level hashed one node per lane;
 // below, the step is a tree top: blocks of TREE_TOP_SPAN parents, all their
-// levels, one permutation per 16 lanes (merkle.hip).
+// levels, one permutation per 16 lanes (merkle.hip). In a launch over several
+// trees the tops' children together stay within TREE_TOP_BATCH (tree_steps).
 constexpr uint64_t TREE_TOP_CHILDREN = 1u << 14;
 constexpr uint32_t TREE_TOP_SPAN = 32;
-constexpr uint64_t TREE_TOP_BATCH = 1u << 15;  // children of the tops of one batched launch, together
-constexpr uint32_t TREE_WIDE_SPAN = 512;  // parents per block of a wide level
+constexpr uint64_t TREE_TOP_BATCH = 1u << 15;
+constexpr uint32_t TREE_WIDE_SPAN = 512;  // leaves, or parents of a wide level, per block of a batched launch
 // Trees of at most this many leaves hash them one permutation per 16 lanes
-// too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch.
+// too, TREE_TOP_SPAN leaves per block, and the levels above in the same launch,
+// when such trees have at most LEAF_TOP_BATCH leaves together (leaf_top_spans).
 constexpr uint64_t LEAF_TOP_LEAVES = 1u << 13;
-constexpr uint64_t LEAF_TOP_BATCH = 1u << 15;  // together, in one batched launch
+constexpr uint64_t LEAF_TOP_BATCH = 1u << 15;
 inline uint32_t leaf_top_span(uint64_t L) { return (uint32_t)(L < TREE_TOP_SPAN ? L : TREE_TOP_SPAN); }
 std::vector<uint32_t> leaf_top_spans(const std::vector<uint64_t> &leaves);  // per table of one launch (batch.cpp)
 // roots: 32-byte slots, written by the blocks that hash a root

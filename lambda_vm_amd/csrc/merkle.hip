@@ -16,6 +16,8 @@
 
 namespace lvm {
 
+static_assert(TREE_WIDE_SPAN == TREE_THREADS, "batched launches are sized in leaves and parents per block of the kernels");
+
 // XOR the big-endian encoding of an element into a lane held as 32-bit
 // halves: the little-endian lane of BE(v) is bswap64(v), v canonical.
 __device__ __forceinline__ void absorb_be(uint32_t &l, uint32_t &h, uint64_t v) {
