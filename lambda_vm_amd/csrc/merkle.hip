@@ -30,7 +30,7 @@ __device__ __forceinline__ void absorb_be(uint32_t &l, uint32_t &h, uint64_t v) 
 // the committed words are whole rows, so the leaf's data is one contiguous
 // run of 2*pitch words. CANON: the words may lie in [p, 2^64) (rows handed in
 // by a caller; this library's own LDE rows are canonical).
-// VALU-bound (0.96 of the issue rate on wide tables): what counts is
+// VALU-bound (0.95 of the issue rate on wide tables): what counts is
 // instructions. The last block masks the words past the message instead of
 // branching per word, which had the compiler copy the 50-register state at
 // each of 17 joins (1300 cycles, 7 % of a permutation).
